@@ -158,7 +158,7 @@ void free_plan_buffers(fct_wfbp_gpu_plan* p) {
                   p->d_slab_vrange, p->d_rebin,  p->d_Hn,        p->d_tw,       p->d_thk_off,
                   p->d_thk_idx,  p->d_thk_w,     p->d_filtered,  p->d_scale, p->d_native,
                   p->d_raw_stage, p->d_vol_stage, p->d_gbar, p->d_thkT_off, p->d_thkT_idx,
-                  p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_af_raw, p->d_af_vmax};
+                  p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_ray_tab, p->d_ray_pad, p->d_ray_rec, p->d_af_raw, p->d_af_vmax};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (int b = 0; b < 2; ++b)
@@ -297,7 +297,43 @@ fct::RayProjArgs ray_args(const fct_wfbp_gpu_plan* p) {
   const double z1 = fct_tables::slice_z(r.start_pos, r.end_pos, p->csw, 1);
   a.gz0 = (float)z0;
   a.gdz = (float)(z1 - z0);
+  a.dx0 = x0;
+  a.ddx = dx;
+  a.dy0 = cw ? -y0 : y0;
+  a.ddy = cw ? -dy : dy;
+  a.dz0 = z0;
+  a.ddz = z1 - z0;
   return a;
+}
+
+// A plan-owned device buffer allocated on first use; nullptr (and no error
+// left behind) when it does not fit or the plan's stream is being captured
+// into a graph, where the callers take a path without it.
+void* try_scratch(fct_wfbp_gpu_plan* p, size_t bytes) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  void* d = nullptr;
+  if (hipStreamIsCapturing(p->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+      hipMalloc(&d, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return d;
+}
+
+// The plan's ray tables, filled on first use on its stream; false: the
+// general kernels run (geometry outside the tables' rule, or no memory).
+bool ray_tables(fct_wfbp_gpu_plan* p, const fct::RayProjArgs& a, fct::RayTables* t) {
+  if (!p->d_ray_tab) {
+    if (!fct::ray_tables_apply(a)) return false;
+    p->d_ray_tab = try_scratch(p, fct::ray_table_bytes(a));
+    if (!p->d_ray_tab) return false;
+  }
+  *t = fct::ray_table_layout(a, p->d_ray_tab);
+  if (!p->ray_tab_ready) {
+    if (fct::launch_ray_table(a, *t, p->stream) != hipSuccess) return false;
+    p->ray_tab_ready = true;
+  }
+  return true;
 }
 
 // Thickening of requested slices [s0, s1) from the native slices.
@@ -1188,6 +1224,16 @@ FCT_API int fct_wfbp_gpu_ray_project(fct_wfbp_gpu_plan* p, const float* native, 
   fct::RayProjArgs a = ray_args(p);
   a.vol_in = native;
   a.raw_out = raw;
+  fct::RayTables t;
+  if (ray_tables(p, a, &t)) {
+    if (!p->d_ray_pad)
+      p->d_ray_pad =
+          static_cast<float*>(try_scratch(p, 2 * fct::ray_pad_elems(a) * sizeof(float)));
+    if (p->d_ray_pad) {
+      HIP_TRY(p->ctx, fct::launch_ray_project_table(a, t, p->d_ray_pad, p->stream));
+      return FCT_OK;
+    }
+  }
   HIP_TRY(p->ctx, fct::launch_ray_project(a, false, p->stream));
   return FCT_OK;
 }
@@ -1201,6 +1247,16 @@ FCT_API int fct_wfbp_gpu_ray_backproject(fct_wfbp_gpu_plan* p, const float* raw,
   fct::RayProjArgs a = ray_args(p);
   a.raw_in = raw;
   a.vol_out = native;
+  fct::RayTables t;
+  if (ray_tables(p, a, &t)) {
+    if (!p->d_ray_rec)
+      p->d_ray_rec =
+          static_cast<float*>(try_scratch(p, (size_t)p->raw_elems() * 3 * sizeof(float)));
+    if (p->d_ray_rec) {
+      HIP_TRY(p->ctx, fct::launch_ray_gather(a, t, p->d_ray_rec, p->ncu, p->stream));
+      return FCT_OK;
+    }
+  }
   HIP_TRY(p->ctx, fct::launch_fill(native, (size_t)p->n_native * p->recon.ny * p->recon.nx, 0.0f,
                                    p->stream));
   HIP_TRY(p->ctx, fct::launch_ray_project(a, true, p->stream));

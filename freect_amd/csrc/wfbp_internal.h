@@ -150,6 +150,22 @@ struct RayProjArgs {
   double r, dsd, dgamma, drow, cc, cr, angle0, dtheta, z0, dz;
   double ffs_off[4][3];      // per focal state (dr, da, dz) along (e_w, e_u, e_z)
   float gx0, gdx, gy0, gdy, gz0, gdz;   // voxel-centre grids (FP32 of FP64)
+  double dx0, ddx, dy0, ddy, dz0, ddz;  // and in FP64
+};
+
+// Geometry tables of the table-driven ray projector (rayproj.hip).
+struct RayTables {
+  float4* ray;     // [view][channel] A, B, T0, DT (low bit of DT: x planes)
+  float4* view;    // [view][2]: cos, sin, R + o0, o1; (-cr drow - oz) / gdz, o0, -, -
+  double* zoff;    // [view] focal spot z in slices
+  float* len2;     // [focal state][channel] squared in-plane source-detector distance
+  double zsrc[4];  // focal state's z offset
+};
+
+struct RayGather {
+  int32_t tiles_x, tiles_y, slabs, nsplit;   // 8 x 8 column tiles, slabs, splits of the views
+  const float* rec;  // [view][row][channel] A, B, value x path length (ray_record_kernel)
+  double reach;    // mm of table z beyond a slab whose views can meet it
 };
 
 struct BpAdjArgs {
@@ -170,6 +186,18 @@ hipError_t launch_rebin_filter(const RebinFilterArgs& a, hipStream_t s);
 // Ray-driven projection of vol_in onto raw_out (views [v0, v1)), or with
 // transpose its exact transpose from raw_in into vol_out (accumulated).
 hipError_t launch_ray_project(const RayProjArgs& a, bool transpose, hipStream_t s);
+// Table-driven forms: whether they apply, the tables (of ray_table_bytes) and
+// the projector's padded volume copies (2 x ray_pad_elems floats).
+bool ray_tables_apply(const RayProjArgs& a);
+size_t ray_table_bytes(const RayProjArgs& a);
+size_t ray_pad_elems(const RayProjArgs& a);
+RayTables ray_table_layout(const RayProjArgs& a, void* mem);
+hipError_t launch_ray_table(const RayProjArgs& a, const RayTables& t, hipStream_t s);
+hipError_t launch_ray_project_table(const RayProjArgs& a, const RayTables& t, float* pad,
+                                    hipStream_t s);
+// rec: 3 floats per ray.
+hipError_t launch_ray_gather(const RayProjArgs& a, const RayTables& t, float* rec, int ncu,
+                             hipStream_t s);
 // Adaptive filtration of raw views [v0, v1): per view the largest finite
 // |p| (vmax), then every sample blended with its 3 x 3 (row, channel) mean by
 // lambda = clamp((p - (1 - s) vmax) / (s vmax), 0, 1).  out != in.
@@ -275,6 +303,10 @@ struct fct_wfbp_gpu_plan {
   float* d_native = nullptr;
   float* d_raw_stage = nullptr;
   float* d_vol_stage = nullptr;
+  void* d_ray_tab = nullptr;        // ray projector tables (first use; ready: filled)
+  bool ray_tab_ready = false;
+  float* d_ray_pad = nullptr;       // padded volume copies of the ray projector (first use)
+  float* d_ray_rec = nullptr;       // per-ray records of its transpose (first use)
   float* d_gbar = nullptr;          // adjoint scratch, [view][row][cpitch] FP32
   int32_t* d_thkT_off = nullptr;    // transposed thickening table
   int32_t* d_thkT_idx = nullptr;

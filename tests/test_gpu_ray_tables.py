@@ -1,0 +1,92 @@
+"""The table-driven ray projector and its gathered transpose at the sizes
+where they can go wrong: matrices that are not multiples of the 8 x 8 tiles or
+of the 32 x 32 transposition, one slice more than a slab, odd row and channel
+counts, a falling slice grid, coarse voxels, FFS, an off-centre field -- and
+a geometry and a graph capture that take the general kernels.  Each against
+the FP64 restatement; the bound is that of the FP32 sample positions (a few
+ulps of a position of up to ~600 voxels, 2e-5 of the largest output), as for
+the general kernels.
+"""
+import numpy as np
+import pytest
+
+from freect_amd import scans as S
+from helpers import gpu_ctx, to_np
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return gpu_ctx()
+
+
+def _setup(nx, ny, nz, rows, chans, fov, ffs=0, flip=False, rotation=1, ppr=96):
+    w = S.tiny(nx=nx, n_slices=nz, n_channels=chans, n_rows=rows, ppr=ppr, rotations=1.2,
+               ffs_mode=ffs)
+    rc = w.recon.replace(ny=ny, recon_fov=fov, x_origin=-6.0, y_origin=4.0)
+    if flip:
+        rc = rc.replace(start_pos=rc.end_pos, end_pos=rc.start_pos)
+    return w.scan.replace(rotation=rotation, angle0=0.4), rc
+
+
+CASES = [dict(nx=33, ny=21, nz=2, rows=8, chans=96, fov=300.0),
+         dict(nx=40, ny=17, nz=17, rows=11, chans=130, fov=350.0, rotation=-1),
+         dict(nx=9, ny=64, nz=33, rows=16, chans=65, fov=120.0, flip=True),
+         dict(nx=70, ny=70, nz=16, rows=9, chans=200, fov=400.0, ffs=1),
+         dict(nx=31, ny=30, nz=12, rows=7, chans=97, fov=250.0, ffs=2, flip=True),
+         # Outside the tables' rule: the volume's corners pass the focal spot.
+         dict(nx=24, ny=24, nz=6, rows=8, chans=96, fov=900.0)]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_ray_pair_matches_oracle(ctx, oracle, case):
+    from freect_amd import wfbp
+    sc, rc = _setup(**CASES[case])
+    p = wfbp.Plan(ctx, sc, rc)
+    nz = p.info.n_slices_native
+    gen = torch.Generator(device="cuda").manual_seed(case)
+    x = torch.rand((nz, rc.ny, rc.nx), device="cuda", generator=gen)
+    y = torch.rand((sc.n_views, sc.n_rows, sc.n_channels), device="cuda", generator=gen)
+    px, pty = p.alloc_raw().fill_(float("nan")), p.alloc_native().fill_(float("nan"))
+    for _ in range(2):   # first use builds the tables, the second reuses them
+        p.ray_project(x, px)
+        p.ray_backproject(y, pty)
+    p.synchronize()
+    ref = oracle.ray_project(sc, rc, to_np(x).astype(np.float64))
+    reft = oracle.ray_backproject(sc, rc, to_np(y).astype(np.float64), nz)
+    e = np.abs(to_np(px) - ref).max() / np.abs(ref).max()
+    et = np.abs(to_np(pty) - reft).max() / np.abs(reft).max()
+    assert e < 2e-5 and et < 2e-5, (e, et)
+
+
+def test_first_call_inside_a_capture(ctx):
+    # No table may be allocated inside a capture: the general kernels are
+    # recorded, and later calls outside agree with the replays.
+    from freect_amd import wfbp
+    sc, rc = _setup(**CASES[1])
+    p = wfbp.Plan(ctx, sc, rc)
+    x = torch.rand((p.info.n_slices_native, rc.ny, rc.nx), device="cuda")
+    px, pt = p.alloc_raw(), p.alloc_native()
+    s = torch.cuda.Stream()
+    p.set_stream(s)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        p.ray_project(x, px)
+        p.ray_backproject(px, pt)
+    for _ in range(3):
+        px.zero_()
+        pt.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        a, b = px.clone(), pt.clone()
+    qx, qt = p.alloc_raw(), p.alloc_native()
+    p.ray_project(x, qx)
+    p.ray_backproject(qx, qt)
+    p.synchronize()
+    assert (a - qx).abs().max() <= 2e-5 * qx.abs().max()
+    assert (b - qt).abs().max() <= 2e-5 * qt.abs().max()
