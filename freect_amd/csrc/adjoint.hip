@@ -5,15 +5,20 @@
 // cuda_kernels.cuh:11-93, 198-287) is linear in the raw data for a fixed
 // geometry: W(q) and its per-theta~ sum depend on geometry only.  Transposes:
 //   backprojection^T: per voxel and theta~, the weight sum over the selected
-//     views is formed first, then every selected sample scatters
-//     scale * xbar * W / sum W times its four bilinear weights (FP32 hardware
-//     atomics; summation order, not values, is non-deterministic);
+//     views is formed first, then every selected sample adds
+//     scale * xbar * W / sum W times its four bilinear weights -- gathered per
+//     detector sample, or (where the gather has no scratch: a graph capture
+//     before its first use) scattered by FP32 hardware atomics;
 //   filter^T: the filter (symmetric Toeplitz), run by rebin_filter.hip's
 //     filter-only mode;
 //   rebin^T: every parallel sample scatters its four bilinear weights to the
 //     clamped fan samples it read.
 // Selection and the FP32 weights are computed by the same code as the forward
 // kernels, so the transpose is exact up to FP32 summation order.
+#include <algorithm>
+#include <cmath>
+
+#include "wave_ops.h"
 #include "wfbp_internal.h"
 
 namespace fct {
@@ -131,6 +136,306 @@ __global__ __launch_bounds__(64) void bp_adjoint_kernel(BpAdjArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Gathered form: every detector sample collects from the voxels that read it.
+// ---------------------------------------------------------------------------
+// Volume order of a theta~: planes of the axis its parallel rays run along
+// (the primary axis: x where |cos| >= |sin|, else y), slices, then the other
+// in-plane axis, so that the 64 neighbouring channels of a wave read
+// neighbouring addresses.
+
+// What the other kernels need of every voxel column for the theta~ [t0, t0 +
+// nt): (rows per mm of z for the even and the odd views, kappa asin(p / R),
+// p), the forward kernels' FP32 values; p = 1e30 outside the FOV, which no
+// channel matches.
+__global__ __launch_bounds__(256) void bp_adjoint_column_kernel(BpAdjArgs a, AdjGather q) {
+  const BpArgs& b = a.bp;
+  const FctBpConsts& g = b.g;
+  const int ns = q.swap ? b.ny : b.nx;
+  const int i = blockIdx.x * 256 + threadIdx.x, n = b.nx * b.ny;
+  if (i >= n) return;
+  const int prim = i / ns, sec = i - prim * ns;
+  const float x = b.xs[q.swap ? prim : sec], y = b.ys[q.swap ? sec : prim];
+  const bool active = fct_in_fov(x, y, g);
+  for (int ti = blockIdx.y; ti < q.nt; ti += gridDim.y) {
+    const float* csp = reinterpret_cast<const float*>(b.cs + q.t0 + ti);
+    const float c = ld_uniform(csp), sn = ld_uniform(csp + 1);
+    const float p = fmaf(x, sn, -(y * c));
+    const float sq = sqrt_rn_large(fmaf(-p, p, g.R2));
+    const float f = fmaf(x, c, y * sn);
+    const float4 e = make_float4(div_rn_normal(g.hr, (sq - f) * g.tanc),
+                                 div_rn_normal(g.hr, (sq + f) * g.tanc),
+                                 g.kappa * fct_asinf(p * g.invR), p);
+    q.col[(size_t)ti * n + i] = active ? e : make_float4(0.0f, 0.0f, 0.0f, 1e30f);
+  }
+}
+
+// xbar * scale / sum W of every voxel for the theta~ [t0, t0 + nt) (0 where no
+// view selects the voxel), in that order: one wave per 64 voxels along the
+// secondary axis and eight slices.
+constexpr int kAdjSlices = 8;
+template <bool CENTERED>
+__global__ __launch_bounds__(64) void bp_adjoint_weights_kernel(BpAdjArgs a, AdjGather q) {
+  const BpArgs& b = a.bp;
+  const FctBpConsts& g = b.g;
+  const int ns = q.swap ? b.ny : b.nx, np = q.swap ? b.nx : b.ny;
+  const int groups = (ns + 63) >> 6, nsl = (b.n_native + kAdjSlices - 1) / kAdjSlices;
+  const int id = xcd_block(blockIdx.x, gridDim.x);
+  const int slab = id / (groups * np), rest = id - slab * groups * np;
+  const int prim = rest / groups, sec = (rest - prim * groups) * 64 + threadIdx.x;
+  const int ix = q.swap ? prim : sec, iy = q.swap ? sec : prim;
+  const bool inb = sec < ns;
+  const bool active = inb && fct_in_fov(b.xs[min(ix, b.nx - 1)], b.ys[min(iy, b.ny - 1)], g);
+  const int s0 = slab * kAdjSlices, nz = min(kAdjSlices, b.n_native - s0);
+  const int chunk = s0 / fct_tables::kSliceChunk;
+  float zs[kAdjSlices], xb[kAdjSlices];
+#pragma unroll
+  for (int i = 0; i < kAdjSlices; ++i) {
+    zs[i] = b.zs[s0 + min(i, nz - 1)];
+    xb[i] = (i < nz && active) ? a.xbar[((size_t)(s0 + i) * b.ny + iy) * b.nx + ix] * b.scale
+                               : 0.0f;
+  }
+  const bool some = __any(active);
+  const float* ztc = b.zt + (size_t)chunk * b.nviews;
+  const int* wrc = reinterpret_cast<const int*>(b.wrange + (size_t)chunk * b.nviews);
+  const size_t plane = (size_t)b.nx * b.ny;
+  float* out = q.wgt + ((size_t)prim * b.n_native + s0) * ns + sec;
+  for (int ti = 0; ti < q.nt; ++ti, out += plane * b.n_native) {
+    const int t = q.t0 + ti;
+    float den[kAdjSlices];
+#pragma unroll
+    for (int i = 0; i < kAdjSlices; ++i) den[i] = 0.0f;
+    if (some) {
+      const float4 col = q.col[(size_t)ti * plane + (size_t)prim * ns + min(sec, ns - 1)];
+      const float p = col.w, kb = col.z;
+#pragma unroll
+      for (int par = 0; par < 2; ++par) {
+        const float pidx = par ? fmaf(-p, g.inv_ds, g.cc) : fmaf(p, g.inv_ds, g.cc);
+        const float pfl = floorf(pidx);
+        const bool ok = active && pfl >= 0.0f && pfl <= (float)(g.ncols - 2);
+        const float invL = ok ? (par ? col.y : col.x) : 0.0f;
+        for (int v = t + par * b.H; v < b.nviews; v += 2 * b.H) {
+          const int wx = ld_uniform(wrc + 2 * v), wy = ld_uniform(wrc + 2 * v + 1);
+          if (wx > s0 + nz - 1 || wy < s0) continue;
+          const float row0 = ok ? fmaf((par ? -kb : kb) - ld_uniform(ztc + v), invL, g.cr) : -1e30f;
+          const float qa = fmaf(zs[0], invL, row0), qb = fmaf(zs[kAdjSlices - 1], invL, row0);
+          if (!__any(fmaxf(qa, qb) >= 0.0f && fminf(qa, qb) < (float)(g.nrows - 1))) continue;
+#pragma unroll
+          for (int i = 0; i < kAdjSlices; ++i) {
+            if (s0 + i < wx || s0 + i > wy) continue;
+            const float qi = fmaf(zs[i], invL, row0);
+            const int iq = floor_int(qi);
+            bool sel = ok && (uint32_t)iq <= (uint32_t)(g.nrows - 2);
+            if (!CENTERED) sel = sel && !(fabsf(qi - g.cr) > g.hr);
+            const float W = fct_w_of_row(qi, g);
+            den[i] += sel ? W : 0.0f;
+          }
+        }
+      }
+    }
+    if (inb)
+#pragma unroll
+      for (int i = 0; i < kAdjSlices; ++i)
+        if (i < nz) out[(size_t)i * ns] = den[i] > 0.0f ? xb[i] / den[i] : 0.0f;
+  }
+}
+
+// The matched pair's volume in the swapped order [x][slice][y].
+__global__ __launch_bounds__(256) void swap_volume_kernel(const float* __restrict__ in,
+                                                          float* __restrict__ out, int nx, int ny,
+                                                          int nz) {
+  __shared__ float tile[32][33];
+  const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int z = blockIdx.z; z < nz; z += gridDim.z) {
+    for (int r = ty; r < 32; r += 8)
+      if (bx + tx < nx && by + r < ny) tile[r][tx] = in[((size_t)z * ny + by + r) * nx + bx + tx];
+    __syncthreads();
+    for (int r = ty; r < 32; r += 8)
+      if (bx + r < nx && by + tx < ny) out[((size_t)(bx + r) * nz + z) * ny + by + tx] = tile[tx][r];
+    __syncthreads();
+  }
+}
+
+// One wave per (view, 64 channels, RC detector rows), a lane per channel with
+// its rows in LDS.  Plane by plane along the primary axis, the voxel columns
+// whose channel position lies within one channel of the lane's (a fixed
+// small number of candidates around the ray, tested with the forward
+// kernels' FP32 position) add their slices into the lane's rows (one LDS read
+// and write of two rows per slice, conflict-free).  Bound by VALU issue: 25
+// instructions per slice of a candidate, of whose lanes half to three quarters
+// hold one.  2952 views x 16 x 736 from 384 x 384 x 32 voxels: 287 ms with
+// four global atomics per sample -> 4.5 (weights) + 10.8 ms.  RC rows per
+// wave: 16 or 32, so that the rows in LDS leave at least 16 waves per CU.
+template <int RC, bool CENTERED, bool MATCHED>
+__global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjGather q) {
+  // Detector rows rlo .. rlo + rspan + 1 (below): this wave's and the
+  // neighbouring waves' rows next to them, which are dropped.
+  __shared__ float acc[(RC + 2) * 64];
+  const BpArgs& b = a.bp;
+  const FctBpConsts& g = b.g;
+  const int lane = threadIdx.x, H = b.H;
+  const int cg = b.cpitch >> 6, nrc = (g.nrows + RC - 1) / RC;
+  const int kv = (b.nviews + H - 1) / H;
+  int id = xcd_block(blockIdx.x, gridDim.x);
+  const int ch = (id % cg) * 64 + lane;
+  id /= cg;
+  const int split = id % q.nsplit;
+  id /= q.nsplit;
+  const int R0 = (id % nrc) * RC;
+  id /= nrc;
+  const int kk = id % kv, ti = id / kv;
+  const int t = q.t0 + ti, v = t + kk * H;
+  if (v >= b.nviews) return;
+  const bool odd = kk & 1;
+  const float* csp = reinterpret_cast<const float*>(b.cs + t);
+  const int ns = q.swap ? b.ny : b.nx, np = q.swap ? b.nx : b.ny;
+  const int i0 = (int)((long long)np * split / q.nsplit);
+  const int i1 = (int)((long long)np * (split + 1) / q.nsplit);
+#pragma unroll
+  for (int r = 0; r < RC + 2; ++r) acc[r * 64 + lane] = 0.0f;
+  // Footprints of rows [rlo, rlo + rspan] reach this wave's rows.
+  const int rlo = max(0, R0 - 1), rspan = min(g.nrows - 2, R0 + RC - 1) - rlo;
+  float* lrow = acc + lane;   // row rlo
+
+  // Along the channel's ray, linear in the plane index i: the secondary
+  // position J0 + i J1 (columns within hw of it are within one channel) and
+  // the distance from the focal spot to the column, L0 + i L1.
+  float J0, J1, hw, L0, L1, kb0, zmargin;
+  {
+    const double ds = 1.0 / (double)g.inv_ds, c = ld_uniform(csp), s = ld_uniform(csp + 1);
+    const double pe = ((double)min(ch, g.ncols - 1) - (double)g.cc) * ds, p = odd ? -pe : pe;
+    const double x0 = q.gx0, y0 = q.gy0, dx = q.gdx, dy = q.gdy;
+    const double sqr = sqrt(fmax((double)g.R2 - p * p, 1.0));
+    double f0, f1;
+    if (q.swap) {   // x planes: y = (x s - p) / c
+      J0 = (float)(((x0 * s - p) / c - y0) / dy);
+      J1 = (float)(dx * s / c / dy);
+      hw = (float)fabs(ds / (c * dy));
+      f0 = x0 * c + (x0 * s - p) / c * s;
+      f1 = dx * c + dx * s / c * s;
+    } else {        // y planes: x = (p + y c) / s
+      J0 = (float)(((p + y0 * c) / s - x0) / dx);
+      J1 = (float)(dy * c / s / dx);
+      hw = (float)fabs(ds / (s * dx));
+      f0 = (p + y0 * c) / s * c + y0 * s;
+      f1 = dy * c / s * c + dy * s;
+    }
+    hw = fmaf(hw, 1.001f, 0.01f);   // rounding of the positions
+    L0 = (float)(odd ? sqr + f0 : sqr - f0);
+    L1 = (float)(odd ? f1 : -f1);
+    const float kb = g.kappa * fct_asinf((float)p * g.invR);
+    kb0 = odd ? -kb : kb;
+    // A candidate's column lies within one channel of the ray, and within
+    // hw of it along the secondary axis (sqrt 2 channels at most).
+    zmargin = (float)(1.5 * ds / sqr) * fabsf(g.kappa) + 4.0f * (float)ds * g.tanc *
+              (1.0f + 2.0f / g.hr);
+  }
+  const int nj = __builtin_amdgcn_readfirstlane((int)(2.0f * hw) + 1);
+  const float inv_dz = (float)(1.0 / q.dz);
+  const float ra = ((float)rlo - g.cr) / g.hr * g.tanc;
+  const float rb = ((float)(rlo + rspan + 1) - g.cr) / g.hr * g.tanc;
+  const int nchunks = (b.n_native + fct_tables::kSliceChunk - 1) / fct_tables::kSliceChunk;
+  const float* vol = MATCHED ? (q.swap ? q.wgt : a.xbar)
+                             : q.wgt + (size_t)ti * b.nx * b.ny * b.n_native;
+  const float4* cols = q.col + (size_t)ti * b.nx * b.ny;
+  // (The matched projector reads the volume itself for y planes.)
+  const size_t pstride = MATCHED && !q.swap ? (size_t)b.nx : (size_t)b.n_native * ns;
+  const size_t sstride = MATCHED && !q.swap ? (size_t)b.nx * b.ny : (size_t)ns;
+
+  for (int chunk = 0; rspan >= 0 && chunk < nchunks; ++chunk) {
+    const int a0 = chunk * fct_tables::kSliceChunk;
+    const int na = min(fct_tables::kSliceChunk, b.n_native - a0);
+    int k0 = 0, k1 = na - 1;   // slices a0 + [k0, k1] of this chunk the view may select
+    if (MATCHED) {
+      // Every slab whose view range holds the view (as the backprojection).
+      int first = na, last = -1;
+      for (int s = 0; s < na; s += q.tile_z) {
+        const int* vr = reinterpret_cast<const int*>(b.slab_vrange + (a0 + s) / q.tile_z);
+        if (ld_uniform(vr) <= v && v < ld_uniform(vr + 1)) {
+          first = min(first, s);
+          last = min(s + q.tile_z, na) - 1;
+        }
+      }
+      k0 = first;
+      k1 = last;
+    } else {
+      const int* wr = reinterpret_cast<const int*>(b.wrange + (size_t)chunk * b.nviews + v);
+      k0 = max(k0, ld_uniform(wr) - a0);
+      k1 = min(k1, ld_uniform(wr + 1) - a0);
+    }
+    if (k0 > k1) continue;
+    const float zsl = b.zs[a0 + min(lane, na - 1)];   // slice z, one per lane
+    const float zfirst = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(zsl), 0));
+    const float ztv = ld_uniform(b.zt + (size_t)chunk * b.nviews + v);
+    // Slice positions at which the rows rlo and rlo + rspan + 1 cross the ray.
+    const float zc = ztv - kb0 - zfirst, sm = fmaf(zmargin, fabsf(inv_dz), 0.05f);
+    const float A0 = fmaf(ra, L0, zc) * inv_dz, A1 = ra * L1 * inv_dz;
+    const float B0 = fmaf(rb, L0, zc) * inv_dz, B1 = rb * L1 * inv_dz;
+    for (int i = i0; i < i1; ++i) {
+      const float fi = (float)i, sa = fmaf(fi, A1, A0), sb = fmaf(fi, B1, B0);
+      const int j0 = (int)ceilf(fmaf(fi, J1, J0) - hw);
+      const bool some = ch < g.ncols && j0 < ns && j0 + nj > 0;
+      const int sl = max(wave_min_i(some ? (int)ceilf(fminf(sa, sb) - sm) : INT32_MAX), k0);
+      const int sh = min(wave_max_i(some ? (int)floorf(fmaxf(sa, sb) + sm) : -1), k1);
+      if (sl > sh) continue;
+      const float* vplane = vol + (size_t)i * pstride + (size_t)(a0 + sl) * sstride;
+      for (int m = 0; m < nj; ++m) {
+        const int j = j0 + m, jc = min(max(j, 0), ns - 1);
+        const float4 col = cols[(size_t)i * ns + jc];
+        const float pidx = odd ? fmaf(-col.w, g.inv_ds, g.cc) : fmaf(col.w, g.inv_ds, g.cc);
+        const float pfl = floorf(pidx);
+        const int d = ch - (int)pfl;
+        const bool ok = j == jc && pfl >= 0.0f && pfl <= (float)(g.ncols - 2) && (uint32_t)d <= 1u;
+        if (!ok) continue;
+        const float wp = pidx - pfl;
+        float wc = d ? wp : 1.0f - wp;
+        const float invL = odd ? col.y : col.x;
+        const float row0 = fmaf((odd ? -col.z : col.z) - ztv, invL, g.cr);   // fct_bp_row0
+        // R / l = tanc / (lt / R) with lt = hr / invL.
+        if (MATCHED) wc *= b.scale * (g.tanc / (g.hr * g.invR)) * invL;
+        auto add = [&](int s, float xv) {
+          const float z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(zsl), s));
+          const float qi = fmaf(z, invL, row0);   // fct_bp_row
+          const uint32_t l = (uint32_t)(floor_int(qi) - rlo);
+          bool sel = l <= (uint32_t)rspan;
+          if (!CENTERED) sel = sel && !(fabsf(qi - g.cr) > g.hr);
+          float val = xv * wc;
+          if (!MATCHED)
+            val *= fct_w_of_t(
+                __builtin_amdgcn_fmed3f(fmaf(-fabsf(qi - g.cr), g.wk, FCT_WC), 0.0f, 1.0f));
+          val = sel ? val : 0.0f;
+          const float hi = val * __builtin_amdgcn_fractf(qi);
+          float* r = lrow + min(l, (uint32_t)rspan) * 64;
+          const float r0 = r[0], r1 = r[64];
+          r[0] = r0 + (val - hi);
+          r[64] = r1 + hi;
+        };
+        const float* xp = vplane;
+        int s = sl;
+        for (; s + 3 <= sh; s += 4, xp += 4 * sstride) {
+          float xv[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) xv[u] = xp[u * sstride + (uint32_t)jc];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) add(s + u, xv[u]);
+        }
+        for (; s <= sh; ++s, xp += sstride) add(s, xp[(uint32_t)jc]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RC; ++r)
+    if (R0 + r < g.nrows) {
+      float* o = a.gbar + ((size_t)v * g.nrows + R0 + r) * b.cpitch + ch;
+      const float s = lrow[(R0 + r - rlo) * 64];
+      if (q.nsplit > 1)
+        unsafeAtomicAdd(o, s);
+      else
+        *o = s;
+    }
+}
+
 // Transpose of the rebinning: one block per parallel line (j, effective row
 // q), threads over its channels; the same clamped (focal state, projection,
 // raw row, fan channel) addressing as rebin_filter.hip's gather.
@@ -189,6 +494,56 @@ hipError_t launch_backproject_adjoint(const BpAdjArgs& a, int tile_z, hipStream_
     case 32: return launch_tz<32>(a, s, matched);
   }
   return hipErrorInvalidValue;
+}
+
+hipError_t launch_adjoint_columns(const BpAdjArgs& a, const AdjGather& q, hipStream_t s) {
+  hipLaunchKernelGGL(bp_adjoint_column_kernel,
+                     dim3((a.bp.nx * a.bp.ny + 255) / 256, std::min(q.nt, 65535)), dim3(256), 0, s,
+                     a, q);
+  return hipGetLastError();
+}
+
+hipError_t launch_adjoint_weights(const BpAdjArgs& a, const AdjGather& q, hipStream_t s) {
+  const int ns = q.swap ? a.bp.ny : a.bp.nx, np = q.swap ? a.bp.nx : a.bp.ny;
+  const dim3 grid((unsigned)((ns + 63) / 64 * np *
+                             ((a.bp.n_native + kAdjSlices - 1) / kAdjSlices)));
+  if (a.bp.g.cr == a.bp.g.hr)
+    hipLaunchKernelGGL(bp_adjoint_weights_kernel<true>, grid, dim3(64), 0, s, a, q);
+  else
+    hipLaunchKernelGGL(bp_adjoint_weights_kernel<false>, grid, dim3(64), 0, s, a, q);
+  return hipGetLastError();
+}
+
+hipError_t launch_swap_volume(const float* in, float* out, int nx, int ny, int nz, hipStream_t s) {
+  hipLaunchKernelGGL(swap_volume_kernel,
+                     dim3((nx + 31) / 32, (ny + 31) / 32, std::min(nz, 65535)), dim3(256), 0, s,
+                     in, out, nx, ny, nz);
+  return hipGetLastError();
+}
+
+int adjoint_gather_waves(const BpArgs& b) {   // waves per theta~
+  const int rc = b.g.nrows <= 16 ? 16 : 32;
+  return (b.cpitch / 64) * ((b.g.nrows + rc - 1) / rc) * ((b.nviews + b.H - 1) / b.H);
+}
+
+template <int RC, bool C>
+hipError_t launch_gather_rc(const BpAdjArgs& a, const AdjGather& q, bool matched, hipStream_t s) {
+  const dim3 grid((unsigned)(adjoint_gather_waves(a.bp) * q.nt * q.nsplit));
+  if (matched)
+    hipLaunchKernelGGL((bp_adjoint_gather_kernel<RC, C, true>), grid, dim3(64), 0, s, a, q);
+  else
+    hipLaunchKernelGGL((bp_adjoint_gather_kernel<RC, C, false>), grid, dim3(64), 0, s, a, q);
+  return hipGetLastError();
+}
+
+hipError_t launch_adjoint_gather(const BpAdjArgs& a, const AdjGather& q, bool matched,
+                                 hipStream_t s) {
+  const bool c = a.bp.g.cr == a.bp.g.hr;
+  if (a.bp.g.nrows <= 16)
+    return c ? launch_gather_rc<16, true>(a, q, matched, s)
+             : launch_gather_rc<16, false>(a, q, matched, s);
+  return c ? launch_gather_rc<32, true>(a, q, matched, s)
+           : launch_gather_rc<32, false>(a, q, matched, s);
 }
 
 hipError_t launch_rebin_adjoint(const RebinAdjArgs& a, hipStream_t s) {

@@ -158,7 +158,7 @@ void free_plan_buffers(fct_wfbp_gpu_plan* p) {
                   p->d_slab_vrange, p->d_rebin,  p->d_Hn,        p->d_tw,       p->d_thk_off,
                   p->d_thk_idx,  p->d_thk_w,     p->d_filtered,  p->d_scale, p->d_native,
                   p->d_raw_stage, p->d_vol_stage, p->d_gbar, p->d_thkT_off, p->d_thkT_idx,
-                  p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_ray_tab, p->d_ray_pad, p->d_ray_rec, p->d_af_raw, p->d_af_vmax};
+                  p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_ray_tab, p->d_ray_pad, p->d_ray_rec, p->d_adj_wgt, p->d_af_raw, p->d_af_vmax};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (int b = 0; b < 2; ++b)
@@ -332,6 +332,62 @@ bool ray_tables(fct_wfbp_gpu_plan* p, const fct::RayProjArgs& a, fct::RayTables*
   if (!p->ray_tab_ready) {
     if (fct::launch_ray_table(a, *t, p->stream) != hipSuccess) return false;
     p->ray_tab_ready = true;
+  }
+  return true;
+}
+
+// The transposed backprojection (or matched projection) as a gather, theta~
+// batch by batch; false: not taken (no scratch), nothing launched.
+bool adjoint_gather(fct_wfbp_gpu_plan* p, const fct::BpAdjArgs& a, bool matched, hipError_t* err) {
+  *err = hipSuccess;
+  const size_t vol = (size_t)p->n_native * p->recon.ny * p->recon.nx;
+  const size_t cols = (size_t)p->recon.ny * p->recon.nx;
+  // Column tables (4 floats per column) and voxel weights of enough theta~ for
+  // about 4096 waves of the gather, within 2 GiB (at least one theta~).
+  const int waves = std::max(1, fct::adjoint_gather_waves(a.bp));
+  const size_t per = 4 * cols + (matched ? 0 : vol);
+  size_t nt = std::min<size_t>(p->H, (4096 + waves - 1) / waves);
+  nt = std::max<size_t>(1, std::min<size_t>(nt, ((size_t)2 << 30) / (per * sizeof(float))));
+  const size_t need = nt * per + (matched ? vol : 0);
+  const double lines = (double)((p->recon.nx + 63) / 64) * p->recon.ny +
+                       (double)((p->recon.ny + 63) / 64) * p->recon.nx;
+  if ((double)waves * p->H * 16 >= 2147483647.0 || lines * p->n_native >= 2147483647.0) return false;
+  if (p->adj_wgt_elems < need) {
+    float* d = static_cast<float*>(try_scratch(p, need * sizeof(float)));
+    if (!d) return false;
+    if (p->d_adj_wgt) (void)hipFree(p->d_adj_wgt);   // (waits for the work that reads it)
+    p->d_adj_wgt = d;
+    p->adj_wgt_elems = need;
+  }
+  const fct::RayProjArgs r = ray_args(p);
+  fct::AdjGather q{};
+  q.col = reinterpret_cast<float4*>(p->d_adj_wgt);
+  q.wgt = p->d_adj_wgt + nt * 4 * cols;
+  q.tile_z = p->tile_z;
+  q.gx0 = r.dx0;
+  q.gdx = r.ddx;
+  q.gy0 = r.dy0;
+  q.gdy = r.ddy;
+  q.dz = r.ddz;
+  // The views of a batch differ in how many slices they see, and a wave's whole
+  // ray is as long as the launch: the planes of a ray are shared by several
+  // waves, towards 65536 per launch (4096 x 16 rather than one wave per ray:
+  // 2952 views x 16 x 736 from 384 x 384 x 32 voxels 18.7 -> 10.8 ms).
+  const long long launch = (long long)waves * (long long)nt;
+  const int np = std::min(p->recon.nx, p->recon.ny);
+  q.nsplit = (int)std::max(1LL, std::min<long long>(np / 16, (65536 + launch - 1) / launch));
+  if (q.nsplit > 1)
+    *err = fct::launch_fill(a.gbar, (size_t)p->nviews * p->nrows * p->cpitch, 0.0f, p->stream);
+  if (matched && *err == hipSuccess)
+    *err = fct::launch_swap_volume(a.xbar, q.wgt, p->recon.nx, p->recon.ny, p->n_native, p->stream);
+  for (int t = 0; t < p->H && *err == hipSuccess; t += q.nt) {
+    q.t0 = t;
+    q.swap = p->h_xplanes[t];
+    q.nt = 1;
+    while (t + q.nt < p->H && q.nt < (int)nt && p->h_xplanes[t + q.nt] == q.swap) ++q.nt;
+    *err = fct::launch_adjoint_columns(a, q, p->stream);
+    if (!matched && *err == hipSuccess) *err = fct::launch_adjoint_weights(a, q, p->stream);
+    if (*err == hipSuccess) *err = fct::launch_adjoint_gather(a, q, matched, p->stream);
   }
   return true;
 }
@@ -940,6 +996,8 @@ FCT_API int fct_wfbp_gpu_plan_create(fct_wfbp_gpu_ctx* ctx, const fct_scan_geome
   std::vector<float2> cs(p->H);
   const double angle0 = cw ? -s.angle0 : s.angle0;
   for (int t = 0; t < p->H; ++t) fct_tables::view_cos_sin(angle0, p->dtheta, t, &cs[t].x, &cs[t].y);
+  p->h_xplanes.resize(p->H);
+  for (int t = 0; t < p->H; ++t) p->h_xplanes[t] = std::fabs(cs[t].x) >= std::fabs(cs[t].y);
 
   std::vector<int2> vr;
   if (!slab_view_ranges(p, zn, p->tile_z, &vr))
@@ -1335,12 +1393,17 @@ FCT_API int fct_wfbp_gpu_backproject_adjoint(fct_wfbp_gpu_plan* p, const float* 
                                              float* filtered_bar) {
   if (!p || !native_bar || !filtered_bar) return FCT_ERR_INVALID_ARGUMENT;
   HIP_TRY(p->ctx, hipSetDevice(p->device));
-  HIP_TRY(p->ctx, fct::launch_fill(filtered_bar, (size_t)p->nviews * p->nrows * p->cpitch, 0.0f,
-                                   p->stream));
   fct::BpAdjArgs a{};
   a.bp = bp_args(p);
   a.xbar = native_bar;
   a.gbar = filtered_bar;
+  hipError_t e;
+  if (adjoint_gather(p, a, false, &e)) {
+    HIP_TRY(p->ctx, e);
+    return FCT_OK;
+  }
+  HIP_TRY(p->ctx, fct::launch_fill(filtered_bar, (size_t)p->nviews * p->nrows * p->cpitch, 0.0f,
+                                   p->stream));
   HIP_TRY(p->ctx, fct::launch_backproject_adjoint(a, p->tile_z, p->stream));
   return FCT_OK;
 }
@@ -1349,12 +1412,17 @@ FCT_API int fct_wfbp_gpu_matched_project(fct_wfbp_gpu_plan* p, const float* nati
                                          float* lines) {
   if (!p || !native || !lines) return FCT_ERR_INVALID_ARGUMENT;
   HIP_TRY(p->ctx, hipSetDevice(p->device));
-  HIP_TRY(p->ctx, fct::launch_fill(lines, (size_t)p->nviews * p->nrows * p->cpitch, 0.0f,
-                                   p->stream));
   fct::BpAdjArgs a{};
   a.bp = bp_args(p);
   a.xbar = native;
   a.gbar = lines;
+  hipError_t e;
+  if (adjoint_gather(p, a, true, &e)) {
+    HIP_TRY(p->ctx, e);
+    return FCT_OK;
+  }
+  HIP_TRY(p->ctx, fct::launch_fill(lines, (size_t)p->nviews * p->nrows * p->cpitch, 0.0f,
+                                   p->stream));
   HIP_TRY(p->ctx, fct::launch_backproject_adjoint(a, p->tile_z, p->stream, true));
   return FCT_OK;
 }

@@ -174,6 +174,15 @@ struct BpAdjArgs {
   float* gbar;               // [view][row][cpitch] FP32, accumulated into
 };
 
+// Gathered transpose of the backprojection (adjoint.hip) for the theta~
+// [t0, t0 + nt), all with the same primary axis (x planes: swap 1).
+struct AdjGather {
+  float* wgt;      // [nt][primary][slice][secondary] xbar scale / sum W; matched: the volume, swapped
+  float4* col;     // [nt][primary][secondary] per-column geometry (bp_adjoint_column_kernel)
+  int32_t t0, nt, swap, tile_z, nsplit;   // nsplit: waves sharing a ray's planes
+  double gx0, gdx, gy0, gdy, dz;   // voxel-centre grid, slice step (mm, signed)
+};
+
 struct RebinAdjArgs {
   const float* gbar;         // [view][row][cpitch] (parallel, effective detector)
   float* pbar;               // [raw view][raw row][raw ch], accumulated into
@@ -216,6 +225,15 @@ hipError_t launch_quad_rescale(void* quads, size_t n_entries, int precision, con
                                int ncu, hipStream_t s);
 hipError_t launch_backproject_adjoint(const BpAdjArgs& a, int tile_z, hipStream_t s,
                                       bool matched = false);
+// The gathered form of launch_backproject_adjoint, theta~ batch by batch: the
+// column table, the voxels' weights (not for the matched projector, which reads the volume,
+// swapped for x planes), then the detector samples (gbar overwritten).
+hipError_t launch_adjoint_columns(const BpAdjArgs& a, const AdjGather& q, hipStream_t s);
+hipError_t launch_adjoint_weights(const BpAdjArgs& a, const AdjGather& q, hipStream_t s);
+hipError_t launch_swap_volume(const float* in, float* out, int nx, int ny, int nz, hipStream_t s);
+int adjoint_gather_waves(const BpArgs& b);   // waves per theta~
+hipError_t launch_adjoint_gather(const BpAdjArgs& a, const AdjGather& q, bool matched,
+                                 hipStream_t s);
 hipError_t launch_rebin_adjoint(const RebinAdjArgs& a, hipStream_t s);
 hipError_t launch_fill(float* p, size_t n, float v, hipStream_t s);
 hipError_t launch_backproject(const BpArgs& a, int tile_z, int variant, int precision, int mode,
@@ -307,6 +325,9 @@ struct fct_wfbp_gpu_plan {
   bool ray_tab_ready = false;
   float* d_ray_pad = nullptr;       // padded volume copies of the ray projector (first use)
   float* d_ray_rec = nullptr;       // per-ray records of its transpose (first use)
+  float* d_adj_wgt = nullptr;       // gathered transpose: voxel weights / swapped volume (first use)
+  size_t adj_wgt_elems = 0;
+  std::vector<uint8_t> h_xplanes;   // per theta~: its parallel rays run along x planes
   float* d_gbar = nullptr;          // adjoint scratch, [view][row][cpitch] FP32
   int32_t* d_thkT_off = nullptr;    // transposed thickening table
   int32_t* d_thkT_idx = nullptr;

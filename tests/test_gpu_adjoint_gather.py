@@ -1,0 +1,68 @@
+"""The gathered transposes of the backprojection and of the matched projector
+against the scattering kernels, which a graph capture on a fresh plan records
+(no scratch may be allocated inside a capture).  Both take the same FP32
+selection and weights, so they differ by summation order and by the products'
+rounding only: a few ulps of a detector sample's sum of up to a few thousand
+terms, bounded here by 1e-5 of the largest sample.  The shapes are those where
+the gather can go wrong: detector rows that leave a remainder after 16 or 32,
+an off-centre row, more slices than one chunk of 64, matrices of one column
+group more than 64, fine and coarse voxels, a falling slice grid, FFS.
+"""
+import pytest
+
+from freect_amd import scans as S
+from helpers import gpu_ctx
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return gpu_ctx()
+
+
+CASES = [dict(nx=32, ny=32, n_slices=8, n_rows=8),
+         dict(nx=65, ny=20, n_slices=9, n_rows=17, fov=350.0),
+         dict(nx=20, ny=70, n_slices=66, n_rows=16, fov=120.0, rotations=6.0, tile_z=4),
+         dict(nx=40, ny=40, n_slices=12, n_rows=33, cr=0.3, rotation=-1),
+         dict(nx=130, ny=130, n_slices=3, n_rows=9, fov=200.0, flip=True),
+         dict(nx=24, ny=31, n_slices=10, n_rows=12, ffs=3, ppr=192),
+         dict(nx=16, ny=16, n_slices=1, n_rows=5, rotations=0.3)]
+
+
+def _plan(ctx, nx, ny, n_slices, n_rows, fov=400.0, rotations=2.3, tile_z=8, cr=0.0, rotation=1,
+          flip=False, ffs=0, ppr=96):
+    from freect_amd import wfbp
+    w = S.tiny(nx=nx, n_slices=n_slices, n_channels=96, n_rows=n_rows, ppr=ppr,
+               rotations=rotations, ffs_mode=ffs)
+    sc = w.scan.replace(rotation=rotation, central_row=w.scan.central_row + cr)
+    rc = w.recon.replace(ny=ny, recon_fov=fov, x_origin=3.0)
+    if flip:
+        rc = rc.replace(start_pos=rc.end_pos, end_pos=rc.start_pos)
+    return wfbp.Plan(ctx, sc, rc, tile_z=tile_z)
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+@pytest.mark.parametrize("op", ["backproject_adjoint", "matched_project"])
+def test_gather_equals_scatter(ctx, case, op):
+    p, general = _plan(ctx, **CASES[case]), _plan(ctx, **CASES[case])
+    gen = torch.Generator(device="cuda").manual_seed(case)
+    x = torch.rand((p.info.n_slices_native, p.recon.ny, p.recon.nx), device="cuda",
+                   generator=gen) + 0.1
+    got, ref = p.alloc_lines().fill_(float("nan")), p.alloc_lines()
+    for _ in range(2):   # with and without the first use's allocation
+        getattr(p, op)(x, got)
+    s = torch.cuda.Stream()
+    general.set_stream(s)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        getattr(general, op)(x, ref)
+    for _ in range(2):
+        g.replay()
+        torch.cuda.synchronize()
+        assert ref.abs().max() > 0
+        assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
