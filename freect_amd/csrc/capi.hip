@@ -155,7 +155,7 @@ int validate(fct_wfbp_gpu_ctx* ctx, const fct_scan_geometry* s, const fct_recon_
 
 void free_plan_buffers(fct_wfbp_gpu_plan* p) {
   void* bufs[] = {p->d_xs,       p->d_ys,        p->d_cs,        p->d_zs,       p->d_zt,
-                  p->d_slab_vrange, p->d_rebin,  p->d_Hn,        p->d_tw,       p->d_thk_off,
+                  p->d_slab_vrange, p->d_rebin, p->d_rebinT,  p->d_Hn,        p->d_tw,       p->d_thk_off,
                   p->d_thk_idx,  p->d_thk_w,     p->d_filtered,  p->d_scale, p->d_native,
                   p->d_raw_stage, p->d_vol_stage, p->d_gbar, p->d_thkT_off, p->d_thkT_idx,
                   p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_ray_tab, p->d_ray_pad, p->d_ray_rec, p->d_adj_wgt, p->d_af_raw, p->d_af_vmax};
@@ -1059,6 +1059,31 @@ FCT_API int fct_wfbp_gpu_plan_create(fct_wfbp_gpu_ctx* ctx, const fct_scan_geome
       if (e.valid)
         p->rebin_reach = std::max(p->rebin_reach, (e.aoff + 1) * p->ffs.S + e.rho + 1);
     }
+  // The same table by the raw (focal state, channel) it reads, for the
+  // transpose: the entries, then the offsets of each channel's.
+  std::vector<fct::RebinTDev> tabT;
+  {
+    const int n = p->raw_scan.n_channels, keys = p->ffs.S * n;
+    std::vector<std::vector<fct::RebinTDev>> per(keys);
+    for (int zb = 0; zb < zpar; ++zb)
+      for (int c = 0; c < p->ncols; ++c) {
+        const fct::RebinDev& e = tab[(size_t)zb * p->ncols + c];
+        if (!e.state) continue;
+        auto& lo = per[(e.state - 1) * n + e.b0];
+        lo.push_back(fct::RebinTDev{c | zb << 16, e.aoff, e.fa, 1.0f - e.fb});
+        per[(e.state - 1) * n + e.b1].push_back(fct::RebinTDev{c | zb << 16, e.aoff, e.fa, e.fb});
+      }
+    std::vector<int32_t> off(1, 0);
+    for (const auto& l : per) {
+      tabT.insert(tabT.end(), l.begin(), l.end());
+      off.push_back((int32_t)tabT.size());
+    }
+    p->rebinT_entries = (int)tabT.size();
+    tabT.resize(tabT.size() + (off.size() * sizeof(int32_t) + sizeof(fct::RebinTDev) - 1) /
+                                  sizeof(fct::RebinTDev));
+    std::memcpy(static_cast<void*>(tabT.data() + p->rebinT_entries), off.data(),
+                off.size() * sizeof(int32_t));
+  }
   // The gather addresses a line pair's taps by 32-bit offsets from the first
   // view group they can reach (rebin_filter.hip): the groups of the table's
   // aoff span (+ 4: the pair's second view, the interpolation's next view,
@@ -1165,6 +1190,7 @@ FCT_API int fct_wfbp_gpu_plan_create(fct_wfbp_gpu_ctx* ctx, const fct_scan_geome
   PLAN_TRY(upload(&p->d_wrange, wrange, p->stream));
   PLAN_TRY(upload(&p->d_rebin, tab, p->stream));
   p->h_rebin = tab;
+  PLAN_TRY(upload(&p->d_rebinT, tabT, p->stream));
   PLAN_TRY(upload(&p->d_Hn, Hn, p->stream));
   PLAN_TRY(upload(&p->d_tw, tw, p->stream));
   PLAN_TRY(upload(&p->d_thk_off, toff, p->stream));
@@ -1443,15 +1469,15 @@ FCT_API int fct_wfbp_gpu_rebin_adjoint(fct_wfbp_gpu_plan* p, const float* filter
                                        float* raw_bar) {
   if (!p || !filtered_bar || !raw_bar) return FCT_ERR_INVALID_ARGUMENT;
   HIP_TRY(p->ctx, hipSetDevice(p->device));
-  HIP_TRY(p->ctx, fct::launch_fill(raw_bar, (size_t)p->raw_elems(), 0.0f, p->stream));
   fct::RebinAdjArgs a{};
   a.gbar = filtered_bar;
   a.pbar = raw_bar;
-  a.tab = p->d_rebin;
+  a.ent = p->d_rebinT;
+  a.off = reinterpret_cast<const int32_t*>(p->d_rebinT + p->rebinT_entries);
   a.nviews = p->nviews;
   a.nrows = p->nrows;
-  a.ncols = p->ncols;
   a.cpitch = p->cpitch;
+  a.raw_nviews = p->raw_scan.n_views;
   a.raw_nrows = p->raw_scan.n_rows;
   a.raw_ncols = p->raw_scan.n_channels;
   a.states = p->ffs.S;

@@ -43,6 +43,14 @@ __device__ __forceinline__ float fp16_channel_weight(float wp) {
   return __builtin_rintf(wp * 2048.0f) * (1.0f / 2048.0f);
 }
 
+// The rebinning table by the raw channel it reads: parallel channel c (low 16
+// bits) and effective-row parity (high), view offset, and the weights of the
+// second view and of this raw channel.
+struct RebinTDev {
+  int32_t c, aoff;
+  float fa, wb;
+};
+
 // Everything the rebin + filter kernel reads.
 struct RebinFilterArgs {
   const float* raw;          // [view][row][ncols]
@@ -185,10 +193,11 @@ struct AdjGather {
 
 struct RebinAdjArgs {
   const float* gbar;         // [view][row][cpitch] (parallel, effective detector)
-  float* pbar;               // [raw view][raw row][raw ch], accumulated into
-  const RebinDev* tab;
-  int32_t nviews, nrows, ncols, cpitch;   // parallel views, effective rows / channels
-  int32_t raw_nrows, raw_ncols, states, zshift;
+  float* pbar;               // [raw view][raw row][raw ch], overwritten
+  const int32_t* off;        // [states * raw_ncols + 1] into ent
+  const RebinTDev* ent;
+  int32_t nviews, nrows, cpitch;          // parallel views, effective rows
+  int32_t raw_nviews, raw_nrows, raw_ncols, states, zshift;
 };
 
 hipError_t launch_rebin_filter(const RebinFilterArgs& a, hipStream_t s);
@@ -309,6 +318,8 @@ struct fct_wfbp_gpu_plan {
   int2* d_wrange = nullptr;
   float4* d_zbounds = nullptr;
   fct::RebinDev* d_rebin = nullptr;
+  fct::RebinTDev* d_rebinT = nullptr;   // by raw channel; its offsets follow the entries
+  int rebinT_entries = 0;
   float* d_Hn = nullptr;
   float2* d_tw = nullptr;
   int32_t* d_thk_off = nullptr;

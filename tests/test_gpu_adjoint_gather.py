@@ -66,3 +66,26 @@ def test_gather_equals_scatter(ctx, case, op):
         torch.cuda.synchronize()
         assert ref.abs().max() > 0
         assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("views,channels,rows,ffs", [(1, 70, 3, 0), (5, 96, 8, 0), (40, 200, 5, 0),
+                                                     (8, 64, 4, 3), (130, 65, 9, 2)])
+def test_rebin_transpose_at_the_scan_ends(ctx, oracle, views, channels, rows, ffs):
+    # Scans shorter than the fan's reach, where most samples go to a clamped
+    # first or last projection.  Sums of at most `views` terms per entry, FP32
+    # weights: 1e-5 of the largest.
+    import numpy as np
+
+    from freect_amd import wfbp
+    w = S.tiny(nx=8, n_slices=2, n_channels=channels, n_rows=rows, ppr=192, rotations=1.0,
+               ffs_mode=ffs)
+    sc = w.scan.replace(n_views=views)
+    p = wfbp.Plan(ctx, sc, w.recon)
+    i = p.info
+    g = np.random.RandomState(views).standard_normal(
+        (i.n_parallel_views, i.n_filtered_rows, i.channel_pitch)).astype(np.float32)
+    out = p.alloc_raw().fill_(float("nan"))
+    p.rebin_adjoint(torch.from_numpy(g).cuda(), out)
+    p.synchronize()
+    ref = oracle.rebin_adjoint(sc, g[..., : i.n_filtered_channels].astype(np.float64))
+    assert np.abs(out.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
