@@ -32,6 +32,8 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+
 #include "wave_ops.h"
 #include "wfbp_internal.h"
 
@@ -337,11 +339,19 @@ __device__ __forceinline__ int2 tile_of(int l, int tiles_x, int tiles_y) {
   return make_int2(sx * kSuper + r2 % w, sy * kSuper + r2 / w);
 }
 
-// One wave reconstructs tile `lin` (slab-major order) of the job described by a.
-template <int TZ, int PREC, int MODE, bool CENTERED>
-__device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin) {
+// How the theta~ of a tile are summed: in one sweep; in a.nseg consecutive
+// segments by as many waves of a workgroup (their sums added in segment
+// order through LDS); or in the same segments one after the other by one
+// wave (the persistent kernel), which gives bitwise the same volume.
+enum BpSplit { kSweep = 0, kSplitWaves = 1, kSplitSerial = 2 };
+
+// One wave reconstructs tile `lin` (slab-major order) of the job described by
+// a; with kSplitWaves its theta~ segment `wave`.  lds: kSplitWaves (nseg - 1)
+// x min(TZ, 8) x 64 floats, kSplitSerial TZ x 64.
+template <int TZ, int PREC, int MODE, bool CENTERED, int SPLIT>
+__device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, float* lds) {
   constexpr uint32_t kEntry = ChanInterp<PREC>::kEntry;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int tiles = a.tiles_x * a.tiles_y;
   const int slab = lin / tiles;
   const int2 txy = tile_of(lin - slab * tiles, a.tiles_x, a.tiles_y);
@@ -356,7 +366,7 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin) {
   const int s0 = slab * TZ;
   const int nz = min(TZ, a.n_native - s0);
   if (!__any(active)) {
-    if (inb)
+    if (inb && wave == 0)
       for (int i = 0; i < nz; ++i) {
         const size_t o = ((size_t)(s0 + i) * a.ny + iy) * a.nx + ix;
         if (MODE == kBpAccumulate || MODE == kBpMatched) a.native[o] = 0.0f;
@@ -402,139 +412,168 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin) {
 
   float acc[TZ];
   int cnt[TZ];
-#pragma unroll
-  for (int i = 0; i < TZ; ++i) {
-    acc[i] = 0.0f;
-    cnt[i] = 0;
-  }
-  for (int t = 0; t < H; ++t) {
-    const int kmin = vr.x <= t ? 0 : (vr.x - t + H - 1) / H;
-    const int kmax = vr.y <= t ? 0 : (vr.y - t + H - 1) / H;
-    if (kmin >= kmax) continue;
-    const float* csp = reinterpret_cast<const float*>(a.cs + t);
-    const float2 cs = make_float2(ld_uniform(csp), ld_uniform(csp + 1));
-    const BpColumn col = bp_column(x, y, cs, g);
-    const float p = col.p, sq = col.sq, f = col.f, kb = col.kb;
-    // The tile's z-interval extremes for this theta~ (tabulated per plan).
-    const float* zbp = reinterpret_cast<const float*>(a.zbounds + (size_t)tile * H + t);
-    const float4 zb =
-        make_float4(ld_uniform(zbp), ld_uniform(zbp + 1), ld_uniform(zbp + 2), ld_uniform(zbp + 3));
-    float num[TZ], den[TZ];
+  int seg = SPLIT == kSplitWaves ? wave : 0;
+  do {
 #pragma unroll
     for (int i = 0; i < TZ; ++i) {
-      // 1e-30 is below half an ulp of any nonzero weight sum (W >= ~1e-13
-      // when a sample is selected), so den ends as the exact sum when a
-      // view contributes and 1e-30 (num = 0, no change to acc) otherwise.
-      // (Through an empty asm: as literals the compiler materialised both
-      // start values again at the view loop's entry, 32 instead of 14 moves
-      // per theta~.)
-      float zero = 0.0f, tiny = 1e-30f;
-      asm("" : "+v"(zero));
-      asm("" : "+v"(tiny));
-      num[i] = zero;
-      den[i] = tiny;
+      acc[i] = 0.0f;
+      cnt[i] = 0;
     }
+    const int t0 = SPLIT == kSweep ? 0 : H * seg / a.nseg;
+    const int t1 = SPLIT == kSweep ? H : H * (seg + 1) / a.nseg;
+    for (int t = t0; t < t1; ++t) {
+      const int kmin = vr.x <= t ? 0 : (vr.x - t + H - 1) / H;
+      const int kmax = vr.y <= t ? 0 : (vr.y - t + H - 1) / H;
+      if (kmin >= kmax) continue;
+      const float* csp = reinterpret_cast<const float*>(a.cs + t);
+      const float2 cs = make_float2(ld_uniform(csp), ld_uniform(csp + 1));
+      const BpColumn col = bp_column(x, y, cs, g);
+      const float p = col.p, sq = col.sq, f = col.f, kb = col.kb;
+      // The tile's z-interval extremes for this theta~ (tabulated per plan).
+      const float* zbp = reinterpret_cast<const float*>(a.zbounds + (size_t)tile * H + t);
+      const float4 zb =
+          make_float4(ld_uniform(zbp), ld_uniform(zbp + 1), ld_uniform(zbp + 2), ld_uniform(zbp + 3));
+      float num[TZ], den[TZ];
+#pragma unroll
+      for (int i = 0; i < TZ; ++i) {
+        // 1e-30 is below half an ulp of any nonzero weight sum (W >= ~1e-13
+        // when a sample is selected), so den ends as the exact sum when a
+        // view contributes and 1e-30 (num = 0, no change to acc) otherwise.
+        // (Through an empty asm: as literals the compiler materialised both
+        // start values again at the view loop's entry, 32 instead of 14 moves
+        // per theta~.)
+        float zero = 0.0f, tiny = 1e-30f;
+        asm("" : "+v"(zero));
+        asm("" : "+v"(tiny));
+        num[i] = zero;
+        den[i] = tiny;
+      }
 
 #pragma unroll
-    for (int par = 0; par < 2; ++par) {
-      int k = kmin + (((kmin & 1) != par) ? 1 : 0);
-      if (k >= kmax) continue;
-      const float pidx = par ? fmaf(-p, g.inv_ds, g.cc) : fmaf(p, g.inv_ds, g.cc);
-      const float lt = (par ? sq + f : sq - f) * g.tanc;
-      const float kbs = par ? -kb : kb;
-      const float pfl = floorf(pidx);
-      const bool chan_ok = active && pfl >= 0.0f && pfl <= (float)(g.ncols - 2);
-      // Rows per mm of z; 0 for the lanes parked off the detector (kFree).
-      const float invLh = kFree && !chan_ok ? 0.0f : div_rn_normal(g.hr, lt);
-      const uint32_t pf = chan_ok ? (uint32_t)(int)pfl : 0u;
-      const float wp = pidx - pfl;
-      // Matched mode: R / l, the voxel-driven footprint's depth correction
-      // (a row spans drow l / Dsd of z at distance l from the source).
-      const float fR = MODE == kBpMatched ? g.tanc / (lt * g.invR) : 0.0f;
-      // z-interval of |q| <= 1 relative to the view's table z, over the wave.
-      const float A = par ? zb.z : zb.x;
-      const float B = par ? zb.w : zb.y;
-      // Slice positions of the interval ends for a view at table z ztv:
-      // ztv * inv_dzs + c, the lower end first (A <= B, so the order is
-      // that of the slice step's sign).
-      const float ca = (A - zfirst) * inv_dzs, cb = (B - zfirst) * inv_dzs;
-      const float clo = inv_dzs > 0.0f ? ca : cb, nchi = -(inv_dzs > 0.0f ? cb : ca);
-      for (; k < kmax; k += 2) {
-        const int v = t + k * H;
-        const float ztv = ld_uniform(ztc + v);
-        // Exact window slice range (native indices).
-        const int2 wr = make_int2(ld_uniform(wrc + 2 * v), ld_uniform(wrc + 2 * v + 1));
-        // One slice of margin on each side covers the rounding of these
-        // positions; the per-sample test below is exact.
-        const int flo = floor_int(fmaf(ztv, inv_dzs, clo));
-        const int fhi = floor_int(fmaf(ztv, ninv_dzs, nchi));   // -ceil(upper end)
-        // (The matched projector pair uses every view that sees the voxel:
-        // no view window.)
-        const int ilo = max(max(0, flo - 1), MODE == kBpMatched ? 0 : wr.x - s0);
-        const int ihi = min(min(nz - 1, 1 - fhi), MODE == kBpMatched ? nz - 1 : wr.y - s0);
-        if (ilo > ihi) {
-          if (can_stop && (up ? ilo > nz - 1 : ihi < 0)) break;
-          continue;
-        }
-        const float row0 =                                 // fct_bp_row0
-            kFree && !chan_ok ? -1.0e30f : fmaf(kbs - ztv, invLh, g.cr);
-        ChanInterp<PREC> ci;
-        ci.init((uint32_t)(v - vr.x) * vstride * kEntry, pf, wp);
-        if (ilo == 0 && ihi == nz - 1) {
-          // Every slice of the slab (the common case): no per-slice branch,
-          // and the taps of four slices are in flight before the first is
-          // used (four, not TZ: more would cost waves per SIMD).  With
-          // nz < TZ the extra slices repeat the last one and are not stored.
-          // Centred WFBP sums take the weight without a selection mask
-          // (bp_weight; the lanes off the detector are parked at row -1e30).
-#pragma unroll
-          for (int h = 0; h < TZ; h += 4) {
-            BpTap<PREC> tap[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              tap[i] = bp_fetch<PREC, MODE, CENTERED>(zs[h + i], invLh, row0, ci, rf, rowB,
-                                                      chan_ok, g);
-            // FP16: the four loads are issued before the weight arithmetic
-            // that waits for them (the scheduler would sink them otherwise).
-            if (PREC == FCT_PRECISION_FP16) __builtin_amdgcn_sched_barrier(0);
-            bp_add4<PREC, MODE, kFree>(tap, ci, fR, g, num + h, den + h, cnt + h);
+      for (int par = 0; par < 2; ++par) {
+        int k = kmin + (((kmin & 1) != par) ? 1 : 0);
+        if (k >= kmax) continue;
+        const float pidx = par ? fmaf(-p, g.inv_ds, g.cc) : fmaf(p, g.inv_ds, g.cc);
+        const float lt = (par ? sq + f : sq - f) * g.tanc;
+        const float kbs = par ? -kb : kb;
+        const float pfl = floorf(pidx);
+        const bool chan_ok = active && pfl >= 0.0f && pfl <= (float)(g.ncols - 2);
+        // Rows per mm of z; 0 for the lanes parked off the detector (kFree).
+        const float invLh = kFree && !chan_ok ? 0.0f : div_rn_normal(g.hr, lt);
+        const uint32_t pf = chan_ok ? (uint32_t)(int)pfl : 0u;
+        const float wp = pidx - pfl;
+        // Matched mode: R / l, the voxel-driven footprint's depth correction
+        // (a row spans drow l / Dsd of z at distance l from the source).
+        const float fR = MODE == kBpMatched ? g.tanc / (lt * g.invR) : 0.0f;
+        // z-interval of |q| <= 1 relative to the view's table z, over the wave.
+        const float A = par ? zb.z : zb.x;
+        const float B = par ? zb.w : zb.y;
+        // Slice positions of the interval ends for a view at table z ztv:
+        // ztv * inv_dzs + c, the lower end first (A <= B, so the order is
+        // that of the slice step's sign).
+        const float ca = (A - zfirst) * inv_dzs, cb = (B - zfirst) * inv_dzs;
+        const float clo = inv_dzs > 0.0f ? ca : cb, nchi = -(inv_dzs > 0.0f ? cb : ca);
+        for (; k < kmax; k += 2) {
+          const int v = t + k * H;
+          const float ztv = ld_uniform(ztc + v);
+          // Exact window slice range (native indices).
+          const int2 wr = make_int2(ld_uniform(wrc + 2 * v), ld_uniform(wrc + 2 * v + 1));
+          // One slice of margin on each side covers the rounding of these
+          // positions; the per-sample test below is exact.
+          const int flo = floor_int(fmaf(ztv, inv_dzs, clo));
+          const int fhi = floor_int(fmaf(ztv, ninv_dzs, nchi));   // -ceil(upper end)
+          // (The matched projector pair uses every view that sees the voxel:
+          // no view window.)
+          const int ilo = max(max(0, flo - 1), MODE == kBpMatched ? 0 : wr.x - s0);
+          const int ihi = min(min(nz - 1, 1 - fhi), MODE == kBpMatched ? nz - 1 : wr.y - s0);
+          if (ilo > ihi) {
+            if (can_stop && (up ? ilo > nz - 1 : ihi < 0)) break;
+            continue;
           }
-        } else if constexpr (PREC == FCT_PRECISION_FP16) {
-          // Part of the slab, FP16: groups of four slices that meet
-          // [ilo, ihi] through the dot block, the slices outside the range
-          // masked like unselected samples (cheaper than per-slice samples
-          // with the two-address dot form; for FP32 / BF16 the masked slices
-          // cost more than they save).
+          const float row0 =                                 // fct_bp_row0
+              kFree && !chan_ok ? -1.0e30f : fmaf(kbs - ztv, invLh, g.cr);
+          ChanInterp<PREC> ci;
+          ci.init((uint32_t)(v - vr.x) * vstride * kEntry, pf, wp);
+          if (ilo == 0 && ihi == nz - 1) {
+            // Every slice of the slab (the common case): no per-slice branch,
+            // and the taps of four slices are in flight before the first is
+            // used (four, not TZ: more would cost waves per SIMD).  With
+            // nz < TZ the extra slices repeat the last one and are not stored.
+            // Centred WFBP sums take the weight without a selection mask
+            // (bp_weight; the lanes off the detector are parked at row -1e30).
 #pragma unroll
-          for (int h = 0; h < TZ; h += 4) {
-            if (ilo > h + 3 || ihi < h) continue;
-            BpTap<PREC> tap[4];
+            for (int h = 0; h < TZ; h += 4) {
+              BpTap<PREC> tap[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              tap[i] = bp_fetch<PREC, MODE, CENTERED>(zs[h + i], invLh, row0, ci, rf, rowB,
-                                                      chan_ok && h + i >= ilo && h + i <= ihi, g);
-            __builtin_amdgcn_sched_barrier(0);
-            bp_add4<PREC, MODE>(tap, ci, fR, g, num + h, den + h, cnt + h);
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < TZ; ++i)
-            if (i >= ilo && i <= ihi) {
-              const BpTap<PREC> tp =
-                  bp_fetch<PREC, MODE, CENTERED>(zs[i], invLh, row0, ci, rf, rowB, chan_ok, g);
-              bp_add<PREC, MODE>(tp, ci, fR, g, num[i], den[i], cnt[i]);
+              for (int i = 0; i < 4; ++i)
+                tap[i] = bp_fetch<PREC, MODE, CENTERED>(zs[h + i], invLh, row0, ci, rf, rowB,
+                                                        chan_ok, g);
+              // FP16: the four loads are issued before the weight arithmetic
+              // that waits for them (the scheduler would sink them otherwise).
+              if (PREC == FCT_PRECISION_FP16) __builtin_amdgcn_sched_barrier(0);
+              bp_add4<PREC, MODE, kFree>(tap, ci, fR, g, num + h, den + h, cnt + h);
             }
+          } else if constexpr (PREC == FCT_PRECISION_FP16) {
+            // Part of the slab, FP16: groups of four slices that meet
+            // [ilo, ihi] through the dot block, the slices outside the range
+            // masked like unselected samples (cheaper than per-slice samples
+            // with the two-address dot form; for FP32 / BF16 the masked slices
+            // cost more than they save).
+#pragma unroll
+            for (int h = 0; h < TZ; h += 4) {
+              if (ilo > h + 3 || ihi < h) continue;
+              BpTap<PREC> tap[4];
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                tap[i] = bp_fetch<PREC, MODE, CENTERED>(zs[h + i], invLh, row0, ci, rf, rowB,
+                                                        chan_ok && h + i >= ilo && h + i <= ihi, g);
+              __builtin_amdgcn_sched_barrier(0);
+              bp_add4<PREC, MODE>(tap, ci, fR, g, num + h, den + h, cnt + h);
+            }
+          } else {
+#pragma unroll
+            for (int i = 0; i < TZ; ++i)
+              if (i >= ilo && i <= ihi) {
+                const BpTap<PREC> tp =
+                    bp_fetch<PREC, MODE, CENTERED>(zs[i], invLh, row0, ci, rf, rowB, chan_ok, g);
+                bp_add<PREC, MODE>(tp, ci, fR, g, num[i], den[i], cnt[i]);
+              }
+          }
         }
       }
-    }
-    if (MODE == kBpAccumulate) {
+      if (MODE == kBpAccumulate) {
 #pragma unroll
-      for (int i = 0; i < TZ; ++i)
-        acc[i] = fmaf(num[i], __builtin_amdgcn_rcpf(den[i]), acc[i]);
-    } else if (MODE == kBpMatched) {
+        for (int i = 0; i < TZ; ++i)
+          acc[i] = fmaf(num[i], __builtin_amdgcn_rcpf(den[i]), acc[i]);
+      } else if (MODE == kBpMatched) {
 #pragma unroll
-      for (int i = 0; i < TZ; ++i) acc[i] += num[i];
+        for (int i = 0; i < TZ; ++i) acc[i] += num[i];
+      }
     }
+    if (SPLIT == kSplitSerial && a.nseg > 1) {
+#pragma unroll
+      for (int i = 0; i < TZ; ++i) {
+        if (seg > 0) acc[i] = lds[i * 64 + lane] + acc[i];
+        lds[i * 64 + lane] = acc[i];
+      }
+    }
+  } while (SPLIT == kSplitSerial && ++seg < a.nseg);
+  if (SPLIT == kSplitWaves) {
+    constexpr int kPart = TZ < 8 ? TZ : 8;
+#pragma unroll
+    for (int h = 0; h < TZ; h += kPart) {
+      if (h) __syncthreads();
+      if (wave > 0)
+#pragma unroll
+        for (int i = 0; i < kPart; ++i)
+          lds[((wave - 1) * kPart + i) * 64 + lane] = acc[h + i];
+      __syncthreads();
+      if (wave == 0)
+        for (int w = 0; w < a.nseg - 1; ++w)
+#pragma unroll
+          for (int i = 0; i < kPart; ++i) acc[h + i] += lds[(w * kPart + i) * 64 + lane];
+    }
+    if (wave > 0) return;
   }
   if (!inb) return;
   if (MODE == kBpAccumulate || MODE == kBpMatched) {
@@ -569,8 +608,19 @@ template <int TZ, int PREC, int MODE, bool CENTERED>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(TZ >= 8 ? bp_min_waves<TZ, PREC>() : 1, 8)))
 void bp_v1_kernel(BpArgs a) {
-  bp_v1_tile<TZ, PREC, MODE, CENTERED>(
-      a, a.slab0 * a.tiles_x * a.tiles_y + xcd_block(blockIdx.x, gridDim.x));
+  bp_v1_tile<TZ, PREC, MODE, CENTERED, kSweep>(
+      a, a.slab0 * a.tiles_x * a.tiles_y + xcd_block(blockIdx.x, gridDim.x), 0, nullptr);
+}
+
+// A workgroup of a.nseg waves per tile.
+template <int TZ, int PREC, int MODE, bool CENTERED>
+__global__ __launch_bounds__(64 * kBpMaxSegments)
+__attribute__((amdgpu_waves_per_eu(TZ >= 8 ? bp_min_waves<TZ, PREC>() : 1, 8)))
+void bp_v1_split_kernel(BpArgs a) {
+  extern __shared__ float bp_lds[];
+  bp_v1_tile<TZ, PREC, MODE, CENTERED, kSplitWaves>(
+      a, a.slab0 * a.tiles_x * a.tiles_y + xcd_block(blockIdx.x, gridDim.x),
+      __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), bp_lds);
 }
 
 // Persistent backprojection of many jobs in one launch.  The tiles of all
@@ -589,6 +639,7 @@ __attribute__((amdgpu_waves_per_eu(bp_min_waves<TZ, PREC>(), 8)))
 void bp_batch_kernel(BpBatchArgs b,
                                                       const BpArgs* __restrict__ jobs,
                                                       const int32_t* __restrict__ tile_start) {
+  __shared__ float lds[TZ * 64];
   const int xcd = blockIdx.x & 7;
   for (int step = 0; step < 8; ++step) {
     const int r = (xcd + step) & 7;
@@ -602,7 +653,8 @@ void bp_batch_kernel(BpBatchArgs b,
       int j = 0;   // job: last j with tile_start[j] <= tile
       for (int span = 32; span > 0; span >>= 1)
         if (j + span < b.n_jobs && ld_uniform(tile_start + j + span) <= tile) j += span;
-      bp_v1_tile<TZ, PREC, kBpAccumulate, CENTERED>(jobs[j], tile - ld_uniform(tile_start + j));
+      bp_v1_tile<TZ, PREC, kBpAccumulate, CENTERED, kSplitSerial>(
+          jobs[j], tile - ld_uniform(tile_start + j), 0, lds);
     }
   }
 }
@@ -610,6 +662,22 @@ void bp_batch_kernel(BpBatchArgs b,
 template <int TZ, int PREC, bool C>
 hipError_t launch3(const BpArgs& a, int mode, hipStream_t s) {
   const int blocks = a.tiles_x * a.tiles_y * (a.slab_count ? a.slab_count : a.nslabs);
+  if constexpr (TZ <= 16) {
+    if (a.nseg > 1 && mode == kBpAccumulate) {
+      hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks),
+                         dim3(64 * a.nseg), (a.nseg - 1) * std::min(TZ, 8) * 64 * sizeof(float), s,
+                         a);
+      return hipGetLastError();
+    }
+    if constexpr (PREC == FCT_PRECISION_FP32) {
+      if (a.nseg > 1 && mode == kBpMatched) {
+        hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks),
+                           dim3(64 * a.nseg), (a.nseg - 1) * std::min(TZ, 8) * 64 * sizeof(float),
+                           s, a);
+        return hipGetLastError();
+      }
+    }
+  }
   if (mode == kBpAccumulate)
     hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks), dim3(64), 0, s, a);
   else if (mode == kBpCount)

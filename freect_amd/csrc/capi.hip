@@ -245,6 +245,7 @@ BpArgs plan_bp_args(const fct_wfbp_gpu_plan* p) {
   a.tiles_x = (p->recon.nx + 7) / 8;
   a.tiles_y = (p->recon.ny + 7) / 8;
   a.nslabs = p->nslabs;
+  a.nseg = bp_segments(a.tiles_x * a.tiles_y, a.nslabs, a.H, p->tile_z);
   return a;
 }
 

@@ -110,7 +110,27 @@ struct BpArgs {
   // streaming reconstruction backprojects groups of slabs as their views
   // arrive.  Unused by the persistent batch kernel.
   int32_t slab0, slab_count;
+  int32_t nseg;              // theta~ segments summed apart (bp_segments)
 };
+constexpr int kBpMaxSegments = 16;
+
+// Segments of theta~ that a volume of so many tiles per slab sums apart, so
+// that a small volume still fills the GPU (a wave per tile and segment): a
+// power of two, up to 16 384 waves (2.3 rounds of the 7 x 1024 resident
+// ones), at least four theta~ each.  Measured (FP32 / BF16 whole chains, 1 /
+// 2 / 4 / 8 / 16 segments): 36 tiles 517 / 290 / 166 / 100 / 64 us; 4096
+// tiles 5.78 / 5.81 / 5.45 / 5.40 / 6.02 ms; 8192 tiles 6.34 / 5.78 / 5.88 /
+// 5.85 / 7.48 ms and 4.89 / 4.81 / 4.84 / 5.32 / 7.08 ms; 33 264 tiles 17.7 /
+// 17.6 / 17.7 / 18.2 / 22.8 ms; 163 840 tiles 50.2 / 50.9 / 51.5 / 56.8 /
+// 77.6 ms (more segments read more views at a time through each L2).  It
+// depends on the volume and the tile depth only, so that every entry point
+// (streamed slab groups, batches) sums in the same order.
+inline int bp_segments(int tiles, int nslabs, int H, int tile_z) {
+  int s = 1;
+  if (tile_z > 16) return s;   // (their sums do not fit a workgroup's registers)
+  while (s < kBpMaxSegments && (int64_t)tiles * nslabs * s < 16384 && H / (2 * s) >= 4) s *= 2;
+  return s;
+}
 
 // Persistent multi-job backprojection (backproject_v1.hip).
 struct BpBatchArgs {
