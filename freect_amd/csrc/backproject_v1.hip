@@ -321,24 +321,6 @@ __device__ __forceinline__ void bp_add4(const BpTap<PREC>* s, const ChanInterp<P
   }
 }
 
-// Order of the tiles of a slab: square blocks of kSuper x kSuper tiles
-// (row-major blocks, row-major tiles inside a block; partial blocks at the
-// right and bottom edges), so that the tiles an XCD runs at the same time
-// cover compact patches of the slice rather than a band of whole tile rows:
-// a narrower detector footprint per view in the XCD's L2 (FP16 full
-// workload 52.5 -> 48.6 ms against row-major order; blocks of 8 or 16
-// tiles alike, 4 and 32 slower).  Only the order changes: every tile is
-// computed as before.
-constexpr int kSuper = 16;
-__device__ __forceinline__ int2 tile_of(int l, int tiles_x, int tiles_y) {
-  const int band = kSuper * tiles_x;                 // tiles of a full block row
-  const int sy = l / band, r = l - sy * band;
-  const int h = min(kSuper, tiles_y - sy * kSuper);  // rows of this block row
-  const int sx = r / (kSuper * h), r2 = r - sx * kSuper * h;
-  const int w = min(kSuper, tiles_x - sx * kSuper);  // columns of this block
-  return make_int2(sx * kSuper + r2 % w, sy * kSuper + r2 / w);
-}
-
 // How the theta~ of a tile are summed: in one sweep; in a.nseg consecutive
 // segments by as many waves of a workgroup (their sums added in segment
 // order through LDS); or in the same segments one after the other by one
@@ -595,6 +577,13 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, f
   }
 }
 
+// The tile of a launch block: block b runs on XCD b mod 8 and takes the next
+// tile of that XCD's share (BpArgs::xcd_first); -1 past its end.
+__device__ __forceinline__ int bp_launch_tile(const BpArgs& a) {
+  const int x = blockIdx.x & 7, lin = a.xcd_first[x] + (int)(blockIdx.x >> 3);
+  return lin < a.xcd_first[x + 1] ? lin : -1;
+}
+
 // Occupancy floor for the 16-bit kernels at TZ <= 8: at least seven waves
 // per SIMD (the few spills this costs sit in the per-theta~ setup, outside
 // the sample loop).  At TZ = 16 five (96 VGPRs; the allocator's own choice
@@ -608,8 +597,10 @@ template <int TZ, int PREC, int MODE, bool CENTERED>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(TZ >= 8 ? bp_min_waves<TZ, PREC>() : 1, 8)))
 void bp_v1_kernel(BpArgs a) {
+  const int lin = bp_launch_tile(a);
+  if (lin < 0) return;
   bp_v1_tile<TZ, PREC, MODE, CENTERED, kSweep>(
-      a, a.slab0 * a.tiles_x * a.tiles_y + xcd_block(blockIdx.x, gridDim.x), 0, nullptr);
+      a, lin, 0, nullptr);
 }
 
 // A workgroup of a.nseg waves per tile.
@@ -618,9 +609,10 @@ __global__ __launch_bounds__(64 * kBpMaxSegments)
 __attribute__((amdgpu_waves_per_eu(TZ >= 8 ? bp_min_waves<TZ, PREC>() : 1, 8)))
 void bp_v1_split_kernel(BpArgs a) {
   extern __shared__ float bp_lds[];
+  const int lin = bp_launch_tile(a);
+  if (lin < 0) return;
   bp_v1_tile<TZ, PREC, MODE, CENTERED, kSplitWaves>(
-      a, a.slab0 * a.tiles_x * a.tiles_y + xcd_block(blockIdx.x, gridDim.x),
-      __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), bp_lds);
+      a, lin, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), bp_lds);
 }
 
 // Persistent backprojection of many jobs in one launch.  The tiles of all
@@ -661,7 +653,9 @@ void bp_batch_kernel(BpBatchArgs b,
 
 template <int TZ, int PREC, bool C>
 hipError_t launch3(const BpArgs& a, int mode, hipStream_t s) {
-  const int blocks = a.tiles_x * a.tiles_y * (a.slab_count ? a.slab_count : a.nslabs);
+  int share = 0;
+  for (int x = 0; x < 8; ++x) share = std::max(share, a.xcd_first[x + 1] - a.xcd_first[x]);
+  const int blocks = 8 * share;
   if constexpr (TZ <= 16) {
     if (a.nseg > 1 && mode == kBpAccumulate) {
       hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks),
@@ -776,6 +770,11 @@ hipError_t launch_backproject_v1(const BpArgs& a, int tile_z, int precision, int
   // Slabs [slab0, slab0 + slab_count) inside the volume (slab_count 0: every slab).
   if (a.slab0 < 0 || a.slab_count < 0 || (a.slab_count == 0 && a.slab0 != 0) ||
       a.slab0 + a.slab_count > a.nslabs)
+    return hipErrorInvalidValue;
+  // The XCDs' shares are those of this range (bp_share).
+  const int tiles = a.tiles_x * a.tiles_y;
+  if (a.xcd_first[0] != a.slab0 * tiles ||
+      a.xcd_first[8] != (a.slab0 + (a.slab_count ? a.slab_count : a.nslabs)) * tiles)
     return hipErrorInvalidValue;
   switch (tile_z) {
     case 4: return launch1<4>(a, precision, mode, s);

@@ -224,6 +224,42 @@ int plan_set_tile_z(fct_wfbp_gpu_plan* p, int tz) {
   return FCT_OK;
 }
 
+// Each XCD takes a run of tiles of about equal cost: a tile with a voxel in
+// the FOV costs its slab's views (and its theta~ loop), one without almost
+// nothing.  Equal counts of tiles left XCDs idle where the slabs differ, at
+// the ends of a volume that the scan covers partly (256 x 256 x 64 slices, 20
+// of 40 mm covered: 5.84 -> 4.4 ms).
+void plan_bp_share(const fct_wfbp_gpu_plan* p, int slab0, int count, BpArgs* a) {
+  const std::vector<int32_t>& act = p->h_tile_active;
+  const int tiles = (int)act.size() - 1, n = count ? count : p->nslabs;
+  a->slab0 = slab0;
+  a->slab_count = count;
+  auto views = [&](int s) {
+    const int2 v = p->h_slab_vrange[slab0 + s];
+    return (long long)(v.y - v.x) + p->H / 4;
+  };
+  auto cost = [&](int s, int l) { return act[l] * views(s) + 2LL * (l - act[l]); };
+  long long total = 0;
+  for (int s = 0; s < n; ++s) total += cost(s, tiles);
+  long long before = 0;
+  int s = 0;
+  a->xcd_first[0] = slab0 * tiles;
+  a->xcd_first[8] = (slab0 + n) * tiles;
+  for (int x = 1; x < 8; ++x) {
+    const long long target = total * x / 8;
+    while (s < n && before + cost(s, tiles) <= target) before += cost(s++, tiles);
+    int lo = 0, hi = s < n ? tiles : 0;   // first l with before + cost(s, l) >= target
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if (before + cost(s, mid) < target)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    a->xcd_first[x] = (slab0 + s) * tiles + lo;
+  }
+}
+
 BpArgs plan_bp_args(const fct_wfbp_gpu_plan* p) {
   BpArgs a{};
   a.xs = p->d_xs;
@@ -246,6 +282,7 @@ BpArgs plan_bp_args(const fct_wfbp_gpu_plan* p) {
   a.tiles_y = (p->recon.ny + 7) / 8;
   a.nslabs = p->nslabs;
   a.nseg = bp_segments(a.tiles_x * a.tiles_y, a.nslabs, a.H, p->tile_z);
+  plan_bp_share(p, 0, 0, &a);
   return a;
 }
 
@@ -688,8 +725,7 @@ int reconstruct_streaming(fct_wfbp_gpu_plan* p, const ViewSource& src, int vpc,
     const int b = groups++ & 1;
     hipStream_t bs = ctx->bp_stream[b];
     hipError_t e = hipStreamWaitEvent(bs, p->ev_rebin, 0);
-    bp.slab0 = s_done;
-    bp.slab_count = s1 - s_done;
+    fct::plan_bp_share(p, s_done, s1 - s_done, &bp);
     s_done = s1;
     if (e == hipSuccess)
       e = fct::launch_backproject(bp, p->tile_z, p->variant, prec, fct::kBpAccumulate, bs);
@@ -989,6 +1025,23 @@ FCT_API int fct_wfbp_gpu_plan_create(fct_wfbp_gpu_ctx* ctx, const fct_scan_geome
   for (int i = 0; i < r.ny; ++i) {
     ys[i] = fct_tables::voxel_coord(i, r.ny, r.recon_fov, r.y_origin);
     if (cw) ys[i] = -ys[i];
+  }
+  // Tiles with a voxel column in the FOV (by the column nearest the axis).
+  {
+    const int tx = (r.nx + 7) / 8, ty = (r.ny + 7) / 8;
+    auto nearest = [](const std::vector<float>& c, int i0) {
+      float m = INFINITY;
+      for (int i = i0; i < std::min((int)c.size(), i0 + 8); ++i) m = std::min(m, std::fabs(c[i]));
+      return m;
+    };
+    std::vector<float> ax(tx), ay(ty);
+    for (int i = 0; i < tx; ++i) ax[i] = nearest(xs, i * 8);
+    for (int i = 0; i < ty; ++i) ay[i] = nearest(ys, i * 8);
+    p->h_tile_active.assign((size_t)tx * ty + 1, 0);
+    for (int l = 0; l < tx * ty; ++l) {
+      const int2 t = fct::tile_of(l, tx, ty);
+      p->h_tile_active[l + 1] = p->h_tile_active[l] + (fct_in_fov(ax[t.x], ay[t.y], p->g) ? 1 : 0);
+    }
   }
   for (int i = 0; i < p->n_native; ++i) zs[i] = (float)(zn[i] - zn[(i / chunk) * chunk]);
   for (int c = 0; c < p->nchunks; ++c)

@@ -111,8 +111,31 @@ struct BpArgs {
   // arrive.  Unused by the persistent batch kernel.
   int32_t slab0, slab_count;
   int32_t nseg;              // theta~ segments summed apart (bp_segments)
+  // Tiles [xcd_first[x], xcd_first[x + 1]) of the launch, in slab-major order,
+  // go to XCD x (plan_bp_share).  Unused by the persistent batch kernel.
+  int32_t xcd_first[9];
 };
 constexpr int kBpMaxSegments = 16;
+
+__host__ __device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
+
+// Order of the tiles of a slab: square blocks of kSuper x kSuper tiles
+// (row-major blocks, row-major tiles inside a block; partial blocks at the
+// right and bottom edges), so that the tiles an XCD runs at the same time
+// cover compact patches of the slice rather than a band of whole tile rows:
+// a narrower detector footprint per view in the XCD's L2 (FP16 full
+// workload 52.5 -> 48.6 ms against row-major order; blocks of 8 or 16
+// tiles alike, 4 and 32 slower).  Only the order changes: every tile is
+// computed as before.
+constexpr int kSuper = 16;
+__host__ __device__ __forceinline__ int2 tile_of(int l, int tiles_x, int tiles_y) {
+  const int band = kSuper * tiles_x;                 // tiles of a full block row
+  const int sy = l / band, r = l - sy * band;
+  const int h = imin(kSuper, tiles_y - sy * kSuper);  // rows of this block row
+  const int sx = r / (kSuper * h), r2 = r - sx * kSuper * h;
+  const int w = imin(kSuper, tiles_x - sx * kSuper);  // columns of this block
+  return make_int2(sx * kSuper + r2 % w, sy * kSuper + r2 / w);
+}
 
 // Segments of theta~ that a volume of so many tiles per slab sums apart, so
 // that a small volume still fills the GPU (a wave per tile and segment): a
@@ -290,6 +313,8 @@ struct fct_wfbp_gpu_plan;
 namespace fct {
 // Plan helpers shared by capi.hip and batch.hip.
 BpArgs plan_bp_args(const fct_wfbp_gpu_plan* p);   // tables only (no buffers)
+// Slabs [slab0, slab0 + count) of a launch (count 0: all), shared among the XCDs.
+void plan_bp_share(const fct_wfbp_gpu_plan* p, int slab0, int count, BpArgs* a);
 int plan_set_tile_z(fct_wfbp_gpu_plan* p, int tz);  // rebuilds the slab view ranges
 // Rebin + filter of the lines some slab reads (the whole-chain entry points).
 int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale);
@@ -376,6 +401,7 @@ struct fct_wfbp_gpu_plan {
   hipEvent_t ev_ratio = nullptr;         // after the storage-scale ratio's copy to h_ratio
   float* h_ratio = nullptr;              // pinned: scale[2] of the latest scale update
   std::vector<int2> h_slab_vrange;      // host copy of d_slab_vrange
+  std::vector<int32_t> h_tile_active;   // [tiles + 1] tiles with a voxel in the FOV before tile l
   std::vector<fct::RebinDev> h_rebin;   // host copy of d_rebin
   std::vector<int32_t> h_thk_need;      // per requested slice: 1 + its last native slice (0: none)
   std::vector<hipEvent_t> ev_chunk;     // per chunk: its copy has landed
