@@ -7,12 +7,22 @@
 //   * per (theta~, view parity) each lane's z-interval of |q| <= 1 is
 //     [zt - kb - lt, zt - kb + lt]; the extremes of its ends over the tile
 //     (DPP wave reductions, tabulated once per plan by bp_zbounds_kernel)
-//     give, per view, the slices any lane of the wave can select, intersected
-//     with the view window's exact slice range (a host table built with the
-//     same FP32 test); other slices are skipped wave-uniformly and the exact
-//     per-sample selection still runs, so selection is unchanged;
-//   * the views of one theta~ and parity move monotonically in z, so the
-//     view loop ends at the first view whose slice range lies past the slab;
+//     give, per view, the slices any lane of the wave can select; other
+//     slices are skipped wave-uniformly and the exact per-sample selection
+//     still runs, so selection is unchanged;
+//   * the views of one theta~ are looked at together, lane l at the l-th: two
+//     ballots give the views that cover the whole slab and those that cover
+//     part of it, and scalar loops over their bits visit no other view.  (A
+//     test per view inside the loop made the loop divergent for the
+//     compiler and read the window table for every view.)  The view window
+//     cuts into a view's slices only near its ends; only those views read
+//     the exact slice range (a host table built with the same FP32 test);
+//   * the sums over theta~ live in LDS: one read, fma and write per theta~
+//     instead of registers that the 72-VGPR kernel spilled.
+//     Together: FP16 512 x 512 x 320 49.4 -> 46.0 ms, six FP16 jobs of 256 x
+//     256 in one launch 35.6 -> 32.8, BF16 256 x 256 x 64 4.87 -> 4.4, FP32 500
+//     x 381 x 88 17.5 -> 17.2 (whole chains; of these the uniform loops 47.6 /
+//     32.5 / 4.35 / 17.3);
 //   * when a view covers the whole slab (the common case) the slices are
 //     processed four at a time without a per-slice branch, the taps of the
 //     four in flight together (with FP16 taps also for views covering part of
@@ -64,10 +74,10 @@ struct ChanInterp<FCT_PRECISION_FP32> {   // plain rows: two 8-byte loads
     u32x2 a, b;
   };
   float wp;
-  uint32_t base;   // byte offset of (view, row 0, pf)
-  __device__ void init(uint32_t view_bytes, uint32_t pf, float w) {
+  uint32_t base;   // byte offset of (row 0, pf) in its view; + the view's for fetch()
+  __device__ void init(uint32_t pf, float w) {
     wp = w;
-    base = view_bytes + pf * kEntry;
+    base = pf * kEntry;
   }
   // Row iq + 1 at the vector offset off + rowB: both loads are range-checked
   // (the hardware's check covers the vector offset, not the scalar one), so
@@ -104,11 +114,11 @@ struct ChanInterp<FCT_PRECISION_FP16> {   // quad entries: one 8-byte load
   // (a position error below 2^-12 channel).
   uint32_t w, nw;
   uint32_t base;
-  __device__ void init(uint32_t view_bytes, uint32_t pf, float wp) {
+  __device__ void init(uint32_t pf, float wp) {
     const float wq = fp16_channel_weight(wp);
     w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(1.0f - wq, wq));
     nw = w ^ 0x80008000u;
-    base = view_bytes + pf * kEntry;
+    base = pf * kEntry;
   }
   __device__ static Raw fetch(const BpRsrc& r, uint32_t off, uint32_t) {
     return __builtin_amdgcn_raw_buffer_load_b64(r.rows, (int)off, 0, 0);
@@ -122,33 +132,46 @@ struct ChanInterp<FCT_PRECISION_FP16> {   // quad entries: one 8-byte load
     const float d = dot2_f16(q1, w, nr0);
     return fmaf(fq, d, -nr0);
   }
-  // The same for four samples, as one block of eight v_dot2_f32_f16 in the
-  // VOP3P form (the builtin selects the two-address v_dot2c form and copies
-  // the accumulator).  Every dot result is read at least three instructions
-  // after it is written (the wait a dot result needs before another VALU
-  // instruction reads it): the second dot of a sample reads the first four
-  // instructions later, and s_nop 2 ends the block.
-  __device__ void values4(const Raw* t, const float* fq, float* val) const {
+  // The same for four samples and their sums, num += W value and den += W, as
+  // one block of eight v_dot2_f32_f16 in the VOP3P form (the builtin selects
+  // the two-address v_dot2c form and copies the accumulator) with the sums
+  // updated in place (left to the compiler, the paths of the view loop end in
+  // different registers and every view copies all sums at the join).  Every
+  // dot result is read at least three instructions after it is written (the
+  // wait a dot result needs before another VALU instruction reads it): the
+  // second dot of a sample reads the first four instructions later, and the
+  // four additions to den follow the last dot.
+  __device__ void accumulate4(const Raw* t, const float* fq, const float* W, float* num,
+                              float* den) const {
     const uint32_t a0 = t[0].x, a1 = t[1].x, a2 = t[2].x, a3 = t[3].x;
     const uint32_t b0 = t[0].y, b1 = t[1].y, b2 = t[2].y, b3 = t[3].y;
     float n0, n1, n2, n3, d0, d1, d2, d3;
-    asm("v_dot2_f32_f16 %0, %8, %16, 0\n\t"
-        "v_dot2_f32_f16 %1, %9, %16, 0\n\t"
-        "v_dot2_f32_f16 %2, %10, %16, 0\n\t"
-        "v_dot2_f32_f16 %3, %11, %16, 0\n\t"
-        "v_dot2_f32_f16 %4, %12, %17, %0\n\t"
-        "v_dot2_f32_f16 %5, %13, %17, %1\n\t"
-        "v_dot2_f32_f16 %6, %14, %17, %2\n\t"
-        "v_dot2_f32_f16 %7, %15, %17, %3\n\t"
-        "s_nop 2"
+    asm("v_dot2_f32_f16 %0, %16, %24, 0\n\t"
+        "v_dot2_f32_f16 %1, %17, %24, 0\n\t"
+        "v_dot2_f32_f16 %2, %18, %24, 0\n\t"
+        "v_dot2_f32_f16 %3, %19, %24, 0\n\t"
+        "v_dot2_f32_f16 %4, %20, %25, %0\n\t"
+        "v_dot2_f32_f16 %5, %21, %25, %1\n\t"
+        "v_dot2_f32_f16 %6, %22, %25, %2\n\t"
+        "v_dot2_f32_f16 %7, %23, %25, %3\n\t"
+        "v_add_f32 %12, %12, %30\n\t"
+        "v_add_f32 %13, %13, %31\n\t"
+        "v_add_f32 %14, %14, %32\n\t"
+        "v_add_f32 %15, %15, %33\n\t"
+        "v_fma_f32 %4, %26, %4, -%0\n\t"
+        "v_fma_f32 %5, %27, %5, -%1\n\t"
+        "v_fma_f32 %6, %28, %6, -%2\n\t"
+        "v_fma_f32 %7, %29, %7, -%3\n\t"
+        "v_fmac_f32 %8, %30, %4\n\t"
+        "v_fmac_f32 %9, %31, %5\n\t"
+        "v_fmac_f32 %10, %32, %6\n\t"
+        "v_fmac_f32 %11, %33, %7"
         : "=&v"(n0), "=&v"(n1), "=&v"(n2), "=&v"(n3), "=&v"(d0), "=&v"(d1), "=&v"(d2),
-          "=&v"(d3)
+          "=&v"(d3), "+v"(num[0]), "+v"(num[1]), "+v"(num[2]), "+v"(num[3]), "+v"(den[0]),
+          "+v"(den[1]), "+v"(den[2]), "+v"(den[3])
         : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(b0), "v"(b1), "v"(b2), "v"(b3), "v"(nw),
-          "v"(w));
-    val[0] = fmaf(fq[0], d0, -n0);
-    val[1] = fmaf(fq[1], d1, -n1);
-    val[2] = fmaf(fq[2], d2, -n2);
-    val[3] = fmaf(fq[3], d3, -n3);
+          "v"(w), "v"(fq[0]), "v"(fq[1]), "v"(fq[2]), "v"(fq[3]), "v"(W[0]), "v"(W[1]),
+          "v"(W[2]), "v"(W[3]));
   }
 };
 
@@ -158,9 +181,9 @@ struct ChanInterp<FCT_PRECISION_BF16> {   // quad entries: one 8-byte load
   typedef u32x2 Raw;
   float wp;
   uint32_t base;
-  __device__ void init(uint32_t view_bytes, uint32_t pf, float w) {
+  __device__ void init(uint32_t pf, float w) {
     wp = w;
-    base = view_bytes + pf * kEntry;
+    base = pf * kEntry;
   }
   __device__ static Raw fetch(const BpRsrc& r, uint32_t off, uint32_t) {
     return __builtin_amdgcn_raw_buffer_load_b64(r.rows, (int)off, 0, 0);
@@ -279,11 +302,12 @@ __device__ __forceinline__ float bp_weight(const BpTap<PREC>& s, float fR, const
   return s.sel ? w : 0.0f;
 }
 
-// Accumulation of a sample of weight W (bp_weight) and interpolated value val.
+// Accumulation of a sample of weight W (bp_weight) and interpolated value
+// val, in place (see accumulate4).
 template <int MODE>
 __device__ __forceinline__ void bp_acc(float W, float val, float& num, float& den) {
-  num = fmaf(W, val, num);
-  if (MODE != kBpMatched) den += W;
+  asm("v_fmac_f32 %0, %1, %2" : "+v"(num) : "v"(W), "v"(val));
+  if (MODE != kBpMatched) asm("v_add_f32 %0, %0, %1" : "+v"(den) : "v"(W));
 }
 
 template <int PREC, int MODE, bool FREE = false>
@@ -296,7 +320,7 @@ __device__ __forceinline__ void bp_add(const BpTap<PREC>& s, const ChanInterp<PR
   bp_acc<MODE>(bp_weight<PREC, MODE, FREE>(s, fR, g), ci.value(s.raw, s.fq), num, den);
 }
 
-// Four samples of one view (the whole-slab path): FP16 through the dot block.
+// Four samples of one view: FP16 through the dot block.
 template <int PREC, int MODE, bool FREE = false>
 __device__ __forceinline__ void bp_add4(const BpTap<PREC>* s, const ChanInterp<PREC>& ci,
                                         float fR, const FctBpConsts& g, float* num, float* den,
@@ -304,16 +328,14 @@ __device__ __forceinline__ void bp_add4(const BpTap<PREC>* s, const ChanInterp<P
   if constexpr (PREC == FCT_PRECISION_FP16 && MODE != kBpCount) {
     // The weights first: their arithmetic overlaps the tap loads.
     typename ChanInterp<PREC>::Raw t[4];
-    float fq[4], W[4], val[4];
+    float fq[4], W[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       t[i] = s[i].raw;
       fq[i] = s[i].fq;
       W[i] = bp_weight<PREC, MODE, FREE>(s[i], fR, g);
     }
-    ci.values4(t, fq, val);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) bp_acc<MODE>(W[i], val[i], num[i], den[i]);
+    ci.accumulate4(t, fq, W, num, den);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -328,8 +350,9 @@ __device__ __forceinline__ void bp_add4(const BpTap<PREC>* s, const ChanInterp<P
 enum BpSplit { kSweep = 0, kSplitWaves = 1, kSplitSerial = 2 };
 
 // One wave reconstructs tile `lin` (slab-major order) of the job described by
-// a; with kSplitWaves its theta~ segment `wave`.  lds: kSplitWaves (nseg - 1)
-// x min(TZ, 8) x 64 floats, kSplitSerial TZ x 64.
+// a; with kSplitWaves its theta~ segment `wave`.  The sums over theta~ live in
+// lds, TZ x 64 floats per wave (kSplitSerial 2 TZ x 64): read, added to and
+// written once per theta~, they would cost registers the view loops need.
 template <int TZ, int PREC, int MODE, bool CENTERED, int SPLIT>
 __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, float* lds) {
   constexpr uint32_t kEntry = ChanInterp<PREC>::kEntry;
@@ -361,26 +384,22 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, f
 #pragma unroll
   for (int i = 0; i < TZ; ++i) zs[i] = ld_uniform(a.zs + s0 + (i < nz ? i : nz - 1));
   // Slice spacing inside the slab (uniform, FP32; used only for skipping).
-  const float zfirst = zs[0], zlast = zs[nz - 1];
+  const float zfirst = zs[0], zlast = ld_uniform(a.zs + s0 + nz - 1);
   const float dzs = nz > 1 ? (zlast - zfirst) / (float)(nz - 1) : 1.0f;
   const float inv_dzs = 1.0f / dzs, ninv_dzs = -inv_dzs;
-  // Along k (views t + k H of one theta~ and parity) the view z moves
-  // monotonically, and with it every bound of a view's slice range [ilo, ihi]
-  // below, all in the same direction: up (in slice index) when the table feed
-  // and the slice step have the same sign.  A view whose range lies entirely
-  // past the slab in that direction is followed only by such views.
-  const bool up = (g.kappa > 0.0f) == (dzs > 0.0f);
   // Centred WFBP sums: the whole-slab samples take their weight without a
   // selection mask (bp_weight), the lanes whose column misses the detector
   // parked at row -1e30 with 0 rows per mm (the per-slice masks of the
   // partial-slab paths already exclude those lanes).
   constexpr bool kFree = CENTERED && MODE == kBpAccumulate;
-  const bool can_stop = nz > 1;
   const float* ztc = a.zt + (size_t)chunk * a.nviews;
   const int* wrc = reinterpret_cast<const int*>(a.wrange + (size_t)chunk * a.nviews);
+  const float half_feed = g.kappa * 3.14159265f, z_inside = g.zrot - 0.5f * fabsf(dzs);
   const int* vrp = reinterpret_cast<const int*>(a.slab_vrange + slab);
   const int2 vr = make_int2(ld_uniform(vrp), ld_uniform(vrp + 1));
   const int H = a.H;
+  // The views of theta~ t are t + k H, k in [qx + (t < rx), qy + (t < ry)).
+  const int qx = vr.x / H, rx = vr.x - qx * H, qy = vr.y / H, ry = vr.y - qy * H;
   const uint32_t vstride = (uint32_t)g.nrows * (uint32_t)a.cpitch;   // entries per view
   const uint32_t rowB = (uint32_t)a.cpitch * kEntry;                 // bytes per row
 
@@ -392,29 +411,25 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, f
   BpRsrc rf;
   rf.rows = __builtin_amdgcn_make_buffer_rsrc((void*)fb, 0, fbytes, kRsrcWord3);
 
-  float acc[TZ];
+  float* acc = lds + lane;   // slice i at acc[i * 64]
   int cnt[TZ];
   int seg = SPLIT == kSplitWaves ? wave : 0;
   do {
 #pragma unroll
     for (int i = 0; i < TZ; ++i) {
-      acc[i] = 0.0f;
+      if (MODE != kBpCount) acc[i * 64] = 0.0f;
       cnt[i] = 0;
     }
     const int t0 = SPLIT == kSweep ? 0 : H * seg / a.nseg;
     const int t1 = SPLIT == kSweep ? H : H * (seg + 1) / a.nseg;
     for (int t = t0; t < t1; ++t) {
-      const int kmin = vr.x <= t ? 0 : (vr.x - t + H - 1) / H;
-      const int kmax = vr.y <= t ? 0 : (vr.y - t + H - 1) / H;
+      const int kmin = qx + (t < rx ? 1 : 0), kmax = qy + (t < ry ? 1 : 0);
       if (kmin >= kmax) continue;
       const float* csp = reinterpret_cast<const float*>(a.cs + t);
       const float2 cs = make_float2(ld_uniform(csp), ld_uniform(csp + 1));
       const BpColumn col = bp_column(x, y, cs, g);
-      const float p = col.p, sq = col.sq, f = col.f, kb = col.kb;
       // The tile's z-interval extremes for this theta~ (tabulated per plan).
-      const float* zbp = reinterpret_cast<const float*>(a.zbounds + (size_t)tile * H + t);
-      const float4 zb =
-          make_float4(ld_uniform(zbp), ld_uniform(zbp + 1), ld_uniform(zbp + 2), ld_uniform(zbp + 3));
+      const float4 zb = ld_uniform4(a.zbounds + (size_t)tile * H + t);
       float num[TZ], den[TZ];
 #pragma unroll
       for (int i = 0; i < TZ; ++i) {
@@ -430,59 +445,73 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, f
         num[i] = zero;
         den[i] = tiny;
       }
-
-#pragma unroll
-      for (int par = 0; par < 2; ++par) {
-        int k = kmin + (((kmin & 1) != par) ? 1 : 0);
-        if (k >= kmax) continue;
-        const float pidx = par ? fmaf(-p, g.inv_ds, g.cc) : fmaf(p, g.inv_ds, g.cc);
-        const float lt = (par ? sq + f : sq - f) * g.tanc;
-        const float kbs = par ? -kb : kb;
-        const float pfl = floorf(pidx);
-        const bool chan_ok = active && pfl >= 0.0f && pfl <= (float)(g.ncols - 2);
-        // Rows per mm of z; 0 for the lanes parked off the detector (kFree).
-        const float invLh = kFree && !chan_ok ? 0.0f : div_rn_normal(g.hr, lt);
-        const uint32_t pf = chan_ok ? (uint32_t)(int)pfl : 0u;
-        const float wp = pidx - pfl;
-        // Matched mode: R / l, the voxel-driven footprint's depth correction
-        // (a row spans drow l / Dsd of z at distance l from the source).
-        const float fR = MODE == kBpMatched ? g.tanc / (lt * g.invR) : 0.0f;
-        // z-interval of |q| <= 1 relative to the view's table z, over the wave.
-        const float A = par ? zb.z : zb.x;
-        const float B = par ? zb.w : zb.y;
-        // Slice positions of the interval ends for a view at table z ztv:
-        // ztv * inv_dzs + c, the lower end first (A <= B, so the order is
-        // that of the slice step's sign).
+      for (int kb = kmin; kb < kmax; kb += 64) {   // (rarely more than one pass)
+        // Lane l looks at view kb + l: its slice range [ilo, ihi] inside the
+        // slab, from the z-interval of |q| <= 1 over the tile (z relative to
+        // the view's table z; one slice of margin on each side covers the
+        // rounding, the per-sample test is exact).  The views of a theta~ are
+        // half a feed apart.  The view window ends none of the slices of a
+        // view whose slices lie at least half a slice inside it; for the
+        // others (near) the exact table applies.  (The matched projector pair
+        // uses every view that sees the voxel: no view window.)
+        const int kl = kb + lane;
+        const float zl = fmaf((float)lane, half_feed, ld_uniform(ztc + t + kb * H));
+        const bool odd = kl & 1;
+        const float A = odd ? zb.z : zb.x, B = odd ? zb.w : zb.y;
         const float ca = (A - zfirst) * inv_dzs, cb = (B - zfirst) * inv_dzs;
-        const float clo = inv_dzs > 0.0f ? ca : cb, nchi = -(inv_dzs > 0.0f ? cb : ca);
-        for (; k < kmax; k += 2) {
-          const int v = t + k * H;
-          const float ztv = ld_uniform(ztc + v);
-          // Exact window slice range (native indices).
-          const int2 wr = make_int2(ld_uniform(wrc + 2 * v), ld_uniform(wrc + 2 * v + 1));
-          // One slice of margin on each side covers the rounding of these
-          // positions; the per-sample test below is exact.
-          const int flo = floor_int(fmaf(ztv, inv_dzs, clo));
-          const int fhi = floor_int(fmaf(ztv, ninv_dzs, nchi));   // -ceil(upper end)
-          // (The matched projector pair uses every view that sees the voxel:
-          // no view window.)
-          const int ilo = max(max(0, flo - 1), MODE == kBpMatched ? 0 : wr.x - s0);
-          const int ihi = min(min(nz - 1, 1 - fhi), MODE == kBpMatched ? nz - 1 : wr.y - s0);
-          if (ilo > ihi) {
-            if (can_stop && (up ? ilo > nz - 1 : ihi < 0)) break;
-            continue;
-          }
-          const float row0 =                                 // fct_bp_row0
-              kFree && !chan_ok ? -1.0e30f : fmaf(kbs - ztv, invLh, g.cr);
+        const int flo = floor_int(fmaf(zl, inv_dzs, inv_dzs > 0.0f ? ca : cb));
+        const int fhi = floor_int(fmaf(zl, ninv_dzs, inv_dzs > 0.0f ? -cb : -ca));   // -ceil
+        const int ilo_l = max(0, flo - 1), ihi_l = min(nz - 1, 1 - fhi);
+        const bool some = kl < kmax && ilo_l <= ihi_l;
+        const float zrel = zl - zfirst;
+        const bool near =
+            MODE != kBpMatched && some &&
+            fmaxf(fabsf(fmaf((float)-ilo_l, dzs, zrel)), fabsf(fmaf((float)-ihi_l, dzs, zrel))) >
+                z_inside;
+        const uint64_t m_some = __builtin_amdgcn_ballot_w64(some);
+        const uint64_t m_near = __builtin_amdgcn_ballot_w64(near);
+        const uint64_t m_whole =
+            __builtin_amdgcn_ballot_w64(some && !near && ilo_l == 0 && ihi_l == nz - 1);
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+          const uint64_t m_par = (kb & 1) == par ? 0x5555555555555555ull : 0xAAAAAAAAAAAAAAAAull;
+          uint64_t whole = m_whole & m_par, part = m_some & ~m_whole & m_par;
+          if (!(whole | part)) continue;
+          const float pidx = par ? fmaf(-col.p, g.inv_ds, g.cc) : fmaf(col.p, g.inv_ds, g.cc);
+          const float lt = (par ? col.sq + col.f : col.sq - col.f) * g.tanc;
+          const float kbs = par ? -col.kb : col.kb;
+          const float pfl = floorf(pidx);
+          const bool chan_ok = active && pfl >= 0.0f && pfl <= (float)(g.ncols - 2);
+          // Rows per mm of z; 0 for the lanes parked off the detector (kFree).
+          const float invLh = kFree && !chan_ok ? 0.0f : div_rn_normal(g.hr, lt);
           ChanInterp<PREC> ci;
-          ci.init((uint32_t)(v - vr.x) * vstride * kEntry, pf, wp);
-          if (ilo == 0 && ihi == nz - 1) {
+          ci.init(chan_ok ? (uint32_t)(int)pfl : 0u, pidx - pfl);
+          // Matched mode: R / l, the voxel-driven footprint's depth correction
+          // (a row spans drow l / Dsd of z at distance l from the source).
+          const float fR = MODE == kBpMatched ? g.tanc / (lt * g.invR) : 0.0f;
+          const uint32_t base = ci.base;
+          auto view = [&](int l, float ztv, float* row0) {
+            *row0 = kFree && !chan_ok ? -1.0e30f : fmaf(kbs - ztv, invLh, g.cr);   // fct_bp_row0
+            ci.base = base + (uint32_t)(t + (kb + l) * H - vr.x) * vstride * kEntry;
+          };
+          // The view's table z is loaded one view ahead.
+          auto ahead = [&](uint64_t m) {
+            return ld_uniform(ztc + t + (kb + (m ? __builtin_ctzll(m) : 0)) * H);
+          };
+          float zt_next = ahead(whole);
+          while (whole) {
             // Every slice of the slab (the common case): no per-slice branch,
             // and the taps of four slices are in flight before the first is
             // used (four, not TZ: more would cost waves per SIMD).  With
             // nz < TZ the extra slices repeat the last one and are not stored.
             // Centred WFBP sums take the weight without a selection mask
             // (bp_weight; the lanes off the detector are parked at row -1e30).
+            const int l = __builtin_ctzll(whole);
+            whole &= whole - 1;
+            const float ztv = zt_next;
+            zt_next = ahead(whole);
+            float row0;
+            view(l, ztv, &row0);
 #pragma unroll
             for (int h = 0; h < TZ; h += 4) {
               BpTap<PREC> tap[4];
@@ -495,76 +524,84 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, f
               if (PREC == FCT_PRECISION_FP16) __builtin_amdgcn_sched_barrier(0);
               bp_add4<PREC, MODE, kFree>(tap, ci, fR, g, num + h, den + h, cnt + h);
             }
-          } else if constexpr (PREC == FCT_PRECISION_FP16) {
-            // Part of the slab, FP16: groups of four slices that meet
-            // [ilo, ihi] through the dot block, the slices outside the range
-            // masked like unselected samples (cheaper than per-slice samples
-            // with the two-address dot form; for FP32 / BF16 the masked slices
-            // cost more than they save).
-#pragma unroll
-            for (int h = 0; h < TZ; h += 4) {
-              if (ilo > h + 3 || ihi < h) continue;
-              BpTap<PREC> tap[4];
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                tap[i] = bp_fetch<PREC, MODE, CENTERED>(zs[h + i], invLh, row0, ci, rf, rowB,
-                                                        chan_ok && h + i >= ilo && h + i <= ihi, g);
-              __builtin_amdgcn_sched_barrier(0);
-              bp_add4<PREC, MODE>(tap, ci, fR, g, num + h, den + h, cnt + h);
+          }
+          while (part) {
+            const int l = __builtin_ctzll(part);
+            part &= part - 1;
+            int ilo = __builtin_amdgcn_readlane(ilo_l, l);
+            int ihi = __builtin_amdgcn_readlane(ihi_l, l);
+            const int v = t + (kb + l) * H;
+            const float ztv = ld_uniform(ztc + v);
+            if (m_near >> l & 1) {   // the window's exact slice range
+              ilo = max(ilo, ld_uniform(wrc + 2 * v) - s0);
+              ihi = min(ihi, ld_uniform(wrc + 2 * v + 1) - s0);
+              if (ilo > ihi) continue;
             }
-          } else {
+            float row0;
+            view(l, ztv, &row0);
+            if constexpr (PREC == FCT_PRECISION_FP16) {
+              // Part of the slab, FP16: groups of four slices that meet
+              // [ilo, ihi] through the dot block, the slices outside the range
+              // masked like unselected samples (cheaper than per-slice samples
+              // with the two-address dot form; for FP32 / BF16 the masked slices
+              // cost more than they save).
 #pragma unroll
-            for (int i = 0; i < TZ; ++i)
-              if (i >= ilo && i <= ihi) {
-                const BpTap<PREC> tp =
-                    bp_fetch<PREC, MODE, CENTERED>(zs[i], invLh, row0, ci, rf, rowB, chan_ok, g);
-                bp_add<PREC, MODE>(tp, ci, fR, g, num[i], den[i], cnt[i]);
+              for (int h = 0; h < TZ; h += 4) {
+                if (ilo > h + 3 || ihi < h) continue;
+                BpTap<PREC> tap[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                  tap[i] = bp_fetch<PREC, MODE, CENTERED>(
+                      zs[h + i], invLh, row0, ci, rf, rowB,
+                      chan_ok && h + i >= ilo && h + i <= ihi, g);
+                __builtin_amdgcn_sched_barrier(0);
+                bp_add4<PREC, MODE>(tap, ci, fR, g, num + h, den + h, cnt + h);
               }
+            } else {
+#pragma unroll
+              for (int i = 0; i < TZ; ++i)
+                if (i >= ilo && i <= ihi) {
+                  const BpTap<PREC> tp = bp_fetch<PREC, MODE, CENTERED>(zs[i], invLh, row0, ci, rf,
+                                                                        rowB, chan_ok, g);
+                  bp_add<PREC, MODE>(tp, ci, fR, g, num[i], den[i], cnt[i]);
+                }
+            }
           }
         }
       }
       if (MODE == kBpAccumulate) {
 #pragma unroll
         for (int i = 0; i < TZ; ++i)
-          acc[i] = fmaf(num[i], __builtin_amdgcn_rcpf(den[i]), acc[i]);
+          acc[i * 64] = fmaf(num[i], __builtin_amdgcn_rcpf(den[i]), acc[i * 64]);
       } else if (MODE == kBpMatched) {
 #pragma unroll
-        for (int i = 0; i < TZ; ++i) acc[i] += num[i];
+        for (int i = 0; i < TZ; ++i) acc[i * 64] += num[i];
       }
     }
     if (SPLIT == kSplitSerial && a.nseg > 1) {
 #pragma unroll
       for (int i = 0; i < TZ; ++i) {
-        if (seg > 0) acc[i] = lds[i * 64 + lane] + acc[i];
-        lds[i * 64 + lane] = acc[i];
+        if (seg > 0) acc[i * 64] += acc[(TZ + i) * 64];
+        acc[(TZ + i) * 64] = acc[i * 64];
       }
     }
   } while (SPLIT == kSplitSerial && ++seg < a.nseg);
-  if (SPLIT == kSplitWaves) {
-    constexpr int kPart = TZ < 8 ? TZ : 8;
-#pragma unroll
-    for (int h = 0; h < TZ; h += kPart) {
-      if (h) __syncthreads();
-      if (wave > 0)
-#pragma unroll
-        for (int i = 0; i < kPart; ++i)
-          lds[((wave - 1) * kPart + i) * 64 + lane] = acc[h + i];
-      __syncthreads();
-      if (wave == 0)
-        for (int w = 0; w < a.nseg - 1; ++w)
-#pragma unroll
-          for (int i = 0; i < kPart; ++i) acc[h + i] += lds[(w * kPart + i) * 64 + lane];
-    }
-    if (wave > 0) return;
-  }
+  if (SPLIT == kSplitWaves) __syncthreads();
   if (!inb) return;
   if (MODE == kBpAccumulate || MODE == kBpMatched) {
     // FP16 / BF16 projections carry one storage scale per scan.
     const float out_scale =
         PREC == FCT_PRECISION_FP32 ? a.scale : a.scale * ld_uniform(a.filt_scale);
-#pragma unroll
-    for (int i = 0; i < TZ; ++i)
-      if (i < nz) a.native[((size_t)(s0 + i) * a.ny + iy) * a.nx + ix] = acc[i] * out_scale;
+    // The segments' waves share the slices out; each sums the segments of its
+    // slices in order.
+    const int nw = SPLIT == kSplitWaves ? a.nseg : 1;
+    const float* part = lds + lane - (SPLIT == kSplitWaves ? wave * TZ * 64 : 0);
+    for (int i = SPLIT == kSplitWaves ? wave : 0; i < nz; i += nw) {
+      float sum = part[i * 64];
+      for (int w = 1; w < nw; ++w) sum += part[(w * TZ + i) * 64];
+      a.native[((size_t)(s0 + i) * a.ny + iy) * a.nx + ix] =
+          sum * out_scale;
+    }
   } else if (MODE == kBpCount) {
     unsigned long long tot = 0;
 #pragma unroll
@@ -590,17 +627,17 @@ __device__ __forceinline__ int bp_launch_tile(const BpArgs& a) {
 // is 97, one over); a floor of six spills inside the view loop.
 template <int TZ, int PREC>
 constexpr int bp_min_waves() {
-  return PREC == FCT_PRECISION_FP32 ? 1 : TZ <= 8 ? 7 : TZ == 16 ? 5 : 1;
+  return TZ <= 8 ? 7 : TZ == 16 && PREC != FCT_PRECISION_FP32 ? 5 : 1;
 }
 
 template <int TZ, int PREC, int MODE, bool CENTERED>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(TZ >= 8 ? bp_min_waves<TZ, PREC>() : 1, 8)))
 void bp_v1_kernel(BpArgs a) {
+  __shared__ float bp_lds[MODE == kBpCount ? 1 : TZ * 64];
   const int lin = bp_launch_tile(a);
   if (lin < 0) return;
-  bp_v1_tile<TZ, PREC, MODE, CENTERED, kSweep>(
-      a, lin, 0, nullptr);
+  bp_v1_tile<TZ, PREC, MODE, CENTERED, kSweep>(a, lin, 0, bp_lds);
 }
 
 // A workgroup of a.nseg waves per tile.
@@ -611,8 +648,9 @@ void bp_v1_split_kernel(BpArgs a) {
   extern __shared__ float bp_lds[];
   const int lin = bp_launch_tile(a);
   if (lin < 0) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   bp_v1_tile<TZ, PREC, MODE, CENTERED, kSplitWaves>(
-      a, lin, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), bp_lds);
+      a, lin, wave, bp_lds + wave * TZ * 64);
 }
 
 // Persistent backprojection of many jobs in one launch.  The tiles of all
@@ -631,7 +669,7 @@ __attribute__((amdgpu_waves_per_eu(bp_min_waves<TZ, PREC>(), 8)))
 void bp_batch_kernel(BpBatchArgs b,
                                                       const BpArgs* __restrict__ jobs,
                                                       const int32_t* __restrict__ tile_start) {
-  __shared__ float lds[TZ * 64];
+  __shared__ float lds[2 * TZ * 64];
   const int xcd = blockIdx.x & 7;
   for (int step = 0; step < 8; ++step) {
     const int r = (xcd + step) & 7;
@@ -659,14 +697,14 @@ hipError_t launch3(const BpArgs& a, int mode, hipStream_t s) {
   if constexpr (TZ <= 16) {
     if (a.nseg > 1 && mode == kBpAccumulate) {
       hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks),
-                         dim3(64 * a.nseg), (a.nseg - 1) * std::min(TZ, 8) * 64 * sizeof(float), s,
+                         dim3(64 * a.nseg), a.nseg * TZ * 64 * sizeof(float), s,
                          a);
       return hipGetLastError();
     }
     if constexpr (PREC == FCT_PRECISION_FP32) {
       if (a.nseg > 1 && mode == kBpMatched) {
         hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks),
-                           dim3(64 * a.nseg), (a.nseg - 1) * std::min(TZ, 8) * 64 * sizeof(float),
+                           dim3(64 * a.nseg), a.nseg * TZ * 64 * sizeof(float),
                            s, a);
         return hipGetLastError();
       }
