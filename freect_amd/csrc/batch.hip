@@ -91,7 +91,7 @@ int upload_jobs(fct_wfbp_gpu_batch* b) {
                               hipMemcpyHostToDevice, b->stream));
   BATCH_TRY(b, hipStreamSynchronize(b->stream));
   int per_cu = 0;
-  BATCH_TRY(b, fct::backproject_batch_waves_per_cu(b->plans[0]->tile_z, b->opts.precision,
+  BATCH_TRY(b, fct::backproject_batch_waves_per_cu(b->plans[0]->tile_z, b->plans[0]->storage(),
                                                     &per_cu));
   const int ncu = std::max(b->plans[0]->ncu, 1);
   b->grid = std::max(8, (std::max(per_cu, 1) * ncu) / 8 * 8);
@@ -116,7 +116,7 @@ int enqueue_backproject(fct_wfbp_gpu_batch* b) {
     a.filt = p->d_filtered;
     a.filt_scale = p->d_scale;
     a.native = p->d_native;
-    BATCH_TRY(b, fct::launch_backproject_v1(a, p->tile_z, b->opts.precision, fct::kBpAccumulate,
+    BATCH_TRY(b, fct::launch_backproject_v1(a, p->tile_z, p->storage(), fct::kBpAccumulate,
                                             b->stream));
     return FCT_OK;
   }
@@ -127,7 +127,7 @@ int enqueue_backproject(fct_wfbp_gpu_batch* b) {
   a.queue = b->d_queue;
   a.n_jobs = (int32_t)b->plans.size();
   a.total_tiles = b->total_tiles;
-  BATCH_TRY(b, fct::launch_backproject_batch(a, b->plans[0]->tile_z, b->opts.precision,
+  BATCH_TRY(b, fct::launch_backproject_batch(a, b->plans[0]->tile_z, b->plans[0]->storage(),
                                              all_centered(b), b->grid, b->stream));
   return FCT_OK;
 }
@@ -135,7 +135,7 @@ int enqueue_backproject(fct_wfbp_gpu_batch* b) {
 int enqueue_rebin_filter(fct_wfbp_gpu_batch* b) {
   for (size_t j = 0; j < b->plans.size(); ++j) {
     fct_wfbp_gpu_plan* p = b->plans[j];
-    const int st = fct::chain_rebin_filter(p, b->raw[j], p->d_filtered, p->d_scale);
+    const int st = fct::chain_rebin_filter(p, b->raw[j], p->d_filtered, p->d_scale, p->pairs);
     if (st != FCT_OK) return st;
   }
   return FCT_OK;
@@ -213,14 +213,31 @@ FCT_API int fct_wfbp_gpu_batch_create(fct_wfbp_gpu_ctx* ctx, int32_t n_jobs,
     int st = fct_wfbp_gpu_plan_create(ctx, &scans[j], &recons[j], &b->opts, b->stream,
                                       &b->plans[j]);
     if (st != FCT_OK) return fail(st);
-    fct_wfbp_gpu_plan* p = b->plans[j];
+  }
+  // One storage for every job (one kernel runs them all): FP32 row pairs, or
+  // rows where a plan cannot hold those or there is no memory for them.
+  bool pairs = true;
+  for (fct_wfbp_gpu_plan* p : b->plans) pairs = pairs && p->pairs;
+  for (fct_wfbp_gpu_plan* p : b->plans) {
+    p->pairs = pairs;
+    const hipError_t e = fct::plan_alloc_filtered(p);
+    if (e != hipSuccess) return fail(hip_status(ctx, "batch buffers", e));
+    pairs = p->pairs;
+  }
+  for (fct_wfbp_gpu_plan* p : b->plans) {
     const size_t nat = (size_t)p->n_native * p->recon.ny * p->recon.nx * sizeof(float);
-    hipError_t e = hipMalloc(&p->d_filtered, p->filtered_bytes());
+    hipError_t e = hipSuccess;
+    if (p->pairs && !pairs) {
+      (void)hipFree(p->d_filtered);
+      p->d_filtered = nullptr;
+      p->pairs = false;
+      e = fct::plan_alloc_filtered(p);
+    }
     if (e == hipSuccess && p->scale_elems())
       e = hipMalloc(reinterpret_cast<void**>(&p->d_scale), p->scale_elems() * 4);
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&p->d_native), nat);
     if (e != hipSuccess) return fail(hip_status(ctx, "batch buffers", e));
-    b->device_bytes += (int64_t)(p->filtered_bytes() + p->scale_elems() * 4 + nat);
+    b->device_bytes += (int64_t)(p->storage_bytes() + p->scale_elems() * 4 + nat);
   }
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&b->d_jobs), n_jobs * sizeof(fct::BpArgs));
   if (e == hipSuccess)

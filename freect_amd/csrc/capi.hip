@@ -174,9 +174,11 @@ void free_plan_buffers(fct_wfbp_gpu_plan* p) {
 
 // Views a slab of tz slices can select: table z within one feed of the
 // slab's slices (a superset of the view window), with a margin of views.
-// False if one slab's views exceed the 4 GiB a buffer resource addresses.
+// False if one slab's views exceed the 4 GiB a buffer resource addresses;
+// *pairs_fit whether they also fit as FP32 row pairs.
 bool slab_view_ranges(const fct_wfbp_gpu_plan* p, const std::vector<double>& zn, int tz,
-                      std::vector<int2>* out) {
+                      std::vector<int2>* out, bool* pairs_fit) {
+  *pairs_fit = true;
   const fct_scan_geometry& s = p->scan;
   const int nslabs = (p->n_native + tz - 1) / tz;
   std::vector<int2>& vr = *out;
@@ -190,9 +192,9 @@ bool slab_view_ranges(const fct_wfbp_gpu_plan* p, const std::vector<double>& zn,
     const double lo = std::floor(va) - 2, hi = std::ceil(vb) + 3;
     vr[sl].x = (int)std::max(0.0, std::min(lo, (double)p->nviews));
     vr[sl].y = (int)std::max(0.0, std::min(hi, (double)p->nviews));
-    if ((size_t)(vr[sl].y - vr[sl].x) * p->nrows * p->cpitch * p->filtered_entry_bytes() >=
-        ((size_t)1 << 32))
-      return false;
+    const size_t entries = (size_t)(vr[sl].y - vr[sl].x) * p->nrows * p->cpitch;
+    if (entries * p->filtered_entry_bytes() >= ((size_t)1 << 32)) return false;
+    if (entries * sizeof(float2) >= ((size_t)1 << 32)) *pairs_fit = false;
   }
   return true;
 }
@@ -212,7 +214,8 @@ int plan_set_tile_z(fct_wfbp_gpu_plan* p, int tz) {
   if (tz != 4 && tz != 8 && tz != 16 && tz != 32) return FCT_ERR_INVALID_ARGUMENT;
   if (tz == p->tile_z) return FCT_OK;
   std::vector<int2> vr;
-  if (!slab_view_ranges(p, native_slice_z(p), tz, &vr))
+  bool pairs_fit;   // (decided for the deepest tile at plan creation)
+  if (!slab_view_ranges(p, native_slice_z(p), tz, &vr, &pairs_fit))
     return set_err(p->ctx, "a slab's view range exceeds 4 GiB of filtered rows"), FCT_ERR_LIMIT;
   int2* d = nullptr;
   HIP_TRY(p->ctx, upload(&d, vr, p->stream));
@@ -555,7 +558,8 @@ namespace fct {
 // Rebin + filter of the whole chain: the lines some slab reads only, the
 // FP16 / BF16 bound from the raw views they read (the stage call
 // fct_wfbp_gpu_rebin_filter filters every line of the scan).
-int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale) {
+int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale,
+                       bool pairs) {
   int2 par, rawr;
   needed_views(p, &par, &rawr);
   const size_t per_view = (size_t)p->raw_scan.n_rows * p->raw_scan.n_channels;
@@ -577,8 +581,36 @@ int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, f
   }
   a.line0 = par.x * p->nrows;
   a.nlines = (par.y - par.x) * p->nrows;
+  a.pairs = pairs;
   HIP_TRY(p->ctx, fct::launch_rebin_filter(a, p->stream));
   return FCT_OK;
+}
+
+int chain_backproject(fct_wfbp_gpu_plan* p, const void* filtered, const float* scale,
+                      float* native, bool pairs) {
+  fct::BpArgs a = bp_args(p);
+  a.filt = filtered;
+  a.filt_scale = scale;
+  a.native = native;
+  HIP_TRY(p->ctx,
+          fct::launch_backproject(a, p->tile_z, p->variant,
+                                  pairs ? kPrecisionPairs : p->opts.precision,
+                                  fct::kBpAccumulate, p->stream));
+  return FCT_OK;
+}
+
+hipError_t plan_alloc_filtered(fct_wfbp_gpu_plan* p) {
+  if (p->d_filtered) return hipSuccess;
+  if (p->pairs) {
+    if (hipMalloc(&p->d_filtered, p->storage_bytes()) == hipSuccess) return hipSuccess;
+    (void)hipGetLastError();
+  }
+  const hipError_t e = hipMalloc(&p->d_filtered, p->filtered_bytes());
+  if (e == hipSuccess)
+    p->pairs = false;
+  else
+    p->d_filtered = nullptr;
+  return e;
 }
 
 }  // namespace fct
@@ -607,7 +639,7 @@ int reconstruct_streaming(fct_wfbp_gpu_plan* p, const ViewSource& src, int vpc,
   int2 par, rawr;
   needed_views(p, &par, &rawr);
   const int nchunks = rawr.y > rawr.x ? (rawr.y - rawr.x + vpc - 1) / vpc : 0;
-  if (!p->d_filtered) HIP_TRY(ctx, hipMalloc(&p->d_filtered, p->filtered_bytes()));
+  HIP_TRY(ctx, fct::plan_alloc_filtered(p));
   if (p->scale_elems() && !p->d_scale)
     HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&p->d_scale), p->scale_elems() * sizeof(float)));
   if (!p->d_native) HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&p->d_native), nat_bytes));
@@ -666,6 +698,7 @@ int reconstruct_streaming(fct_wfbp_gpu_plan* p, const ViewSource& src, int vpc,
   // With adaptive filtration the rebinning reads the filtered copy of each chunk.
   const float* rebin_src = p->af_on ? p->d_af_raw : p->d_raw_stage;
   fct::RebinFilterArgs rf = rf_args(p, rebin_src, p->d_filtered, p->d_scale);
+  rf.pairs = p->pairs;
   rf.skip_scale = 1;
   fct::BpArgs bp = bp_args(p);
   bp.filt = p->d_filtered;
@@ -728,7 +761,7 @@ int reconstruct_streaming(fct_wfbp_gpu_plan* p, const ViewSource& src, int vpc,
     fct::plan_bp_share(p, s_done, s1 - s_done, &bp);
     s_done = s1;
     if (e == hipSuccess)
-      e = fct::launch_backproject(bp, p->tile_z, p->variant, prec, fct::kBpAccumulate, bs);
+      e = fct::launch_backproject(bp, p->tile_z, p->variant, p->storage(), fct::kBpAccumulate, bs);
     if (e == hipSuccess) e = hipEventRecord(p->ev_bp[b], bs);
     bp_busy[b] = true;
     if (e != hipSuccess || !out_early) return e;
@@ -1054,9 +1087,15 @@ FCT_API int fct_wfbp_gpu_plan_create(fct_wfbp_gpu_ctx* ctx, const fct_scan_geome
   for (int t = 0; t < p->H; ++t) p->h_xplanes[t] = std::fabs(cs[t].x) >= std::fabs(cs[t].y);
 
   std::vector<int2> vr;
-  if (!slab_view_ranges(p, zn, p->tile_z, &vr))
+  bool pairs_fit;
+  if (!slab_view_ranges(p, zn, p->tile_z, &vr, &pairs_fit))
     return fail((set_err(ctx, "a slab's view range exceeds 4 GiB of filtered rows"),
                  FCT_ERR_LIMIT));
+  // FP32 whole chains keep row pairs where they fit for every tile depth (a
+  // batch may still change it).
+  std::vector<int2> vr32;
+  p->pairs = p->opts.precision == FCT_PRECISION_FP32 && p->variant == FCT_BP_LEAN &&
+             slab_view_ranges(p, zn, 32, &vr32, &pairs_fit) && pairs_fit;
 
   // Exact view-window slice ranges per (chunk, view): the slices s of the
   // chunk with fct_bp_in_window(zt, zs) true form one interval (the test is
@@ -1575,14 +1614,14 @@ FCT_API int fct_wfbp_gpu_reconstruct(fct_wfbp_gpu_plan* p, const float* raw, flo
   if (host_buffers) return reconstruct_streaming(p, ViewSource{raw, nullptr, nullptr}, 0, 0.0f,
                                                  volume);
   const size_t nat_bytes = (size_t)p->n_native * p->recon.ny * p->recon.nx * sizeof(float);
-  if (!p->d_filtered) HIP_TRY(p->ctx, hipMalloc(&p->d_filtered, p->filtered_bytes()));
+  HIP_TRY(p->ctx, fct::plan_alloc_filtered(p));
   if (p->scale_elems() && !p->d_scale)
     HIP_TRY(p->ctx, hipMalloc(reinterpret_cast<void**>(&p->d_scale),
                               p->scale_elems() * sizeof(float)));
   if (!p->d_native) HIP_TRY(p->ctx, hipMalloc(reinterpret_cast<void**>(&p->d_native), nat_bytes));
-  int st = fct::chain_rebin_filter(p, raw, p->d_filtered, p->d_scale);
+  int st = fct::chain_rebin_filter(p, raw, p->d_filtered, p->d_scale, p->pairs);
   if (st) return st;
-  st = fct_wfbp_gpu_backproject(p, p->d_filtered, p->d_scale, p->d_native);
+  st = fct::chain_backproject(p, p->d_filtered, p->d_scale, p->d_native, p->pairs);
   if (st) return st;
   return fct_wfbp_gpu_thicken(p, p->d_native, volume);
 }

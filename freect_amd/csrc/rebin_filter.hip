@@ -392,6 +392,30 @@ __device__ __forceinline__ void quad_store_pair(const RebinFilterArgs& a, size_t
   if (r > 0) st_nt(q + (e - (size_t)a.cpitch) * 2 + 1, lo);
 }
 
+// Value y of line (view, row r) at channel c into its two row-pair slots (e:
+// entry index of (r, c)); the second slot of the last row is zeroed.
+__device__ __forceinline__ void pair_store(const RebinFilterArgs& a, size_t e, int r, float y) {
+  float* q = static_cast<float*>(a.out);
+  st_nt(q + 2 * e, y);
+  if (r > 0) st_nt(q + 2 * (e - (size_t)a.cpitch) + 1, y);
+  if (r == a.nrows - 1) st_nt(q + 2 * e + 1, 0.0f);
+}
+
+// Rows r (even) and r + 1 of one view: the entry of row r whole, its
+// neighbours' halves.
+__device__ __forceinline__ void pair_store2(const RebinFilterArgs& a, size_t e, int r, float y0,
+                                            float y1) {
+  uint32_t* q = static_cast<uint32_t*>(a.out);
+  const uint32_t lo = __float_as_uint(y0), hi = __float_as_uint(y1);
+  const size_t e1 = e + (size_t)a.cpitch;
+  st_nt(q + 2 * e, lo, hi);
+  if (r + 1 == a.nrows - 1)
+    st_nt(q + 2 * e1, hi, 0u);
+  else
+    st_nt(q + 2 * e1, hi);
+  if (r > 0) st_nt(q + 2 * (e - (size_t)a.cpitch) + 1, lo);
+}
+
 // max|x| over the raw scan as FP32 bits in scale[1] (non-negative floats
 // order like their bit patterns).
 __global__ void scale_reset_kernel(float* scale) {
@@ -486,8 +510,14 @@ __global__ __launch_bounds__(kRfThreads) void rebin_filter_kernel(RebinFilterArg
     float* out = static_cast<float*>(a.out);
     for (int c = threadIdx.x; c < a.cpitch; c += kRfThreads) {
       const bool in = c < a.ncols;
-      out[o0 + c] = in ? Y[c].x : 0.0f;
-      if (has1) out[o1 + c] = in ? -Y[c].y : 0.0f;
+      const float y0 = in ? Y[c].x : 0.0f, y1 = in ? -Y[c].y : 0.0f;
+      if (a.pairs) {
+        pair_store(a, o0 + c, r0, y0);
+        if (has1) pair_store(a, o1 + c, r1, y1);
+        continue;
+      }
+      out[o0 + c] = y0;
+      if (has1) out[o1 + c] = y1;
     }
     return;
   }
@@ -679,8 +709,16 @@ void rebin_filter_reg_kernel(RebinFilterArgs a) {
         if (c < a.cpitch) {
           const FctCplx y = w[fct_fft_final_reg<N>(m)];
           const bool in = c < a.ncols;
-          st_nt(out + o0 + c, in ? y.x : 0.0f);
-          if (has1) st_nt(out + o1 + c, in ? -y.y : 0.0f);
+          const float y0 = in ? y.x : 0.0f, y1 = in ? -y.y : 0.0f;
+          if (!a.pairs) {
+            st_nt(out + o0 + c, y0);
+            if (has1) st_nt(out + o1 + c, y1);
+          } else if (has1 && (r0 & 1) == 0 && r1 == r0 + 1) {
+            pair_store2(a, o0 + c, r0, y0, y1);
+          } else {
+            pair_store(a, o0 + c, r0, y0);
+            if (has1) pair_store(a, o1 + c, r1, y1);
+          }
         }
       }
       continue;

@@ -79,7 +79,18 @@ struct RebinFilterArgs {
   // x raw rows x raw channels), and the smallest aoff and mmax of the table.
   uint32_t group_bytes;
   int32_t aoff_min, mmax_min;
+  int32_t pairs;             // 1: FP32 output as row pairs (kPrecisionPairs)
 };
+
+// FP32 projections stored as row pairs, the layout between the rebinning and
+// the backprojection of the whole chains (plan_pairs): entry (view, row,
+// channel) holds (y[row][channel], y[row + 1][channel]), 0 past the last row,
+// so that the 2 x 2 taps of a sample are 16 consecutive bytes.  An FP32
+// backprojection of rows needs two 8-byte gathers per sample, and the
+// texture-address unit takes 16.7 cycles per 64-lane gather of 8 bytes and
+// 20.3 of 16 (measured, taps of an 8 x 8 tile in L1): 86 % of the kernel's
+// time.  The stage calls keep the row layout of their interface.
+constexpr int kPrecisionPairs = 3;
 
 // Everything the backprojection kernel reads.
 struct BpArgs {
@@ -317,7 +328,15 @@ BpArgs plan_bp_args(const fct_wfbp_gpu_plan* p);   // tables only (no buffers)
 void plan_bp_share(const fct_wfbp_gpu_plan* p, int slab0, int count, BpArgs* a);
 int plan_set_tile_z(fct_wfbp_gpu_plan* p, int tz);  // rebuilds the slab view ranges
 // Rebin + filter of the lines some slab reads (the whole-chain entry points).
-int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale);
+int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale,
+                       bool pairs);
+// The lean backprojection of filtered projections in the plan's own layout
+// (pairs), or in the interface's.
+int chain_backproject(fct_wfbp_gpu_plan* p, const void* filtered, const float* scale,
+                      float* native, bool pairs);
+// Allocates the plan's filtered projections, as pairs where p->pairs; where
+// there is no memory for those, as rows (p->pairs becomes false).
+hipError_t plan_alloc_filtered(fct_wfbp_gpu_plan* p);
 }  // namespace fct
 
 struct fct_wfbp_gpu_ctx {
@@ -372,6 +391,7 @@ struct fct_wfbp_gpu_plan {
   float* d_thk_w = nullptr;
 
   // Intermediate buffers for fct_wfbp_gpu_reconstruct (allocated on first use).
+  bool pairs = false;               // d_filtered holds FP32 row pairs (kPrecisionPairs)
   void* d_filtered = nullptr;
   float* d_scale = nullptr;
   float* d_native = nullptr;
@@ -417,6 +437,9 @@ struct fct_wfbp_gpu_plan {
   size_t filtered_bytes() const {
     return (size_t)nviews * nrows * cpitch * filtered_entry_bytes();
   }
+  // The plan's own buffer between the stages of a whole chain.
+  int storage() const { return pairs ? fct::kPrecisionPairs : opts.precision; }
+  size_t storage_bytes() const { return filtered_bytes() * (pairs ? 2 : 1); }
   size_t scale_elems() const {
     return opts.precision == FCT_PRECISION_FP32 ? 0 : (size_t)fct::kScaleElems;
   }

@@ -1,9 +1,9 @@
 """The lean backprojection's choice of a theta~'s views (a ballot over 64 of
 them at a time, whole slabs first, the exact window table only near the
-window's ends) and its storage of FP32 whole chains: feeds so small that a slab
+window's ends) and the row pairs of FP32 whole chains: feeds so small that a slab
 has more than 64 views per theta~, view windows that cut into the slabs, a table
 that moves down, odd row counts, every tile depth, against the direct kernel,
-which tests each (voxel, view) pair.  Both add the same FP32 terms (the lean
+which tests each (voxel, view) pair on plain rows.  Both add the same FP32 terms (the lean
 kernel's mean through v_rcp_f32, 1 ulp), in another order of a theta~'s views:
 sums over at most a few hundred theta~ differ by rounding, 2e-5 of the largest
 voxel.
@@ -25,17 +25,20 @@ def ctx():
 
 
 @pytest.mark.parametrize("tile_z", [4, 8, 16, 32])
-@pytest.mark.parametrize("rows,feed_rows,ppr,rotations,slices,down,precision",
-                         [(8, 0.2, 12, 90.0, 17, False, "fp32"),
-                          (8, 0.2, 12, 90.0, 17, True, "fp16"),
-                          (16, 4.0, 48, 8.0, 40, False, "fp32"),
-                          (16, 6.0, 48, 6.0, 9, True, "bf16"),
-                          (11, 9.0, 64, 4.0, 20, True, "fp32"),
-                          (11, 9.0, 64, 4.0, 20, False, "fp16")])
+@pytest.mark.parametrize("rows,feed_rows,ppr,rotations,slices,down,channels,precision",
+                         [(8, 0.2, 12, 90.0, 17, False, 96, "fp32"),
+                          (8, 0.2, 12, 90.0, 17, True, 96, "fp16"),
+                          (16, 4.0, 48, 8.0, 40, False, 96, "fp32"),
+                          (16, 6.0, 48, 6.0, 9, True, 96, "bf16"),
+                          (11, 9.0, 64, 4.0, 20, True, 96, "fp32"),
+                          (11, 9.0, 64, 4.0, 20, False, 300, "fp32"),
+                          (12, 9.0, 64, 4.0, 20, False, 257, "fp32"),
+                          (11, 9.0, 64, 4.0, 20, False, 96, "fp16")])
 def test_view_choice_against_direct(ctx, tile_z, rows, feed_rows, ppr, rotations, slices, down,
-                                    precision):
+                                    channels, precision):
     from freect_amd import wfbp
-    w = S.tiny(nx=26, n_slices=slices, n_rows=rows, ppr=ppr, rotations=rotations, seed=5)
+    w = S.tiny(nx=26, n_slices=slices, n_rows=rows, ppr=ppr, rotations=rotations, seed=5,
+               n_channels=channels)
     feed = feed_rows * w.scan.effective().csw * (-1.0 if down else 1.0)
     scan = w.scan.replace(feed=feed, z0=-0.5 * (w.scan.n_views - 1) * feed / ppr)
     raw = ctx.phantom_project(scan, w.phantom, 0.0, w.seed)
