@@ -1403,11 +1403,14 @@ FCT_API int fct_wfbp_gpu_ray_project(fct_wfbp_gpu_plan* p, const float* native, 
   a.raw_out = raw;
   fct::RayTables t;
   if (ray_tables(p, a, &t)) {
-    if (!p->d_ray_pad)
-      p->d_ray_pad =
-          static_cast<float*>(try_scratch(p, 2 * fct::ray_pad_elems(a) * sizeof(float)));
+    const size_t pad = 2 * fct::ray_pad_elems(a);
+    if (!p->d_ray_pad && fct::ray_pad_pairs(a)) {
+      p->d_ray_pad = static_cast<float*>(try_scratch(p, pad * sizeof(float2)));
+      p->ray_pad_pairs = p->d_ray_pad != nullptr;
+    }
+    if (!p->d_ray_pad) p->d_ray_pad = static_cast<float*>(try_scratch(p, pad * sizeof(float)));
     if (p->d_ray_pad) {
-      HIP_TRY(p->ctx, fct::launch_ray_project_table(a, t, p->d_ray_pad, p->stream));
+      HIP_TRY(p->ctx, fct::launch_ray_project_table(a, t, p->d_ray_pad, p->ray_pad_pairs, p->stream));
       return FCT_OK;
     }
   }

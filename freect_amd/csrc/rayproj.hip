@@ -189,10 +189,16 @@ __global__ __launch_bounds__(256) void ray_table_kernel(RayProjArgs a, RayTables
 // with x and y exchanged, so that the projector reads neighbouring samples of
 // neighbouring rays from neighbouring addresses for either plane axis and
 // needs no bounds test (a sample's footprint may reach two planes outside).
+// T float2: entry (z, y, x) holds slices z and z + 1, so that the four taps
+// of a sample are 16 consecutive bytes.
 constexpr int kPad = 2;
-__global__ __launch_bounds__(256) void ray_pad_kernel(RayProjArgs a, float* __restrict__ nat,
-                                                      float* __restrict__ swp) {
-  __shared__ float tile[32][33];
+__device__ __forceinline__ void pad_entry(float* e, float v, float) { *e = v; }
+__device__ __forceinline__ void pad_entry(float2* e, float v, float up) { *e = make_float2(v, up); }
+
+template <class T>
+__global__ __launch_bounds__(256) void ray_pad_kernel(RayProjArgs a, T* __restrict__ nat,
+                                                      T* __restrict__ swp) {
+  __shared__ T tile[32][33];
   const int px = a.nx + 2 * kPad, py = a.ny + 2 * kPad;
   const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
@@ -201,8 +207,12 @@ __global__ __launch_bounds__(256) void ray_pad_kernel(RayProjArgs a, float* __re
     const size_t plane = (size_t)kz * px * py;
     for (int r = ty; r < 32; r += 8) {
       const int X = bx + tx, Y = by + r, x = X - kPad, y = Y - kPad;
-      const bool in = x >= 0 && x < a.nx && y >= 0 && y < a.ny && z >= 0 && z < a.nz;
-      const float v = in ? a.vol_in[((size_t)z * a.ny + y) * a.nx + x] : 0.0f;
+      const bool in = x >= 0 && x < a.nx && y >= 0 && y < a.ny;
+      auto at = [&](int s) {
+        return in && s >= 0 && s < a.nz ? a.vol_in[((size_t)s * a.ny + y) * a.nx + x] : 0.0f;
+      };
+      T v;
+      pad_entry(&v, at(z), sizeof(T) == sizeof(float) ? 0.0f : at(z + 1));
       if (X < px && Y < py) nat[plane + (size_t)Y * px + X] = v;
       tile[r][tx] = v;
     }
@@ -230,25 +240,36 @@ constexpr int kRsrcWord3 = 0x00020000;   // raw buffer, 32-bit data format (gfx9
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 
-// A plane's four taps: two 8-byte loads (slices k and k + 1 at j, j + 1).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// A plane's four taps: one 16-byte load (T float2), or two 8-byte loads
+// (slices k and k + 1 at j, j + 1).
 struct RayTap {
   u32x2 a, b;
   float wq, wz;
 };
 
+template <class T>
 struct RayWalk {
   float Aq, Bq, Az, Bz;
-  __amdgpu_buffer_rsrc_t r0, r1;   // the padded volume from slice -2 and from slice -1
-  int plane_bytes, row_bytes, origin;   // origin: byte offset of (0, 0, 0) past the padding
+  __amdgpu_buffer_rsrc_t r0, r1;   // the padded volume from slice -2 and (float) from slice -1
+  // Entries of a plane, bytes of a row, byte offset of (0, 0, 0) past the padding.
+  int plane, row_bytes, origin;
   __device__ __forceinline__ RayTap fetch(int i) const {
     RayTap t;
     const float fq = fmaf((float)i, Bq, Aq), fz = fmaf((float)i, Bz, Az);
     const int j = floor_int(fq), k = floor_int(fz);
     t.wq = __builtin_amdgcn_fractf(fq);
     t.wz = __builtin_amdgcn_fractf(fz);
-    const int o = __mul24(k, plane_bytes) + origin + (j << 2);
-    t.a = __builtin_amdgcn_raw_buffer_load_b64(r0, o, i * row_bytes, 0);
-    t.b = __builtin_amdgcn_raw_buffer_load_b64(r1, o, i * row_bytes, 0);
+    const int o = (__mul24(k, plane) + j) * (int)sizeof(T) + origin;
+    if constexpr (sizeof(T) == sizeof(float2)) {
+      const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(r0, o, i * row_bytes, 0);
+      t.a = u32x2{q.x, q.z};
+      t.b = u32x2{q.y, q.w};
+    } else {
+      t.a = __builtin_amdgcn_raw_buffer_load_b64(r0, o, i * row_bytes, 0);
+      t.b = __builtin_amdgcn_raw_buffer_load_b64(r1, o, i * row_bytes, 0);
+    }
     return t;
   }
 };
@@ -264,15 +285,17 @@ __device__ __forceinline__ float ray_combine(const RayTap& t) {
 // four rows per workgroup: the waves of a workgroup read the same columns of
 // neighbouring slices.  A wave's lanes advance plane by plane together; the
 // planes that every one of its rays samples run unmasked, four at a time
-// (eight loads in flight).  About 15 VALU instructions and two 8-byte loads
-// per sample instead of 40 and four: 1476 views x 16 x 736 rays through
-// 384 x 384 x 32 voxels 30.8 -> 5.9 ms.  The loads bind it (19 cycles of a
-// CU's L1 each, VALU 2.8 ms of the 5.9); 1 to 16 rows per workgroup and 2 to
-// 8 planes in flight are within 2 %.
+// (their loads in flight).  About 15 VALU instructions and one 16-byte load
+// per sample instead of 40 and four loads: 1476 views x 16 x 736 rays through
+// 384 x 384 x 32 voxels 30.8 -> 5.9 ms with two 8-byte loads (which bound it:
+// 19 cycles of a CU's L1 each, VALU 2.8 ms of the 5.9), 4.3 ms with one of 16
+// bytes (20 cycles).  1 to 16 rows per workgroup and 2 to 8 planes in flight
+// are within 2 %.
 constexpr int kRayRows = 4;
+template <class T>
 __global__ __launch_bounds__(64 * kRayRows) void ray_project_table_kernel(RayProjArgs a, RayTables t,
-                                                                const float* __restrict__ nat,
-                                                                const float* __restrict__ swp,
+                                                                const T* __restrict__ nat,
+                                                                const T* __restrict__ swp,
                                                                 uint32_t pad_bytes) {
   const int cg = (a.ncols + 63) >> 6, rg = (a.nrows + kRayRows - 1) / kRayRows;
   const int id = xcd_block(blockIdx.x, gridDim.x);
@@ -286,7 +309,7 @@ __global__ __launch_bounds__(64 * kRayRows) void ray_project_table_kernel(RayPro
   const double oz = a.states > 1 ? t.zsrc[v % a.states] : 0.0;
   const double wz = ((double)row - a.cr) * a.drow - oz;
   const double g = wz / a.ddz;
-  RayWalk w;
+  RayWalk<T> w;
   w.Aq = e.x;
   w.Bq = e.y;
   w.Az = (float)(t.zoff[v] + (double)e.z * g);
@@ -297,7 +320,8 @@ __global__ __launch_bounds__(64 * kRayRows) void ray_project_table_kernel(RayPro
   const bool any_plane = in && flo <= fhi;
   const int ilo = any_plane ? (int)ceilf(flo) : 0, ihi = any_plane ? (int)floorf(fhi) : -1;
   const int px = a.nx + 2 * kPad, py = a.ny + 2 * kPad;
-  w.plane_bytes = px * py * 4;
+  w.plane = px * py;
+  const uint32_t plane_bytes = (uint32_t)w.plane * (uint32_t)sizeof(T);
   float acc = 0.0f;
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
@@ -309,10 +333,10 @@ __global__ __launch_bounds__(64 * kRayRows) void ray_project_table_kernel(RayPro
     if (!mine) continue;
     const char* base = reinterpret_cast<const char*>(m ? swp : nat);
     w.r0 = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)pad_bytes, kRsrcWord3);
-    w.r1 = __builtin_amdgcn_make_buffer_rsrc((void*)(base + w.plane_bytes), 0,
-                                             (int)(pad_bytes - (uint32_t)w.plane_bytes), kRsrcWord3);
-    w.row_bytes = (m ? py : px) * 4;
-    w.origin = kPad * (w.plane_bytes + w.row_bytes + 4);
+    w.r1 = __builtin_amdgcn_make_buffer_rsrc((void*)(base + plane_bytes), 0,
+                                             (int)(pad_bytes - plane_bytes), kRsrcWord3);
+    w.row_bytes = (m ? py : px) * (int)sizeof(T);
+    w.origin = kPad * ((int)plane_bytes + w.row_bytes + (int)sizeof(T));
     int i = u0;
     for (; i <= u1 && i < b0; ++i)
       if (i >= ilo && i <= ihi) acc += ray_combine(w.fetch(i));
@@ -561,17 +585,29 @@ hipError_t launch_ray_table(const RayProjArgs& a, const RayTables& t, hipStream_
   return hipGetLastError();
 }
 
-hipError_t launch_ray_project_table(const RayProjArgs& a, const RayTables& t, float* pad,
-                                    hipStream_t s) {
+// Whether a padded copy with two slices per entry is within a buffer
+// resource's range too (else the copies hold one).
+bool ray_pad_pairs(const RayProjArgs& a) {
+  return (double)ray_pad_elems(a) * sizeof(float2) < 4294967000.0;
+}
+
+template <class T>
+hipError_t launch_project_table(const RayProjArgs& a, const RayTables& t, T* pad, hipStream_t s) {
   const size_t n = ray_pad_elems(a);
-  hipLaunchKernelGGL(ray_pad_kernel,
+  hipLaunchKernelGGL(ray_pad_kernel<T>,
                      dim3((a.nx + 2 * kPad + 31) / 32, (a.ny + 2 * kPad + 31) / 32,
                           std::min(a.nz + 2 * kPad, 65535)),
                      dim3(256), 0, s, a, pad, pad + n);
   const int blocks = a.v1 * ((a.nrows + kRayRows - 1) / kRayRows) * ((a.ncols + 63) / 64);
-  hipLaunchKernelGGL(ray_project_table_kernel, dim3(blocks), dim3(64 * kRayRows), 0, s, a, t, pad,
-                     pad + n, (uint32_t)(n * sizeof(float)));
+  hipLaunchKernelGGL(ray_project_table_kernel<T>, dim3(blocks), dim3(64 * kRayRows), 0, s, a, t, pad,
+                     pad + n, (uint32_t)(n * sizeof(T)));
   return hipGetLastError();
+}
+
+hipError_t launch_ray_project_table(const RayProjArgs& a, const RayTables& t, float* pad,
+                                    bool pairs, hipStream_t s) {
+  return pairs ? launch_project_table(a, t, reinterpret_cast<float2*>(pad), s)
+               : launch_project_table(a, t, pad, s);
 }
 
 hipError_t launch_ray_gather(const RayProjArgs& a, const RayTables& t, float* rec, int ncu,

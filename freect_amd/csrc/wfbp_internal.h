@@ -259,14 +259,16 @@ hipError_t launch_rebin_filter(const RebinFilterArgs& a, hipStream_t s);
 // transpose its exact transpose from raw_in into vol_out (accumulated).
 hipError_t launch_ray_project(const RayProjArgs& a, bool transpose, hipStream_t s);
 // Table-driven forms: whether they apply, the tables (of ray_table_bytes) and
-// the projector's padded volume copies (2 x ray_pad_elems floats).
+// the projector's padded volume copies (2 x ray_pad_elems entries of one
+// slice, or of two where ray_pad_pairs).
 bool ray_tables_apply(const RayProjArgs& a);
 size_t ray_table_bytes(const RayProjArgs& a);
 size_t ray_pad_elems(const RayProjArgs& a);
+bool ray_pad_pairs(const RayProjArgs& a);
 RayTables ray_table_layout(const RayProjArgs& a, void* mem);
 hipError_t launch_ray_table(const RayProjArgs& a, const RayTables& t, hipStream_t s);
 hipError_t launch_ray_project_table(const RayProjArgs& a, const RayTables& t, float* pad,
-                                    hipStream_t s);
+                                    bool pairs, hipStream_t s);
 // rec: 3 floats per ray.
 hipError_t launch_ray_gather(const RayProjArgs& a, const RayTables& t, float* rec, int ncu,
                              hipStream_t s);
@@ -400,6 +402,7 @@ struct fct_wfbp_gpu_plan {
   void* d_ray_tab = nullptr;        // ray projector tables (first use; ready: filled)
   bool ray_tab_ready = false;
   float* d_ray_pad = nullptr;       // padded volume copies of the ray projector (first use)
+  bool ray_pad_pairs = false;       // with two slices per entry
   float* d_ray_rec = nullptr;       // per-ray records of its transpose (first use)
   float* d_adj_wgt = nullptr;       // gathered transpose: voxel weights / swapped volume (first use)
   size_t adj_wgt_elems = 0;

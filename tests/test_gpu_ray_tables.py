@@ -90,3 +90,30 @@ def test_first_call_inside_a_capture(ctx):
     p.synchronize()
     assert (a - qx).abs().max() <= 2e-5 * qx.abs().max()
     assert (b - qt).abs().max() <= 2e-5 * qt.abs().max()
+
+
+def test_volume_beyond_the_paired_copies(ctx):
+    # A volume whose padded copies exceed 4 GiB with two slices per entry: the
+    # copies hold one.  Its only nonzero slices are those of a small plan on
+    # the same grid (two slices per entry).  Slice positions of up to ~1100
+    # slices carry half an ulp, 1.2e-4 slices, twice (the ray's start and the
+    # sample): at most 2.4e-4 of a difference of neighbouring values, a third
+    # on average against a mean value of a half: 2e-4 of the largest output.
+    from freect_amd import wfbp
+    sc, rc = _setup(nx=512, ny=512, nz=2, rows=8, chans=96, fov=300.0, ppr=24)
+    csw = sc.effective().csw
+    big = wfbp.Plan(ctx, sc, rc.replace(start_pos=-1020 * csw, end_pos=1020.5 * csw))
+    small = wfbp.Plan(ctx, sc, rc.replace(start_pos=-8 * csw, end_pos=7.5 * csw))
+    nz, ns = big.info.n_slices_native, small.info.n_slices_native
+    assert ns == 16 and (nz + 4) * 516 * 516 * 8 > 4294967000 > (nz + 4) * 516 * 516 * 4
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.rand((ns, 512, 512), device="cuda", generator=gen)
+    xb = torch.zeros((nz, 512, 512), device="cuda")
+    xb[1012:1012 + ns] = x
+    a, b = small.alloc_raw().fill_(float("nan")), big.alloc_raw().fill_(float("nan"))
+    small.ray_project(x, a)
+    big.ray_project(xb, b)
+    small.synchronize()
+    big.synchronize()
+    assert a.abs().max() > 0
+    assert (a - b).abs().max() <= 2e-4 * a.abs().max()
