@@ -171,7 +171,10 @@ __global__ __launch_bounds__(256) void bp_adjoint_column_kernel(BpAdjArgs a, Adj
 
 // xbar * scale / sum W of every voxel for the theta~ [t0, t0 + nt) (0 where no
 // view selects the voxel), in that order: one wave per 64 voxels along the
-// secondary axis and eight slices.
+// secondary axis and eight slices.  Bound by the writes (9.3 GB for 384 x 384 x
+// 32 voxels x 492 theta~) and by VALU issue together: 4.5 -> 3.75 ms with the
+// mask-free weight and the reciprocal, which is the forward kernel's
+// (num v_rcp(den)), in place of a division.
 constexpr int kAdjSlices = 8;
 template <bool CENTERED>
 __global__ __launch_bounds__(64) void bp_adjoint_weights_kernel(BpAdjArgs a, AdjGather q) {
@@ -223,9 +226,16 @@ __global__ __launch_bounds__(64) void bp_adjoint_weights_kernel(BpAdjArgs a, Adj
           for (int i = 0; i < kAdjSlices; ++i) {
             if (s0 + i < wx || s0 + i > wy) continue;
             const float qi = fmaf(zs[i], invL, row0);
+            if (CENTERED) {
+              // W = 0 exactly on every row outside the detector and in the
+              // lanes at row -1e30 (t clamped to [0, 1]): no mask.
+              den[i] += fct_w_of_t(
+                  __builtin_amdgcn_fmed3f(fmaf(-fabsf(qi - g.cr), g.wk, FCT_WC), 0.0f, 1.0f));
+              continue;
+            }
             const int iq = floor_int(qi);
-            bool sel = ok && (uint32_t)iq <= (uint32_t)(g.nrows - 2);
-            if (!CENTERED) sel = sel && !(fabsf(qi - g.cr) > g.hr);
+            const bool sel = ok && (uint32_t)iq <= (uint32_t)(g.nrows - 2) &&
+                             !(fabsf(qi - g.cr) > g.hr);
             const float W = fct_w_of_row(qi, g);
             den[i] += sel ? W : 0.0f;
           }
@@ -235,7 +245,7 @@ __global__ __launch_bounds__(64) void bp_adjoint_weights_kernel(BpAdjArgs a, Adj
     if (inb)
 #pragma unroll
       for (int i = 0; i < kAdjSlices; ++i)
-        if (i < nz) out[(size_t)i * ns] = den[i] > 0.0f ? xb[i] / den[i] : 0.0f;
+        if (i < nz) out[(size_t)i * ns] = den[i] > 0.0f ? xb[i] * __builtin_amdgcn_rcpf(den[i]) : 0.0f;
   }
 }
 
@@ -264,7 +274,7 @@ __global__ __launch_bounds__(256) void swap_volume_kernel(const float* __restric
 // and write of two rows per slice, conflict-free).  Bound by VALU issue: 25
 // instructions per slice of a candidate, of whose lanes half to three quarters
 // hold one.  2952 views x 16 x 736 from 384 x 384 x 32 voxels: 287 ms with
-// four global atomics per sample -> 4.5 (weights) + 10.8 ms.  RC rows per
+// four global atomics per sample -> 3.75 (weights) + 11.3 ms.  RC rows per
 // wave: 16 or 32, so that the rows in LDS leave at least 16 waves per CU.
 template <int RC, bool CENTERED, bool MATCHED>
 __global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjGather q) {
