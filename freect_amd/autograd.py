@@ -34,7 +34,7 @@ class WFBPFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, raw, plan):
         native = plan.alloc_native()
-        plan.forward_native(raw.contiguous(), native)
+        plan.forward_volume(raw.contiguous(), native)
         ctx.plan = plan
         return native
 

@@ -558,17 +558,10 @@ namespace fct {
 // Rebin + filter of the whole chain: the lines some slab reads only, the
 // FP16 / BF16 bound from the raw views they read (the stage call
 // fct_wfbp_gpu_rebin_filter filters every line of the scan).
-int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale,
-                       bool pairs) {
+int chain_lines(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale, bool pairs) {
   int2 par, rawr;
   needed_views(p, &par, &rawr);
   const size_t per_view = (size_t)p->raw_scan.n_rows * p->raw_scan.n_channels;
-  if (p->af_on) {   // adaptive filtration of the views read, into the plan's buffer
-    HIP_TRY(p->ctx, fct::launch_adaptive_filter(raw, p->d_af_raw, p->d_af_vmax, rawr.x, rawr.y,
-                                                p->raw_scan.n_rows, p->raw_scan.n_channels,
-                                                p->af_s, p->stream));
-    raw = p->d_af_raw;
-  }
   fct::RebinFilterArgs a = rf_args(p, raw, filtered, scale);
   if (p->opts.precision != FCT_PRECISION_FP32) {
     HIP_TRY(p->ctx, fct::launch_scale_reset(scale, p->stream));
@@ -584,6 +577,19 @@ int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, f
   a.pairs = pairs;
   HIP_TRY(p->ctx, fct::launch_rebin_filter(a, p->stream));
   return FCT_OK;
+}
+
+int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale,
+                       bool pairs) {
+  if (p->af_on) {   // adaptive filtration of the views read, into the plan's buffer
+    int2 par, rawr;
+    needed_views(p, &par, &rawr);
+    HIP_TRY(p->ctx, fct::launch_adaptive_filter(raw, p->d_af_raw, p->d_af_vmax, rawr.x, rawr.y,
+                                                p->raw_scan.n_rows, p->raw_scan.n_channels,
+                                                p->af_s, p->stream));
+    raw = p->d_af_raw;
+  }
+  return chain_lines(p, raw, filtered, scale, pairs);
 }
 
 int chain_backproject(fct_wfbp_gpu_plan* p, const void* filtered, const float* scale,
@@ -1383,6 +1389,21 @@ FCT_API int fct_wfbp_gpu_backproject(fct_wfbp_gpu_plan* p, const void* filtered,
   HIP_TRY(p->ctx, fct::launch_backproject(a, p->tile_z, p->variant, p->opts.precision,
                                           fct::kBpAccumulate, p->stream));
   return FCT_OK;
+}
+
+FCT_API int fct_wfbp_gpu_forward_native(fct_wfbp_gpu_plan* p, const float* raw, void* scratch,
+                                        int64_t scratch_bytes, float* native) {
+  if (!p || !raw || !scratch || !native) return FCT_ERR_INVALID_ARGUMENT;
+  if (p->opts.precision != FCT_PRECISION_FP32)
+    return set_err(p->ctx, "forward_native needs an FP32 plan"), FCT_ERR_INVALID_ARGUMENT;
+  if (scratch_bytes < 0 || (size_t)scratch_bytes < p->filtered_bytes())
+    return set_err(p->ctx, "forward_native: scratch smaller than filtered_bytes"),
+           FCT_ERR_INVALID_ARGUMENT;
+  HIP_TRY(p->ctx, hipSetDevice(p->device));
+  const bool pairs = p->pairs && (size_t)scratch_bytes >= 2 * p->filtered_bytes() &&
+                     (reinterpret_cast<uintptr_t>(scratch) & 7) == 0;
+  const int st = fct::chain_lines(p, raw, scratch, nullptr, pairs);
+  return st ? st : fct::chain_backproject(p, scratch, nullptr, native, pairs);
 }
 
 FCT_API int fct_wfbp_gpu_thicken(fct_wfbp_gpu_plan* p, const float* native, float* volume) {

@@ -86,6 +86,7 @@ SIGNATURES = {
     "fct_wfbp_gpu_set_stream": (C.c_int, [_VP, _VP]),
     "fct_wfbp_gpu_rebin_filter": (C.c_int, [_VP, _VP, _VP, _VP]),
     "fct_wfbp_gpu_backproject": (C.c_int, [_VP, _VP, _VP, _VP]),
+    "fct_wfbp_gpu_forward_native": (C.c_int, [_VP, _VP, _VP, C.c_int64, _VP]),
     "fct_wfbp_gpu_thicken": (C.c_int, [_VP, _VP, _VP]),
     "fct_wfbp_gpu_reconstruct": (C.c_int, [_VP, _VP, _VP, C.c_int32]),
     "fct_wfbp_gpu_reconstruct_stream": (C.c_int, [_VP, _VP, _VP, C.c_int32, C.c_float, _VP]),
@@ -536,6 +537,21 @@ class Plan:
         self.rebin_filter(raw, filt)
         self.backproject(filt, None, native)
         return filt
+
+    def forward_volume(self, raw, native):
+        """raw -> native volume as forward_native, without the filtered
+        projections: only what the volume needs of them, in the layout the
+        backprojection reads fastest."""
+        import torch
+        n = 2 * self.info.filtered_bytes
+        try:
+            scratch = torch.empty(n, dtype=torch.uint8, device=self._dev())
+        except torch.cuda.OutOfMemoryError:   # the row layout
+            n //= 2
+            scratch = torch.empty(n, dtype=torch.uint8, device=self._dev())
+        self.ctx.check(load_library().fct_wfbp_gpu_forward_native(
+            self.h, self._raw(raw, "raw"), scratch.data_ptr(), n,
+            self._native(native, "native")), "forward_native")
 
     def count_voxel_views(self, per_voxel=None) -> int:
         tot = C.c_int64(0)

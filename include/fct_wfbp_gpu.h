@@ -212,6 +212,14 @@ FCT_API int fct_wfbp_gpu_rebin_filter(fct_wfbp_gpu_plan* plan, const float* raw,
 FCT_API int fct_wfbp_gpu_backproject(fct_wfbp_gpu_plan* plan, const void* filtered,
                                      const float* scale, float* native);
 
+/* Raw scan to native volume (rebinning, filter, backprojection of the lines
+ * and views the volume needs; no adaptive filtration), FP32 plans, device
+ * buffers.  scratch holds the filtered projections between the stages, at
+ * least filtered_bytes; with twice that the faster row-pair layout is used
+ * where the plan can hold it.  The volume is the same either way. */
+FCT_API int fct_wfbp_gpu_forward_native(fct_wfbp_gpu_plan* plan, const float* raw, void* scratch,
+                                        int64_t scratch_bytes, float* native);
+
 /* Triangular slice thickening (ReconstructionMachine.cu:387-434,
  * cuda_kernels.cuh:289-320). */
 FCT_API int fct_wfbp_gpu_thicken(fct_wfbp_gpu_plan* plan, const float* native, float* volume);

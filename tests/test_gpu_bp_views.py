@@ -51,3 +51,27 @@ def test_view_choice_against_direct(ctx, tile_z, rows, feed_rows, ppr, rotations
         vols.append(v)
     assert vols[0].abs().max() > 0
     assert (vols[1] - vols[0]).abs().max() <= 2e-5 * vols[0].abs().max()
+
+
+@pytest.mark.parametrize("rows,channels", [(8, 96), (11, 300)])
+def test_forward_volume_layouts(ctx, rows, channels):
+    # The chain to the native volume through row pairs, through rows (no room
+    # for pairs) and through the stage calls: the same arithmetic, bitwise.
+    from freect_amd import wfbp
+    w = S.tiny(nx=26, n_slices=20, n_rows=rows, rotations=3.0, seed=5, n_channels=channels)
+    raw = ctx.phantom_project(w.scan, w.phantom, 0.0, w.seed)
+    p = wfbp.Plan(ctx, w.scan, w.recon)
+    ref, vol = p.alloc_native(), p.alloc_native().fill_(float("nan"))
+    p.forward_native(raw, ref)
+    p.forward_volume(raw, vol)
+    p.synchronize()
+    assert ref.abs().max() > 0 and torch.equal(vol, ref)
+    n = p.info.filtered_bytes
+    buf = torch.full((2 * n,), 255, dtype=torch.uint8, device="cuda")   # NaNs
+    call = wfbp.load_library().fct_wfbp_gpu_forward_native
+    for off, size in ((0, n), (4, 2 * n - 4)):   # rows: too small, and misaligned, for pairs
+        vol.fill_(float("nan"))
+        assert call(p.h, raw.data_ptr(), buf.data_ptr() + off, size, vol.data_ptr()) == 0
+        p.synchronize()
+        assert torch.equal(vol, ref)
+    assert call(p.h, raw.data_ptr(), buf.data_ptr(), n - 1, vol.data_ptr()) == 1
