@@ -732,7 +732,7 @@ hipError_t launch3(const BpArgs& a, int mode, hipStream_t s) {
                          a);
       return hipGetLastError();
     }
-    if constexpr (PREC == FCT_PRECISION_FP32) {
+    if constexpr (PREC == FCT_PRECISION_FP32 || PREC == kPrecisionPairs) {
       if (a.nseg > 1 && mode == kBpMatched) {
         hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks),
                            dim3(64 * a.nseg), a.nseg * TZ * 64 * sizeof(float),
@@ -743,14 +743,12 @@ hipError_t launch3(const BpArgs& a, int mode, hipStream_t s) {
   }
   if (mode == kBpAccumulate)
     hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks), dim3(64), 0, s, a);
-  else if constexpr (PREC != kPrecisionPairs) {
-    if (mode == kBpCount)
-      hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpCount, C>), dim3(blocks), dim3(64), 0, s, a);
-    else if (mode == kBpMatched && PREC == FCT_PRECISION_FP32)
-      hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks), dim3(64), 0, s, a);
-    else
-      return hipErrorInvalidValue;
-  }
+  else if (mode == kBpCount && PREC != kPrecisionPairs)
+    hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpCount, C>), dim3(blocks), dim3(64), 0, s, a);
+  else if (mode == kBpMatched && (PREC == FCT_PRECISION_FP32 || PREC == kPrecisionPairs))
+    hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks), dim3(64), 0, s, a);
+  else
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
@@ -766,9 +764,7 @@ hipError_t launch1(const BpArgs& a, int precision, int mode, hipStream_t s) {
     case FCT_PRECISION_FP32: return launch2<TZ, FCT_PRECISION_FP32>(a, mode, s);
     case FCT_PRECISION_FP16: return launch2<TZ, FCT_PRECISION_FP16>(a, mode, s);
     case FCT_PRECISION_BF16: return launch2<TZ, FCT_PRECISION_BF16>(a, mode, s);
-    case kPrecisionPairs:
-      if (mode != kBpAccumulate) break;
-      return launch2<TZ, kPrecisionPairs>(a, mode, s);
+    case kPrecisionPairs: return launch2<TZ, kPrecisionPairs>(a, mode, s);
   }
   return hipErrorInvalidValue;
 }

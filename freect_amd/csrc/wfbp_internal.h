@@ -312,6 +312,8 @@ hipError_t launch_backproject_batch(const BpBatchArgs& b, int tile_z, int precis
                                     bool centered, int grid, hipStream_t s);
 hipError_t backproject_batch_waves_per_cu(int tile_z, int precision, int* waves);
 hipError_t launch_thicken(const ThickenArgs& a, hipStream_t s);
+hipError_t launch_row_pairs(const float* rows, void* out, int nviews, int nrows, int cpitch,
+                            hipStream_t s);
 hipError_t launch_phantom(const PhantomArgs& a, hipStream_t s);
 
 // kBpMatched: the plain R / l-weighted sum over every view that sees the

@@ -75,3 +75,24 @@ def test_forward_volume_layouts(ctx, rows, channels):
         p.synchronize()
         assert torch.equal(vol, ref)
     assert call(p.h, raw.data_ptr(), buf.data_ptr(), n - 1, vol.data_ptr()) == 1
+
+
+@pytest.mark.parametrize("rows,nx", [(9, 60), (8, 61), (8, 8)])
+def test_matched_backprojection_of_row_pairs(ctx, rows, nx):
+    # Volumes large enough for the row pairs, and one that is not, against
+    # the projector that is its transpose: <M x, y> = <x, M^T y>, positive x
+    # and y, so that the FP32 rounding of sums of at most a few thousand terms
+    # stays below 1e-5 of the product.
+    from freect_amd import wfbp
+    w = S.tiny(nx=nx, n_slices=19, n_rows=rows, rotations=2.5, seed=5)
+    p = wfbp.Plan(ctx, w.scan, w.recon)
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.rand((p.info.n_slices_native, nx, nx), device="cuda", generator=gen)
+    y = p.alloc_lines()
+    y.copy_(torch.rand(y.shape, device="cuda", generator=gen))
+    px, py = p.alloc_lines(), p.alloc_native().fill_(float("nan"))
+    p.matched_project(x, px)
+    p.matched_backproject(y, py)
+    p.synchronize()
+    a, b = (px.double() * y.double()).sum().item(), (x.double() * py.double()).sum().item()
+    assert a > 0 and abs(a - b) <= 1e-5 * a
