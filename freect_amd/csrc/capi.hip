@@ -172,27 +172,44 @@ void free_plan_buffers(fct_wfbp_gpu_plan* p) {
   if (p->h_ratio) (void)hipHostFree(p->h_ratio);
 }
 
-// Views a slab of tz slices can select: table z within one feed of the
-// slab's slices (a superset of the view window), with a margin of views.
+// Views a slab of tz slices can select, with a margin of views: table z within
+// one feed of the slab's slices (a superset of the view window) and within
+// the cone's reach of them.  |q| <= 1 is |z - zt + kb| <= lt with lt = (sqrt(R^2
+// - p^2) - f) tan(cone / 2) <= (R + r) tan(cone / 2) and |kb| <= |kappa| asin(r /
+// R) for a voxel at radius r.  At pitches above about 0.8 the cone is the
+// nearer bound: fewer views to upload, rebin and look at (a scan streamed from
+// host memory, 3.5 rotations of 64 rows at pitch 0.984 for 60 mm: 28.0 -> 26.8
+// ms; six FP16 jobs 34.4 -> 33.9 ms, on one box).
 // False if one slab's views exceed the 4 GiB a buffer resource addresses;
 // *pairs_fit whether they also fit as FP32 row pairs.
 bool slab_view_ranges(const fct_wfbp_gpu_plan* p, const std::vector<double>& zn, int tz,
                       std::vector<int2>* out, bool* pairs_fit) {
   *pairs_fit = true;
   const fct_scan_geometry& s = p->scan;
+  const double half = 0.5 * p->recon.recon_fov;
+  const double r = std::min({std::hypot(std::fabs(p->recon.x_origin) + half,
+                                        std::fabs(p->recon.y_origin) + half),
+                             std::sqrt((double)p->g.half_fov_sq) * 1.0001, s.r});
+  const double cone = ((s.r + r) * (double)p->g.tanc +
+                       std::fabs((double)p->g.kappa) * std::asin(r / s.r)) * 1.0001 +
+                      std::fabs(p->dz);
   const int nslabs = (p->n_native + tz - 1) / tz;
   std::vector<int2>& vr = *out;
   vr.assign(nslabs, make_int2(0, 0));
   for (int sl = 0; sl < nslabs; ++sl) {
     const int a0 = sl * tz, a1 = std::min(p->n_native, a0 + tz) - 1;
-    const double zlo = std::min(zn[a0], zn[a1]) - std::fabs(s.feed);
-    const double zhi = std::max(zn[a0], zn[a1]) + std::fabs(s.feed);
-    double va = (zlo - s.z0) / p->dz, vb = (zhi - s.z0) / p->dz;
-    if (va > vb) std::swap(va, vb);
-    const double lo = std::floor(va) - 2, hi = std::ceil(vb) + 3;
-    vr[sl].x = (int)std::max(0.0, std::min(lo, (double)p->nviews));
-    vr[sl].y = (int)std::max(0.0, std::min(hi, (double)p->nviews));
-    const size_t entries = (size_t)(vr[sl].y - vr[sl].x) * p->nrows * p->cpitch;
+    auto within = [&](double span) {
+      double va = (std::min(zn[a0], zn[a1]) - span - s.z0) / p->dz;
+      double vb = (std::max(zn[a0], zn[a1]) + span - s.z0) / p->dz;
+      if (va > vb) std::swap(va, vb);
+      const double lo = std::floor(va) - 2, hi = std::ceil(vb) + 3;
+      return make_int2((int)std::max(0.0, std::min(lo, (double)p->nviews)),
+                       (int)std::max(0.0, std::min(hi, (double)p->nviews)));
+    };
+    vr[sl] = within(std::min(std::fabs(s.feed), cone));
+    // (The limit is stated for the views within a feed.)
+    const int2 most = within(std::fabs(s.feed));
+    const size_t entries = (size_t)(most.y - most.x) * p->nrows * p->cpitch;
     if (entries * p->filtered_entry_bytes() >= ((size_t)1 << 32)) return false;
     if (entries * sizeof(float2) >= ((size_t)1 << 32)) *pairs_fit = false;
   }
