@@ -652,13 +652,14 @@ __device__ __forceinline__ int bp_launch_tile(const BpArgs& a) {
   return lin < a.xcd_first[x + 1] ? lin : -1;
 }
 
-// Occupancy floor for the 16-bit kernels at TZ <= 8: at least seven waves
-// per SIMD (the few spills this costs sit in the per-theta~ setup, outside
-// the sample loop).  At TZ = 16 five (96 VGPRs; the allocator's own choice
-// is 97, one over); a floor of six spills inside the view loop.
+// Occupancy floor at TZ <= 8: at least seven waves per SIMD (72 VGPRs; only
+// the persistent FP32 kernel spills, five in the per-theta~ set-up; eight
+// spill in every kernel but BF16).  At TZ = 16 five: left to itself the
+// allocator takes 97 VGPRs for FP16 and 114 for FP32 row pairs, whose chain
+// of 500 x 381 x 88 then takes 20.6 instead of 16.0 ms.
 template <int TZ, int PREC>
 constexpr int bp_min_waves() {
-  return TZ <= 8 ? 7 : TZ == 16 && (PREC == FCT_PRECISION_FP16 || PREC == FCT_PRECISION_BF16) ? 5 : 1;
+  return TZ <= 8 ? 7 : TZ == 16 ? 5 : 1;
 }
 
 template <int TZ, int PREC, int MODE, bool CENTERED>
