@@ -35,7 +35,8 @@
 //     own vector offset: the texture-address unit takes 16.7 cycles per
 //     64-lane gather of 8 bytes and 20.3 of 16, so the pairs took the FP32
 //     chain of 500 x 381 x 88 voxels from 17.2 to 12.8 ms and of 256 x 256 x 64
-//     from 3.84 to 3.19, bitwise the same volumes; FP16 / BF16 projections are stored as 2 x 2 quads, one 8-byte
+//     from 3.84 to 3.19, bitwise the same volumes; 16-bit row pairs (whole
+//     chains) are one 8-byte load; FP16 / BF16 projections are stored as 2 x 2 quads, one 8-byte
 //     load per sample, and scaled once per scan at the end; FP16 quads are
 //     interpolated across channels by two v_dot2_f32_f16 with the channel
 //     weights packed as FP16 (exact products, FP32 sums); lanes that select
@@ -226,6 +227,54 @@ struct ChanInterp<FCT_PRECISION_BF16> {   // quad entries: one 8-byte load
   }
 };
 
+// 16-bit row pairs: the 8 bytes of entries (iq, pf) and (iq, pf + 1) hold the
+// quad's halves in another order (FP16 puts them back for the dot products,
+// two instructions per sample).  The gathers cost the same, the lines they
+// touch are half as many: 512 x 512 x 320 FP16 46.1 -> 45.5 ms, flying focal
+// spot 10.95 -> 10.45, 256 x 256 x 64 BF16 4.28 -> 4.05 (whole chains, bitwise
+// the same volumes; six FP16 jobs in one launch 33.0 both).
+template <>
+struct ChanInterp<kPrecisionPairsF16> : ChanInterp<FCT_PRECISION_FP16> {
+  static constexpr uint32_t kEntry = 4;
+  __device__ void init(uint32_t pf, float wp) {
+    ChanInterp<FCT_PRECISION_FP16>::init(pf, wp);
+    base = pf * kEntry;
+  }
+  __device__ static Raw quad(const Raw& t) {
+    const uint32_t x = t.x, y = t.y;
+    return Raw{__builtin_amdgcn_perm(y, x, 0x05040100u), __builtin_amdgcn_perm(y, x, 0x07060302u)};
+  }
+  __device__ float value(const Raw& t, float fq) const {
+    return ChanInterp<FCT_PRECISION_FP16>::value(quad(t), fq);
+  }
+  __device__ void accumulate4(const Raw* t, const float* fq, const float* W, float* num,
+                              float* den) const {
+    const Raw q[4] = {quad(t[0]), quad(t[1]), quad(t[2]), quad(t[3])};
+    ChanInterp<FCT_PRECISION_FP16>::accumulate4(q, fq, W, num, den);
+  }
+};
+
+template <>
+struct ChanInterp<kPrecisionPairsB16> : ChanInterp<FCT_PRECISION_BF16> {
+  static constexpr uint32_t kEntry = 4;
+  __device__ void init(uint32_t pf, float w) {
+    wp = w;
+    base = pf * kEntry;
+  }
+  __device__ float value(const Raw& t, float fq) const {
+    const uint32_t q0 = t.x, q1 = t.y;
+    const float a0 = __uint_as_float(q0 << 16), b0 = __uint_as_float(q0 & 0xFFFF0000u);
+    const float a1 = __uint_as_float(q1 << 16), b1 = __uint_as_float(q1 & 0xFFFF0000u);
+    const float r0 = fmaf(wp, a1 - a0, a0), r1 = fmaf(wp, b1 - b0, b0);
+    return fmaf(fq, r1 - r0, r0);
+  }
+};
+
+template <int PREC>
+constexpr bool kF16 = PREC == FCT_PRECISION_FP16 || PREC == kPrecisionPairsF16;
+template <int PREC>
+constexpr bool kRowPairs = PREC >= kPrecisionPairs;   // (whole chains and the matched sum only)
+
 // Per (voxel column, theta~): p, sqrt(R^2 - p^2), the in-plane offset f and
 // the cone-angle z term kb (fct_bp_column for the views of both parities,
 // which share p, sqrt and asin).
@@ -354,7 +403,7 @@ template <int PREC, int MODE, bool FREE = false>
 __device__ __forceinline__ void bp_add4(const BpTap<PREC>* s, const ChanInterp<PREC>& ci,
                                         float fR, const FctBpConsts& g, float* num, float* den,
                                         int* cnt) {
-  if constexpr (PREC == FCT_PRECISION_FP16 && MODE != kBpCount) {
+  if constexpr (kF16<PREC> && MODE != kBpCount) {
     // The weights first: their arithmetic overlaps the tap loads.
     typename ChanInterp<PREC>::Raw t[4];
     float fq[4], W[4];
@@ -550,7 +599,7 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, f
                                                         chan_ok, g);
               // FP16: the four loads are issued before the weight arithmetic
               // that waits for them (the scheduler would sink them otherwise).
-              if (PREC == FCT_PRECISION_FP16) __builtin_amdgcn_sched_barrier(0);
+              if (kF16<PREC>) __builtin_amdgcn_sched_barrier(0);
               bp_add4<PREC, MODE, kFree>(tap, ci, fR, g, num + h, den + h, cnt + h);
             }
           }
@@ -568,7 +617,7 @@ __device__ __forceinline__ void bp_v1_tile(const BpArgs& a, int lin, int wave, f
             }
             float row0;
             view(l, ztv, &row0);
-            if constexpr (PREC == FCT_PRECISION_FP16) {
+            if constexpr (kF16<PREC>) {
               // Part of the slab, FP16: groups of four slices that meet
               // [ilo, ihi] through the dot block, the slices outside the range
               // masked like unselected samples (cheaper than per-slice samples
@@ -744,10 +793,10 @@ hipError_t launch3(const BpArgs& a, int mode, hipStream_t s) {
   }
   if (mode == kBpAccumulate)
     hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks), dim3(64), 0, s, a);
-  else if (mode == kBpCount && PREC != kPrecisionPairs)
-    hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpCount, C>), dim3(blocks), dim3(64), 0, s, a);
+  else if (mode == kBpCount && !kRowPairs<PREC>)
+    hipLaunchKernelGGL((bp_v1_kernel<TZ, kRowPairs<PREC> ? FCT_PRECISION_FP32 : PREC, kBpCount, C>), dim3(blocks), dim3(64), 0, s, a);
   else if (mode == kBpMatched && (PREC == FCT_PRECISION_FP32 || PREC == kPrecisionPairs))
-    hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((bp_v1_kernel<TZ, PREC == kPrecisionPairs ? kPrecisionPairs : FCT_PRECISION_FP32, kBpMatched, C>), dim3(blocks), dim3(64), 0, s, a);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
@@ -766,6 +815,8 @@ hipError_t launch1(const BpArgs& a, int precision, int mode, hipStream_t s) {
     case FCT_PRECISION_FP16: return launch2<TZ, FCT_PRECISION_FP16>(a, mode, s);
     case FCT_PRECISION_BF16: return launch2<TZ, FCT_PRECISION_BF16>(a, mode, s);
     case kPrecisionPairs: return launch2<TZ, kPrecisionPairs>(a, mode, s);
+    case kPrecisionPairsF16: return launch2<TZ, kPrecisionPairsF16>(a, mode, s);
+    case kPrecisionPairsB16: return launch2<TZ, kPrecisionPairsB16>(a, mode, s);
   }
   return hipErrorInvalidValue;
 }
@@ -789,6 +840,8 @@ hipError_t launch_batch1(const BpBatchArgs& b, int precision, bool centered, int
     case FCT_PRECISION_FP16: return launch_batch2<TZ, FCT_PRECISION_FP16>(b, centered, grid, s);
     case FCT_PRECISION_BF16: return launch_batch2<TZ, FCT_PRECISION_BF16>(b, centered, grid, s);
     case kPrecisionPairs: return launch_batch2<TZ, kPrecisionPairs>(b, centered, grid, s);
+    case kPrecisionPairsF16: return launch_batch2<TZ, kPrecisionPairsF16>(b, centered, grid, s);
+    case kPrecisionPairsB16: return launch_batch2<TZ, kPrecisionPairsB16>(b, centered, grid, s);
   }
   return hipErrorInvalidValue;
 }
@@ -811,16 +864,18 @@ hipError_t backproject_batch_waves_per_cu(int tile_z, int precision, int* waves)
   // Occupancy of the FP32 / FP16 / BF16 instantiations (the centred and
   // general forms use the same registers to within a few).
   const void* f = nullptr;
-#define FCT_BATCH_K(TZ)                                                             \
-  case TZ:                                                                          \
-    f = precision == FCT_PRECISION_FP32                                             \
-            ? (const void*)bp_batch_kernel<TZ, FCT_PRECISION_FP32, false>           \
-            : precision == FCT_PRECISION_FP16                                       \
-                  ? (const void*)bp_batch_kernel<TZ, FCT_PRECISION_FP16, false>     \
-                  : precision == FCT_PRECISION_BF16                                 \
-                        ? (const void*)bp_batch_kernel<TZ, FCT_PRECISION_BF16, false> \
-                        : (const void*)bp_batch_kernel<TZ, kPrecisionPairs, false>; \
-    break;
+#define FCT_BATCH_K(TZ)                                                                       \
+  case TZ: {                                                                                  \
+    const void* k[] = {(const void*)bp_batch_kernel<TZ, FCT_PRECISION_FP32, false>,           \
+                       (const void*)bp_batch_kernel<TZ, FCT_PRECISION_FP16, false>,           \
+                       (const void*)bp_batch_kernel<TZ, FCT_PRECISION_BF16, false>,           \
+                       (const void*)bp_batch_kernel<TZ, kPrecisionPairs, false>,              \
+                       (const void*)bp_batch_kernel<TZ, kPrecisionPairsF16, false>,           \
+                       (const void*)bp_batch_kernel<TZ, kPrecisionPairsB16, false>};          \
+    if (precision < 0 || precision > kPrecisionPairsB16) return hipErrorInvalidValue;         \
+    f = k[precision];                                                                         \
+    break;                                                                                    \
+  }
   switch (tile_z) {
     FCT_BATCH_K(4)
     FCT_BATCH_K(8)

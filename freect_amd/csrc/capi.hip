@@ -623,7 +623,7 @@ int chain_backproject(fct_wfbp_gpu_plan* p, const void* filtered, const float* s
   a.native = native;
   HIP_TRY(p->ctx,
           fct::launch_backproject(a, p->tile_z, p->variant,
-                                  pairs ? kPrecisionPairs : p->opts.precision,
+                                  pairs ? pair_storage(p->opts.precision) : p->opts.precision,
                                   fct::kBpAccumulate, p->stream));
   return FCT_OK;
 }
@@ -901,8 +901,9 @@ int reconstruct_streaming(fct_wfbp_gpu_plan* p, const ViewSource& src, int vpc,
         if (e == hipSuccess && j_done > par.x)
           e = fct::launch_quad_rescale(
               static_cast<char*>(p->d_filtered) +
-                  (size_t)par.x * entries_per_view * p->filtered_entry_bytes(),
-              (size_t)(j_done - par.x) * entries_per_view, prec, p->d_scale, p->ncu, p->stream);
+                  (size_t)par.x * entries_per_view * p->storage_entry_bytes(),
+              (size_t)(j_done - par.x) * entries_per_view * p->storage_entry_bytes() / 8, prec,
+              p->d_scale, p->ncu, p->stream);   // (a row holds a multiple of 64 entries)
       }
       if (e == hipSuccess && (grew || !committed)) {
         e = fct::launch_scale_commit(p->d_scale, p->stream);
@@ -1123,8 +1124,9 @@ FCT_API int fct_wfbp_gpu_plan_create(fct_wfbp_gpu_ctx* ctx, const fct_scan_geome
   // FP32 whole chains keep row pairs where they fit for every tile depth (a
   // batch may still change it).
   std::vector<int2> vr32;
-  p->pairs = p->opts.precision == FCT_PRECISION_FP32 && p->variant == FCT_BP_LEAN &&
-             slab_view_ranges(p, zn, 32, &vr32, &pairs_fit) && pairs_fit;
+  p->pairs = p->variant == FCT_BP_LEAN &&
+             (p->opts.precision != FCT_PRECISION_FP32 ||
+              (slab_view_ranges(p, zn, 32, &vr32, &pairs_fit) && pairs_fit));
 
   // Exact view-window slice ranges per (chunk, view): the slices s of the
   // chunk with fct_bp_in_window(zt, zs) true form one interval (the test is
@@ -1607,7 +1609,8 @@ FCT_API int fct_wfbp_gpu_matched_backproject(fct_wfbp_gpu_plan* p, const float* 
   // views x 16 x 736, 256 x 256 x 32: 2.09 -> 1.61 ms and
   // 0.05 for the pass).
   const size_t lines_n = (size_t)p->nviews * p->nrows * p->cpitch;
-  if (p->pairs && (double)p->n_native * p->recon.ny * p->recon.nx * 2.0 * p->H >
+  if (p->pairs && p->opts.precision == FCT_PRECISION_FP32 &&
+      (double)p->n_native * p->recon.ny * p->recon.nx * 2.0 * p->H >
                       16.0 * (double)lines_n) {
     if (!p->d_filtered) p->d_filtered = try_scratch(p, p->storage_bytes());
     if (p->d_filtered) {

@@ -416,6 +416,42 @@ __device__ __forceinline__ void pair_store2(const RebinFilterArgs& a, size_t e, 
   if (r > 0) st_nt(q + 2 * (e - (size_t)a.cpitch) + 1, lo);
 }
 
+// The same in 16 bits.
+template <class T>
+__device__ __forceinline__ void pair_store16(const RebinFilterArgs& a, size_t e, int r, float y) {
+  uint16_t* q = static_cast<uint16_t*>(a.out);
+  const uint16_t h = __builtin_bit_cast(uint16_t, to_store<T>(y));
+  __builtin_nontemporal_store(h, q + 2 * e);
+  if (r > 0) __builtin_nontemporal_store(h, q + 2 * (e - (size_t)a.cpitch) + 1);
+  if (r == a.nrows - 1) __builtin_nontemporal_store((uint16_t)0, q + 2 * e + 1);
+}
+
+template <class T>
+__device__ __forceinline__ void pair_store16x2(const RebinFilterArgs& a, size_t e, int r, float y0,
+                                               float y1) {
+  uint32_t* q = static_cast<uint32_t*>(a.out);
+  uint16_t* h = static_cast<uint16_t*>(a.out);
+  const uint32_t v = pack2<T>(y0, y1);
+  const size_t e1 = e + (size_t)a.cpitch;
+  st_nt(q + e, v);
+  if (r + 1 == a.nrows - 1)
+    st_nt(q + e1, v >> 16);
+  else
+    __builtin_nontemporal_store((uint16_t)(v >> 16), h + 2 * e1);
+  if (r > 0) __builtin_nontemporal_store((uint16_t)v, h + 2 * (e - (size_t)a.cpitch) + 1);
+}
+
+template <class T>
+__device__ __forceinline__ void pair_lines16(const RebinFilterArgs& a, size_t e0, size_t e1, int r0,
+                                             int r1, bool has1, bool same, float y0, float y1) {
+  if (same) {
+    pair_store16x2<T>(a, e0, r0, y0, y1);
+  } else {
+    pair_store16<T>(a, e0, r0, y0);
+    if (has1) pair_store16<T>(a, e1, r1, y1);
+  }
+}
+
 // max|x| over the raw scan as FP32 bits in scale[1] (non-negative floats
 // order like their bit patterns).
 __global__ void scale_reset_kernel(float* scale) {
@@ -527,7 +563,11 @@ __global__ __launch_bounds__(kRfThreads) void rebin_filter_kernel(RebinFilterArg
   for (int c = threadIdx.x; c < a.cpitch; c += kRfThreads) {
     const bool in = c < a.ncols;
     const float y0 = in ? Y[c].x * is : 0.0f, y1 = in ? -Y[c].y * is : 0.0f;
-    if (a.precision == FCT_PRECISION_FP16)
+    if (a.pairs && a.precision == FCT_PRECISION_FP16)
+      pair_lines16<__half>(a, o0 + c, o1 + c, r0, r1, has1, false, y0, y1);
+    else if (a.pairs)
+      pair_lines16<__hip_bfloat16>(a, o0 + c, o1 + c, r0, r1, has1, false, y0, y1);
+    else if (a.precision == FCT_PRECISION_FP16)
       quad_store_lines<__half>(a, o0, o1, r0, r1, has1, c, y0, y1);
     else
       quad_store_lines<__hip_bfloat16>(a, o0, o1, r0, r1, has1, c, y0, y1);
@@ -730,6 +770,19 @@ void rebin_filter_reg_kernel(RebinFilterArgs a) {
       const bool in = t + m * T < a.ncols;
       ya[m] = in ? y.x * is : 0.0f;
       yb[m] = in ? -y.y * is : 0.0f;
+    }
+    if (a.pairs) {
+      const bool same = has1 && (r0 & 1) == 0 && r1 == r0 + 1;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int c = t + m * T;
+        if (c >= a.cpitch) continue;
+        if (a.precision == FCT_PRECISION_FP16)
+          pair_lines16<__half>(a, o0 + c, o1 + c, r0, r1, has1, same, ya[m], yb[m]);
+        else
+          pair_lines16<__hip_bfloat16>(a, o0 + c, o1 + c, r0, r1, has1, same, ya[m], yb[m]);
+      }
+      continue;
     }
     if (has1 && (r0 & 1) == 0 && r1 == r0 + 1) {
       // Rows r0 (even) and r0 + 1 of one view: the 2 x 2 quads of row r0 are

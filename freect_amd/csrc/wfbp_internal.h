@@ -79,7 +79,7 @@ struct RebinFilterArgs {
   // x raw rows x raw channels), and the smallest aoff and mmax of the table.
   uint32_t group_bytes;
   int32_t aoff_min, mmax_min;
-  int32_t pairs;             // 1: FP32 output as row pairs (kPrecisionPairs)
+  int32_t pairs;             // 1: output as row pairs (kPrecisionPairs and its 16-bit forms)
 };
 
 // FP32 projections stored as row pairs, the layout between the rebinning and
@@ -90,7 +90,16 @@ struct RebinFilterArgs {
 // texture-address unit takes 16.7 cycles per 64-lane gather of 8 bytes and
 // 20.3 of 16 (measured, taps of an 8 x 8 tile in L1): 86 % of the kernel's
 // time.  The stage calls keep the row layout of their interface.
-constexpr int kPrecisionPairs = 3;
+//
+// FP16 / BF16 chains keep the same pairs in 16 bits (4 bytes per entry, the
+// scan's scale as for the quads): the taps are 8 consecutive bytes as with
+// the quads of the interface, in half the lines.
+constexpr int kPrecisionPairs = 3, kPrecisionPairsF16 = 4, kPrecisionPairsB16 = 5;
+inline int pair_storage(int precision) {
+  return precision == FCT_PRECISION_FP32   ? kPrecisionPairs
+         : precision == FCT_PRECISION_FP16 ? kPrecisionPairsF16
+                                           : kPrecisionPairsB16;
+}
 
 // Everything the backprojection kernel reads.
 struct BpArgs {
@@ -397,7 +406,7 @@ struct fct_wfbp_gpu_plan {
   float* d_thk_w = nullptr;
 
   // Intermediate buffers for fct_wfbp_gpu_reconstruct (allocated on first use).
-  bool pairs = false;               // d_filtered holds FP32 row pairs (kPrecisionPairs)
+  bool pairs = false;               // d_filtered holds row pairs (kPrecisionPairs)
   void* d_filtered = nullptr;
   float* d_scale = nullptr;
   float* d_native = nullptr;
@@ -445,8 +454,13 @@ struct fct_wfbp_gpu_plan {
     return (size_t)nviews * nrows * cpitch * filtered_entry_bytes();
   }
   // The plan's own buffer between the stages of a whole chain.
-  int storage() const { return pairs ? fct::kPrecisionPairs : opts.precision; }
-  size_t storage_bytes() const { return filtered_bytes() * (pairs ? 2 : 1); }
+  int storage() const { return pairs ? fct::pair_storage(opts.precision) : opts.precision; }
+  size_t storage_entry_bytes() const {
+    return pairs ? (opts.precision == FCT_PRECISION_FP32 ? 8 : 4) : filtered_entry_bytes();
+  }
+  size_t storage_bytes() const {
+    return (size_t)nviews * nrows * cpitch * storage_entry_bytes();
+  }
   size_t scale_elems() const {
     return opts.precision == FCT_PRECISION_FP32 ? 0 : (size_t)fct::kScaleElems;
   }

@@ -1,9 +1,9 @@
 """The lean backprojection's choice of a theta~'s views (a ballot over 64 of
 them at a time, whole slabs first, the exact window table only near the
-window's ends) and the row pairs of FP32 whole chains: feeds so small that a slab
+window's ends) and the row pairs of whole chains: feeds so small that a slab
 has more than 64 views per theta~, view windows that cut into the slabs, a table
 that moves down, odd row counts, every tile depth, against the direct kernel,
-which tests each (voxel, view) pair on plain rows.  Both add the same FP32 terms (the lean
+which tests each (voxel, view) pair on plain rows or quads.  Both add the same FP32 terms (the lean
 kernel's mean through v_rcp_f32, 1 ulp), in another order of a theta~'s views:
 sums over at most a few hundred theta~ differ by rounding, 2e-5 of the largest
 voxel.
@@ -33,7 +33,9 @@ def ctx():
                           (11, 9.0, 64, 4.0, 20, True, 96, "fp32"),
                           (11, 9.0, 64, 4.0, 20, False, 300, "fp32"),
                           (12, 9.0, 64, 4.0, 20, False, 257, "fp32"),
-                          (11, 9.0, 64, 4.0, 20, False, 96, "fp16")])
+                          (11, 9.0, 64, 4.0, 20, False, 96, "fp16"),
+                          (11, 9.0, 64, 4.0, 20, False, 300, "bf16"),
+                          (12, 9.0, 64, 4.0, 20, True, 257, "fp16")])
 def test_view_choice_against_direct(ctx, tile_z, rows, feed_rows, ppr, rotations, slices, down,
                                     channels, precision):
     from freect_amd import wfbp
