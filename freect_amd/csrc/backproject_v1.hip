@@ -36,13 +36,12 @@
 //     64-lane gather of 8 bytes and 20.3 of 16, so the pairs took the FP32
 //     chain of 500 x 381 x 88 voxels from 17.2 to 12.8 ms and of 256 x 256 x 64
 //     from 3.84 to 3.19, bitwise the same volumes; 16-bit row pairs (whole
-//     chains) are one 8-byte load; FP16 / BF16 projections are stored as 2 x 2 quads, one 8-byte
-//     load per sample, and scaled once per scan at the end; FP16 quads are
-//     interpolated across channels by two v_dot2_f32_f16 with the channel
-//     weights packed as FP16 (exact products, FP32 sums); lanes that select
-//     nothing read whatever the range-checked buffer returns (filtered
-//     values of the slab, or 0 outside it) and get weight 0 instead of a
-//     branch;
+//     chains) and 2 x 2 quads (stage calls) are one 8-byte load, and are
+//     scaled once per scan at the end; FP16 is interpolated across channels
+//     by two v_dot2_f32_f16 with the channel weights packed as FP16 (exact
+//     products, FP32 sums); lanes that select nothing read whatever the
+//     range-checked buffer returns (filtered values of the slab, or 0
+//     outside it) and get weight 0 instead of a branch;
 //   * the per-theta~ mean uses v_rcp.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>

@@ -628,8 +628,13 @@ __device__ __forceinline__ void fft_forward_regs(FctCplx* v, FctCplx* lds, int t
   }
 }
 
+// Three waves per SIMD (162 VGPRs; 128 spill and are slower at N <= 2048, 4.96
+// against 3.97 ms for all lines of the full workload).  A block of N = 4096 is
+// eight waves, of which three per SIMD hold only one: there four (128 VGPRs,
+// two blocks per CU, some twiddles spilled) take the rebinning of 1728 x 64 x
+// 1472 samples (phi + z FFS) from 1.9 to 1.4 ms, its chain from 10.34 to 9.85.
 template <int N>
-__global__ __launch_bounds__(N / 8) __attribute__((amdgpu_waves_per_eu(3, 8)))
+__global__ __launch_bounds__(N / 8) __attribute__((amdgpu_waves_per_eu(N == 4096 ? 4 : 3, 8)))
 void rebin_filter_reg_kernel(RebinFilterArgs a) {
   using S = FctFftShape<N>;
   constexpr int T = S::T;

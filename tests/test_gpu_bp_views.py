@@ -35,7 +35,8 @@ def ctx():
                           (12, 9.0, 64, 4.0, 20, False, 257, "fp32"),
                           (11, 9.0, 64, 4.0, 20, False, 96, "fp16"),
                           (11, 9.0, 64, 4.0, 20, False, 300, "bf16"),
-                          (12, 9.0, 64, 4.0, 20, True, 257, "fp16")])
+                          (12, 9.0, 64, 4.0, 20, True, 257, "fp16"),
+                          (12, 9.0, 32, 4.0, 20, True, 1100, "fp16")])
 def test_view_choice_against_direct(ctx, tile_z, rows, feed_rows, ppr, rotations, slices, down,
                                     channels, precision):
     from freect_amd import wfbp
