@@ -158,7 +158,8 @@ void free_plan_buffers(fct_wfbp_gpu_plan* p) {
                   p->d_slab_vrange, p->d_rebin, p->d_rebinT,  p->d_Hn,        p->d_tw,       p->d_thk_off,
                   p->d_thk_idx,  p->d_thk_w,     p->d_filtered,  p->d_scale, p->d_native,
                   p->d_raw_stage, p->d_vol_stage, p->d_gbar, p->d_thkT_off, p->d_thkT_idx,
-                  p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_ray_tab, p->d_ray_pad, p->d_ray_rec, p->d_adj_wgt, p->d_af_raw, p->d_af_vmax};
+                  p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_ray_tab, p->d_ray_pad, p->d_ray_rec,
+                  p->d_adj_scratch[0], p->d_adj_scratch[1], p->d_af_raw, p->d_af_vmax};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (int b = 0; b < 2; ++b)
@@ -412,21 +413,19 @@ bool adjoint_gather(fct_wfbp_gpu_plan* p, const fct::BpAdjArgs& a, bool matched,
   const size_t per = 4 * cols + (matched ? 0 : vol);
   size_t nt = std::min<size_t>(p->H, (4096 + waves - 1) / waves);
   nt = std::max<size_t>(1, std::min<size_t>(nt, ((size_t)2 << 30) / (per * sizeof(float))));
-  const size_t need = nt * per + (matched ? vol : 0);
+  const size_t need = nt * per + (matched ? vol : 0);   // the plan's alone: the same at every call
   const double lines = (double)((p->recon.nx + 63) / 64) * p->recon.ny +
                        (double)((p->recon.ny + 63) / 64) * p->recon.nx;
   if ((double)waves * p->H * 16 >= 2147483647.0 || lines * p->n_native >= 2147483647.0) return false;
-  if (p->adj_wgt_elems < need) {
-    float* d = static_cast<float*>(try_scratch(p, need * sizeof(float)));
-    if (!d) return false;
-    if (p->d_adj_wgt) (void)hipFree(p->d_adj_wgt);   // (waits for the work that reads it)
-    p->d_adj_wgt = d;
-    p->adj_wgt_elems = need;
-  }
+  // One buffer for each of the two uses, kept until the plan is destroyed and
+  // never exchanged for a larger one: a captured graph holds its address.
+  float*& scratch = p->d_adj_scratch[matched];
+  if (!scratch) scratch = static_cast<float*>(try_scratch(p, need * sizeof(float)));
+  if (!scratch) return false;
   const fct::RayProjArgs r = ray_args(p);
   fct::AdjGather q{};
-  q.col = reinterpret_cast<float4*>(p->d_adj_wgt);
-  q.wgt = p->d_adj_wgt + nt * 4 * cols;
+  q.col = reinterpret_cast<float4*>(scratch);
+  q.wgt = scratch + nt * 4 * cols;
   q.tile_z = p->tile_z;
   q.gx0 = r.dx0;
   q.gdx = r.ddx;

@@ -417,8 +417,9 @@ struct fct_wfbp_gpu_plan {
   float* d_ray_pad = nullptr;       // padded volume copies of the ray projector (first use)
   bool ray_pad_pairs = false;       // with two slices per entry
   float* d_ray_rec = nullptr;       // per-ray records of its transpose (first use)
-  float* d_adj_wgt = nullptr;       // gathered transpose: voxel weights / swapped volume (first use)
-  size_t adj_wgt_elems = 0;
+  // Gathered transposes (first use of each): columns and voxel weights of the
+  // backprojection's, columns and swapped volume of the matched projector's.
+  float* d_adj_scratch[2] = {nullptr, nullptr};
   std::vector<uint8_t> h_xplanes;   // per theta~: its parallel rays run along x planes
   float* d_gbar = nullptr;          // adjoint scratch, [view][row][cpitch] FP32
   int32_t* d_thkT_off = nullptr;    // transposed thickening table
