@@ -358,14 +358,19 @@ __global__ __launch_bounds__(64 * kRayRows) void ray_project_table_kernel(RayPro
 
 // Per ray of the transpose: its in-plane sample positions (fq = A + i B, the
 // general kernels' FP32 values) and its value times the path length per plane.
-__global__ __launch_bounds__(256) void ray_record_kernel(RayProjArgs a, float* __restrict__ rec) {
+// The planes are those of the table, which the projector and the gather read
+// too: decided once more here, from the ray with its row's slope, the axis of
+// a ray within an FP32 rounding of the diagonal could differ from theirs, and
+// the gather lost the ray.
+__global__ __launch_bounds__(256) void ray_record_kernel(RayProjArgs a, RayTables t,
+                                                         float* __restrict__ rec) {
   const int cg = (a.ncols + 255) >> 8;
   const int v = blockIdx.x / cg, c = (blockIdx.x - v * cg) * 256 + threadIdx.x;
   if (c >= a.ncols) return;
   const RayDir d = ray_dir(a, v, c);
+  const bool xmajor = __float_as_int(t.ray[(size_t)v * a.ncols + c].w) & 1;
   for (int row = 0; row < a.nrows; ++row) {
     const Ray r = ray_of(a, d, row);
-    const bool xmajor = fabsf(r.ux) >= fabsf(r.uy);
     const float p0 = xmajor ? a.gx0 : a.gy0, dp = xmajor ? a.gdx : a.gdy;
     const float q0 = xmajor ? a.gy0 : a.gx0, dq = xmajor ? a.gdy : a.gdx;
     const float sp = xmajor ? r.sx : r.sy, sq = xmajor ? r.sy : r.sx;
@@ -635,7 +640,7 @@ hipError_t launch_ray_gather(const RayProjArgs& a, const RayTables& t, float* re
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(ray_record_kernel, dim3(a.v1 * ((a.ncols + 255) / 256)), dim3(256), 0, s, a,
-                     rec);
+                     t, rec);
   const dim3 grid((unsigned)(waves * q.nsplit));
   const bool ffs = a.states > 1;
   if (K == 16 && ffs)

@@ -117,3 +117,42 @@ def test_volume_beyond_the_paired_copies(ctx):
     big.synchronize()
     assert a.abs().max() > 0
     assert (a - b).abs().max() <= 2e-4 * a.abs().max()
+
+
+def test_rays_on_the_diagonal(ctx):
+    # Rays within an FP32 rounding of 45 degrees, of which the in-plane
+    # direction and the direction with the row's slope round to different plane
+    # axes: the projector and its transpose take the same one.  One ray at a
+    # time, <P x, e> = <x, P^T e> with positive x: sums of at most 4 x 40 FP32
+    # terms each way, 1e-5 of the product.
+    import math
+
+    from freect_amd import wfbp
+    w = S.tiny(nx=40, n_slices=20, n_rows=16, rotations=0.1)
+    sc, chan = w.scan, 30
+    beta = (chan - sc.central_channel) * sc.channel_spacing / sc.dsd
+    height = (np.arange(sc.n_rows) - sc.central_row) * sc.row_spacing
+
+    def x_planes(scan, length):
+        d = scan.dsd * np.array([math.cos(scan.angle0 + beta), math.sin(scan.angle0 + beta)])
+        u = np.abs((d[:, None] / length).astype(np.float32))
+        return u[0] >= u[1]
+
+    tried = 0
+    for off in np.linspace(-6e-8, 6e-8, 13):
+        scan = sc.replace(angle0=1.25 * math.pi - beta + float(off))
+        rows = np.flatnonzero(x_planes(scan, scan.dsd) != x_planes(scan, np.hypot(scan.dsd, height)))
+        if rows.size == 0:
+            continue
+        p = wfbp.Plan(ctx, scan, w.recon)
+        x = torch.rand(p.alloc_native().shape, device="cuda") + 0.1
+        px, e, xt = p.alloc_raw(), p.alloc_raw().zero_(), p.alloc_native()
+        p.ray_project(x, px)
+        for row in rows[[0, -1]]:
+            e.zero_()[0, row, chan] = 1.0
+            p.ray_backproject(e, xt)
+            p.synchronize()
+            a, b = px[0, row, chan].item(), (x.double() * xt.double()).sum().item()
+            assert a > 1.0 and abs(a - b) <= 1e-5 * a, (off, row, a, b)
+            tried += 1
+    assert tried > 0
