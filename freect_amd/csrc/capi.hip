@@ -578,11 +578,18 @@ void needed_views(const fct_wfbp_gpu_plan* p, int2* par, int2* raw) {
 namespace fct {
 
 // Rebin + filter of the whole chain: the lines some slab reads only, the
-// FP16 / BF16 bound from the raw views they read (the stage call
-// fct_wfbp_gpu_rebin_filter filters every line of the scan).
-int chain_lines(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale, bool pairs) {
+// adaptive filtration and the FP16 / BF16 bound over the raw views they read
+// (the stage call fct_wfbp_gpu_rebin_filter filters every line of the scan).
+int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale,
+                       bool pairs) {
   int2 par, rawr;
   needed_views(p, &par, &rawr);
+  if (p->af_on) {   // into the plan's buffer
+    HIP_TRY(p->ctx, fct::launch_adaptive_filter(raw, p->d_af_raw, p->d_af_vmax, rawr.x, rawr.y,
+                                                p->raw_scan.n_rows, p->raw_scan.n_channels,
+                                                p->af_s, p->stream));
+    raw = p->d_af_raw;
+  }
   const size_t per_view = (size_t)p->raw_scan.n_rows * p->raw_scan.n_channels;
   fct::RebinFilterArgs a = rf_args(p, raw, filtered, scale);
   if (p->opts.precision != FCT_PRECISION_FP32) {
@@ -599,19 +606,6 @@ int chain_lines(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* s
   a.pairs = pairs;
   HIP_TRY(p->ctx, fct::launch_rebin_filter(a, p->stream));
   return FCT_OK;
-}
-
-int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale,
-                       bool pairs) {
-  if (p->af_on) {   // adaptive filtration of the views read, into the plan's buffer
-    int2 par, rawr;
-    needed_views(p, &par, &rawr);
-    HIP_TRY(p->ctx, fct::launch_adaptive_filter(raw, p->d_af_raw, p->d_af_vmax, rawr.x, rawr.y,
-                                                p->raw_scan.n_rows, p->raw_scan.n_channels,
-                                                p->af_s, p->stream));
-    raw = p->d_af_raw;
-  }
-  return chain_lines(p, raw, filtered, scale, pairs);
 }
 
 int chain_backproject(fct_wfbp_gpu_plan* p, const void* filtered, const float* scale,
@@ -1426,7 +1420,7 @@ FCT_API int fct_wfbp_gpu_forward_native(fct_wfbp_gpu_plan* p, const float* raw, 
   HIP_TRY(p->ctx, hipSetDevice(p->device));
   const bool pairs = p->pairs && (size_t)scratch_bytes >= 2 * p->filtered_bytes() &&
                      (reinterpret_cast<uintptr_t>(scratch) & 7) == 0;
-  const int st = fct::chain_lines(p, raw, scratch, nullptr, pairs);
+  const int st = fct::chain_rebin_filter(p, raw, scratch, nullptr, pairs);
   return st ? st : fct::chain_backproject(p, scratch, nullptr, native, pairs);
 }
 

@@ -341,8 +341,6 @@ BpArgs plan_bp_args(const fct_wfbp_gpu_plan* p);   // tables only (no buffers)
 void plan_bp_share(const fct_wfbp_gpu_plan* p, int slab0, int count, BpArgs* a);
 int plan_set_tile_z(fct_wfbp_gpu_plan* p, int tz);  // rebuilds the slab view ranges
 // Rebin + filter of the lines some slab reads (the whole-chain entry points).
-// (Without the adaptive filtration.)
-int chain_lines(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale, bool pairs);
 int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, float* scale,
                        bool pairs);
 // The lean backprojection of filtered projections in the plan's own layout

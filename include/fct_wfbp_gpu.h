@@ -213,8 +213,8 @@ FCT_API int fct_wfbp_gpu_backproject(fct_wfbp_gpu_plan* plan, const void* filter
                                      const float* scale, float* native);
 
 /* Raw scan to native volume (rebinning, filter, backprojection of the lines
- * and views the volume needs; no adaptive filtration), FP32 plans, device
- * buffers.  scratch holds the filtered projections between the stages, at
+ * and views the volume needs; after the adaptive filtration on plans that have
+ * it), FP32 plans, device buffers.  scratch holds the filtered projections between the stages, at
  * least filtered_bytes; with twice that the faster row-pair layout is used
  * where the plan can hold it.  The volume is the same either way. */
 FCT_API int fct_wfbp_gpu_forward_native(fct_wfbp_gpu_plan* plan, const float* raw, void* scratch,

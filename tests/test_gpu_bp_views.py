@@ -99,3 +99,22 @@ def test_matched_backprojection_of_row_pairs(ctx, rows, nx):
     p.synchronize()
     a, b = (px.double() * y.double()).sum().item(), (x.double() * py.double()).sum().item()
     assert a > 0 and abs(a - b) <= 1e-5 * a
+
+
+def test_forward_volume_with_adaptive_filtration(ctx):
+    # On a plan with adaptive filtration the chain to the native volume filters
+    # the raw scan as the stage calls do (the same values from the same views:
+    # bitwise), and so does the forward pass of autograd.wfbp.
+    from freect_amd import autograd, wfbp
+    w = S.tiny(nx=26, n_slices=20, rotations=3.0, seed=5)
+    raw = ctx.phantom_project(w.scan, w.phantom, 1e4, w.seed)
+    recon = w.recon.replace(adaptive_filtration_s=0.3)
+    p = wfbp.Plan(ctx, w.scan, recon, adaptive_filtration=True)
+    plain = wfbp.Plan(ctx, w.scan, recon)
+    ref, vol, other = p.alloc_native(), p.alloc_native().fill_(float("nan")), p.alloc_native()
+    p.forward_native(raw, ref)
+    p.forward_volume(raw, vol)
+    plain.forward_volume(raw, other)
+    torch.cuda.synchronize()
+    assert torch.equal(vol, ref) and not torch.equal(other, ref)
+    assert torch.equal(autograd.wfbp(raw, p), ref)
