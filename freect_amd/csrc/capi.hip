@@ -373,12 +373,21 @@ fct::RayProjArgs ray_args(const fct_wfbp_gpu_plan* p) {
 
 // A plan-owned device buffer allocated on first use; nullptr (and no error
 // left behind) when it does not fit or the plan's stream is being captured
-// into a graph, where the callers take a path without it.
+// into a graph, where the callers take a path without it.  A capture that runs
+// on another stream forbids allocations in its mode and would end invalid: the
+// thread's mode is relaxed meanwhile (the buffer is no part of that graph).
 void* try_scratch(fct_wfbp_gpu_plan* p, size_t bytes) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   void* d = nullptr;
-  if (hipStreamIsCapturing(p->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-      hipMalloc(&d, bytes) != hipSuccess) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool ok = hipStreamIsCapturing(p->stream, &cap) == hipSuccess &&
+            cap == hipStreamCaptureStatusNone &&
+            hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  if (ok) {
+    ok = hipMalloc(&d, bytes) == hipSuccess;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  if (!ok) {
     (void)hipGetLastError();
     return nullptr;
   }

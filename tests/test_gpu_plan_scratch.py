@@ -70,3 +70,35 @@ def test_capture_between_first_uses(ctx, op):
         assert ref.abs().max() > 0
         assert (y - ref).abs().max() <= 1e-5 * ref.abs().max()
     del junk
+
+
+@pytest.mark.parametrize("mode", ["global", "thread_local"])
+@pytest.mark.parametrize("op", OPS)
+def test_first_use_beside_a_capture(ctx, op, mode):
+    # The first call of a plan while another stream is being captured: the
+    # capture stays valid and holds its own work only, and the call gives what
+    # it gives outside (the same kernels; sums of atomics, 1e-5 of the largest).
+    from freect_amd import wfbp
+    w = S.tiny(nx=60, n_slices=19, rotations=2.5)
+    p = wfbp.Plan(ctx, w.scan, w.recon)
+    p.set_stream(torch.cuda.Stream())
+    x, y = _ends(p, op)
+    x.uniform_(0.1, 1.0)
+    ref, a = torch.full_like(y, float("nan")), torch.zeros(64, device="cuda")
+    y.fill_(float("nan"))
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream(), capture_error_mode=mode):
+        a.add_(1.0)
+        getattr(p, op)(x, y)
+    torch.cuda.synchronize()
+    first = y.clone()
+    y.fill_(float("nan"))
+    for _ in range(3):
+        g.replay()
+    torch.cuda.synchronize()
+    assert a.eq(3.0).all() and y.isnan().all()
+    getattr(p, op)(x, ref)
+    p.synchronize()
+    assert ref.abs().max() > 0
+    assert (first - ref).abs().max() <= 1e-5 * ref.abs().max()
