@@ -214,36 +214,17 @@ FCT_API int fct_wfbp_gpu_batch_create(fct_wfbp_gpu_ctx* ctx, int32_t n_jobs,
                                       &b->plans[j]);
     if (st != FCT_OK) return fail(st);
   }
-  // One storage for every job (one kernel runs them all): FP32 row pairs, or
-  // rows where a plan cannot hold those or there is no memory for them.
-  bool pairs = true;
-  for (fct_wfbp_gpu_plan* p : b->plans) pairs = pairs && p->pairs;
-  for (fct_wfbp_gpu_plan* p : b->plans) {
-    p->pairs = pairs;
-    const hipError_t e = fct::plan_alloc_filtered(p);
-    if (e != hipSuccess) return fail(hip_status(ctx, "batch buffers", e));
-    pairs = p->pairs;
-  }
-  for (fct_wfbp_gpu_plan* p : b->plans) {
-    const size_t nat = (size_t)p->n_native * p->recon.ny * p->recon.nx * sizeof(float);
-    hipError_t e = hipSuccess;
-    if (p->pairs && !pairs) {
-      (void)hipFree(p->d_filtered);
-      p->d_filtered = nullptr;
-      p->pairs = false;
-      e = fct::plan_alloc_filtered(p);
-    }
-    if (e == hipSuccess && p->scale_elems())
-      e = hipMalloc(reinterpret_cast<void**>(&p->d_scale), p->scale_elems() * 4);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&p->d_native), nat);
-    if (e != hipSuccess) return fail(hip_status(ctx, "batch buffers", e));
-    b->device_bytes += (int64_t)(p->storage_bytes() + p->scale_elems() * 4 + nat);
-  }
-  hipError_t e = hipMalloc(reinterpret_cast<void**>(&b->d_jobs), n_jobs * sizeof(fct::BpArgs));
-  if (e == hipSuccess)
-    e = hipMalloc(reinterpret_cast<void**>(&b->d_tile_start), (n_jobs + 1) * sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&b->d_queue), 8 * sizeof(uint32_t));
-  if (e != hipSuccess) return fail(hip_status(ctx, "batch tables", e));
+  // One layout of the filtered projections for every job (one kernel runs them
+  // all): row pairs, or the interface's where a plan cannot hold those or there
+  // is no memory for the pairs of every job.
+  const fct::Buffer tables[3] = {
+      {reinterpret_cast<void**>(&b->d_jobs), n_jobs * sizeof(fct::BpArgs)},
+      {reinterpret_cast<void**>(&b->d_tile_start), (n_jobs + 1) * sizeof(int32_t)},
+      {reinterpret_cast<void**>(&b->d_queue), 8 * sizeof(uint32_t)}};
+  const hipError_t e = fct::plans_alloc_chain(b->plans.data(), n_jobs, tables, 3, false);
+  if (e != hipSuccess) return fail(hip_status(ctx, "batch buffers", e));
+  for (const fct_wfbp_gpu_plan* p : b->plans)
+    b->device_bytes += (int64_t)(p->storage_bytes() + p->scale_elems() * 4 + p->native_bytes());
   const int st = upload_jobs(b);
   if (st != FCT_OK) return fail(st);
   *out = b;

@@ -371,8 +371,19 @@ fct::RayProjArgs ray_args(const fct_wfbp_gpu_plan* p) {
   return a;
 }
 
+// Free memory of the current device beyond `later` bytes.
+size_t free_memory(size_t later) {
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return avail > later ? avail - later : 0;
+}
+
 // A plan-owned device buffer allocated on first use; nullptr (and no error
-// left behind) when it does not fit or the plan's stream is being captured
+// left behind) when it does not fit beside the buffers the plan's other calls
+// cannot do without, or the plan's stream is being captured
 // into a graph, where the callers take a path without it.  A capture that runs
 // on another stream forbids allocations in its mode and would end invalid: the
 // thread's mode is relaxed meanwhile (the buffer is no part of that graph).
@@ -380,8 +391,10 @@ void* try_scratch(fct_wfbp_gpu_plan* p, size_t bytes) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   void* d = nullptr;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const size_t later = p->later_bytes() + (p->d_filtered ? 0 : p->filtered_bytes()) +
+                       (p->d_native ? 0 : p->native_bytes());
   bool ok = hipStreamIsCapturing(p->stream, &cap) == hipSuccess &&
-            cap == hipStreamCaptureStatusNone &&
+            cap == hipStreamCaptureStatusNone && bytes <= free_memory(later) &&
             hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
   if (ok) {
     ok = hipMalloc(&d, bytes) == hipSuccess;
@@ -630,18 +643,44 @@ int chain_backproject(fct_wfbp_gpu_plan* p, const void* filtered, const float* s
   return FCT_OK;
 }
 
-hipError_t plan_alloc_filtered(fct_wfbp_gpu_plan* p) {
-  if (p->d_filtered) return hipSuccess;
-  if (p->pairs) {
-    if (hipMalloc(&p->d_filtered, p->storage_bytes()) == hipSuccess) return hipSuccess;
-    (void)hipGetLastError();
+hipError_t plans_alloc_chain(fct_wfbp_gpu_plan* const* plans, int n, const Buffer* extra,
+                             int n_extra, bool reserve) try {
+  bool there = true;   // every call but a plan's first
+  for (int i = 0; i < n_extra; ++i) there = there && *extra[i].at;
+  for (int j = 0; j < n; ++j)
+    there = there && plans[j]->d_filtered && plans[j]->d_native &&
+            (plans[j]->d_scale || !plans[j]->scale_elems());
+  if (there) return hipSuccess;
+  std::vector<Buffer> other(extra, extra + n_extra);
+  std::vector<FilteredBuffer> filt;
+  bool pairs = true;
+  for (int j = 0; j < n; ++j) {
+    fct_wfbp_gpu_plan* p = plans[j];
+    other.push_back(Buffer{reinterpret_cast<void**>(&p->d_scale), p->scale_elems() * sizeof(float)});
+    other.push_back(Buffer{reinterpret_cast<void**>(&p->d_native), p->native_bytes()});
+    filt.push_back(FilteredBuffer{&p->d_filtered, p->pairs_bytes(), p->filtered_bytes()});
+    pairs = pairs && p->pairs;
   }
-  const hipError_t e = hipMalloc(&p->d_filtered, p->filtered_bytes());
-  if (e == hipSuccess)
-    p->pairs = false;
-  else
-    p->d_filtered = nullptr;
+  const hipError_t e = alloc_chain(
+      other.data(), (int)other.size(), filt.data(), n, &pairs,
+      [](void** at, size_t bytes) {
+        const hipError_t err = hipMalloc(at, bytes);
+        if (err != hipSuccess) {
+          *at = nullptr;
+          (void)hipGetLastError();
+        }
+        return err;
+      },
+      [](void* d) { (void)hipFree(d); },
+      [&] {
+        size_t later = 0;
+        for (int j = 0; reserve && j < n; ++j) later += plans[j]->later_bytes();
+        return free_memory(later);
+      });
+  for (int j = 0; j < n; ++j) plans[j]->pairs = pairs;
   return e;
+} catch (const std::bad_alloc&) {
+  return hipErrorOutOfMemory;
 }
 
 }  // namespace fct
@@ -665,19 +704,14 @@ int reconstruct_streaming(fct_wfbp_gpu_plan* p, const ViewSource& src, int vpc,
   vpc = std::min(vpc, nv);
   const size_t per_view = (size_t)p->raw_scan.n_rows * p->raw_scan.n_channels;
   const size_t plane = (size_t)p->recon.ny * p->recon.nx;
-  const size_t nat_bytes = (size_t)p->n_native * plane * sizeof(float);
-  const size_t vol_bytes = (size_t)p->n_req * plane * sizeof(float);
+  const size_t vol_bytes = p->volume_bytes();
   int2 par, rawr;
   needed_views(p, &par, &rawr);
   const int nchunks = rawr.y > rawr.x ? (rawr.y - rawr.x + vpc - 1) / vpc : 0;
-  HIP_TRY(ctx, fct::plan_alloc_filtered(p));
-  if (p->scale_elems() && !p->d_scale)
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&p->d_scale), p->scale_elems() * sizeof(float)));
-  if (!p->d_native) HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&p->d_native), nat_bytes));
-  if (!p->d_raw_stage)
-    HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&p->d_raw_stage),
-                           (size_t)p->raw_elems() * sizeof(float)));
-  if (!p->d_vol_stage) HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&p->d_vol_stage), vol_bytes));
+  const fct::Buffer staging[2] = {
+      {reinterpret_cast<void**>(&p->d_raw_stage), (size_t)p->raw_elems() * sizeof(float)},
+      {reinterpret_cast<void**>(&p->d_vol_stage), vol_bytes}};
+  HIP_TRY(ctx, fct::plans_alloc_chain(&p, 1, staging, 2, true));
   if (!ctx->copy_stream)
     HIP_TRY(ctx, hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking));
   for (int b = 0; b < 2; ++b) {
@@ -1682,12 +1716,7 @@ FCT_API int fct_wfbp_gpu_reconstruct(fct_wfbp_gpu_plan* p, const float* raw, flo
   HIP_TRY(p->ctx, hipSetDevice(p->device));
   if (host_buffers) return reconstruct_streaming(p, ViewSource{raw, nullptr, nullptr}, 0, 0.0f,
                                                  volume);
-  const size_t nat_bytes = (size_t)p->n_native * p->recon.ny * p->recon.nx * sizeof(float);
-  HIP_TRY(p->ctx, fct::plan_alloc_filtered(p));
-  if (p->scale_elems() && !p->d_scale)
-    HIP_TRY(p->ctx, hipMalloc(reinterpret_cast<void**>(&p->d_scale),
-                              p->scale_elems() * sizeof(float)));
-  if (!p->d_native) HIP_TRY(p->ctx, hipMalloc(reinterpret_cast<void**>(&p->d_native), nat_bytes));
+  HIP_TRY(p->ctx, fct::plans_alloc_chain(&p, 1, nullptr, 0, true));
   int st = fct::chain_rebin_filter(p, raw, p->d_filtered, p->d_scale, p->pairs);
   if (st) return st;
   st = fct::chain_backproject(p, p->d_filtered, p->d_scale, p->d_native, p->pairs);

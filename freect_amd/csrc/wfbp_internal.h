@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/fct_wfbp_gpu.h"
+#include "chain_buffers.h"
 #include "ffs_geometry.h"
 #include "wfbp_math.h"
 
@@ -347,9 +348,12 @@ int chain_rebin_filter(fct_wfbp_gpu_plan* p, const float* raw, void* filtered, f
 // (pairs), or in the interface's.
 int chain_backproject(fct_wfbp_gpu_plan* p, const void* filtered, const float* scale,
                       float* native, bool pairs);
-// Allocates the plan's filtered projections, as pairs where p->pairs; where
-// there is no memory for those, as rows (p->pairs becomes false).
-hipError_t plan_alloc_filtered(fct_wfbp_gpu_plan* p);
+// alloc_chain on the current device, for n plans of one precision: the scale
+// and native volumes, `extra`, then the filtered projections, as pairs in all of
+// the plans or in none (p->pairs).  reserve: pairs only where they leave what
+// the plans' other calls allocate (later_bytes).
+hipError_t plans_alloc_chain(fct_wfbp_gpu_plan* const* plans, int n, const Buffer* extra,
+                             int n_extra, bool reserve);
 }  // namespace fct
 
 struct fct_wfbp_gpu_ctx {
@@ -454,11 +458,21 @@ struct fct_wfbp_gpu_plan {
   }
   // The plan's own buffer between the stages of a whole chain.
   int storage() const { return pairs ? fct::pair_storage(opts.precision) : opts.precision; }
-  size_t storage_entry_bytes() const {
-    return pairs ? (opts.precision == FCT_PRECISION_FP32 ? 8 : 4) : filtered_entry_bytes();
+  size_t storage_bytes() const { return pairs ? pairs_bytes() : filtered_bytes(); }
+  size_t storage_entry_bytes() const { return storage_bytes() / ((size_t)nviews * nrows * cpitch); }
+  size_t pairs_bytes() const {
+    return (size_t)nviews * nrows * cpitch * (opts.precision == FCT_PRECISION_FP32 ? 8 : 4);
   }
-  size_t storage_bytes() const {
-    return (size_t)nviews * nrows * cpitch * storage_entry_bytes();
+  size_t native_bytes() const {
+    return (size_t)n_native * recon.ny * recon.nx * sizeof(float);
+  }
+  size_t volume_bytes() const { return (size_t)n_req * recon.ny * recon.nx * sizeof(float); }
+  // What calls beside the chain on device buffers may still have to allocate
+  // and have no way around: the host paths' staging, the adjoint's lines.
+  size_t later_bytes() const {
+    return (d_raw_stage ? 0 : (size_t)raw_elems() * sizeof(float)) +
+           (d_vol_stage ? 0 : volume_bytes()) +
+           (d_gbar ? 0 : (size_t)nviews * nrows * cpitch * sizeof(float));
   }
   size_t scale_elems() const {
     return opts.precision == FCT_PRECISION_FP32 ? 0 : (size_t)fct::kScaleElems;
