@@ -89,3 +89,31 @@ def test_rebin_transpose_at_the_scan_ends(ctx, oracle, views, channels, rows, ff
     p.synchronize()
     ref = oracle.rebin_adjoint(sc, g[..., : i.n_filtered_channels].astype(np.float64))
     assert np.abs(out.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+def test_weights_are_divided(ctx):
+    # xbar scale / sum W, correctly rounded, as the scattering kernel divides:
+    # one voxel on the axis and on a channel, in the plane of a view's focal
+    # spot (row 3.5, both halves exact).  Three views of that theta~ see it, all
+    # in the flat part of W, so that sum W = 3 and each W = 1 exactly: the two
+    # samples of the middle view are x / 3 / 2 to the bit.
+    import math
+
+    import numpy as np
+
+    from freect_amd import wfbp
+    w = S.tiny(nx=9, n_slices=4, n_rows=8, ppr=96, rotations=4.0)
+    dz, v = 0.1875, 200   # (half a feed: 9 mm, 0.514 of the 17.5 mm cone at the axis)
+    sc = w.scan.replace(feed=dz * 96, z0=-dz * v, central_channel=48.0)
+    rc = w.recon.replace(start_pos=0.0, end_pos=4 * sc.csw, recon_fov=200.0)
+    p = wfbp.Plan(ctx, sc, rc)
+    x, g = p.alloc_native().zero_(), p.alloc_lines()
+    scale = np.float32(2.0 * math.pi / 96)
+    for xb in np.random.RandomState(0).uniform(1.0, 2.0, 64).astype(np.float32):
+        x[0, 4, 4] = float(xb)
+        p.backproject_adjoint(x, g)
+        p.synchronize()
+        got = g[v, :, 48].cpu().numpy()
+        want = np.zeros(8, np.float32)
+        want[3:5] = xb * scale / np.float32(3.0) / np.float32(2.0)
+        assert np.array_equal(got, want), (got, want)
