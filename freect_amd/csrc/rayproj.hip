@@ -150,8 +150,8 @@ __global__ __launch_bounds__(256) void ray_backproject_kernel(RayProjArgs a) {
 // on its channel only: fq = A + i B (sample position at plane i), the
 // fraction of the way from the focal spot to the detector T = T0 + i DT, and
 // fz = zoff + T (w_row - oz) / gdz.  ray_table_kernel writes (A, B, T0, DT)
-// per (view, channel) from FP64; the low bit of DT says whether the planes
-// are x planes.
+// per (view, channel) from FP64, and a bit that says whether the planes are x
+// planes.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void ray_table_kernel(RayProjArgs a, RayTables t) {
   const int c = blockIdx.x * 256 + threadIdx.x;
@@ -178,11 +178,17 @@ __global__ __launch_bounds__(256) void ray_table_kernel(RayProjArgs a, RayTables
   const double sp = xmajor ? sx : sy, sq = xmajor ? sy : sx;
   const double up = xmajor ? ux : uy, uq = xmajor ? uy : ux;
   const double t0 = (p0 - sp) / up, dt = dp / up;
-  const int dtb = (__float_as_int((float)dt) & ~1) | (xmajor ? 1 : 0);
-  t.ray[(size_t)v * a.ncols + c] = make_float4((float)((sq + t0 * uq - q0) / dq),
-                                               (float)(dt * uq / dq), (float)t0,
-                                               __int_as_float(dtb));
+  t.ray[(size_t)v * a.ncols + c] =
+      make_float4((float)((sq + t0 * uq - q0) / dq), (float)(dt * uq / dq), (float)t0, (float)dt);
+  const uint64_t bits = __ballot(xmajor);   // (a wave: 64 channels from a multiple of 64)
+  if ((c & 63) == 0) t.axis[(size_t)v * ((a.ncols + 63) >> 6) + (c >> 6)] = bits;
   if (v < a.states) t.len2[(size_t)rho * a.ncols + c] = (float)(ux * ux + uy * uy);
+}
+
+// Whether the planes of (view, channel) are x planes.
+__device__ __forceinline__ bool x_planes(const RayTables& t, int ncols, int v, int c) {
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(t.axis + (size_t)v * ((ncols + 63) >> 6));
+  return w[c >> 5] >> (c & 31) & 1;
 }
 
 // The volume with two planes of zeros on every side, in its own order and
@@ -305,7 +311,7 @@ __global__ __launch_bounds__(64 * kRayRows) void ray_project_table_kernel(RayPro
   if (row >= a.nrows) return;
   const bool in = c < a.ncols;
   const float4 e = t.ray[(size_t)v * a.ncols + (in ? c : a.ncols - 1)];
-  const bool xm = __float_as_int(e.w) & 1;
+  const bool xm = ld_uniform(t.axis + (size_t)v * cg + rest % cg) >> (c & 63) & 1;
   const double oz = a.states > 1 ? t.zsrc[v % a.states] : 0.0;
   const double wz = ((double)row - a.cr) * a.drow - oz;
   const double g = wz / a.ddz;
@@ -368,7 +374,7 @@ __global__ __launch_bounds__(256) void ray_record_kernel(RayProjArgs a, RayTable
   const int v = blockIdx.x / cg, c = (blockIdx.x - v * cg) * 256 + threadIdx.x;
   if (c >= a.ncols) return;
   const RayDir d = ray_dir(a, v, c);
-  const bool xmajor = __float_as_int(t.ray[(size_t)v * a.ncols + c].w) & 1;
+  const bool xmajor = x_planes(t, a.ncols, v, c);
   for (int row = 0; row < a.nrows; ++row) {
     const Ray r = ray_of(a, d, row);
     const float p0 = xmajor ? a.gx0 : a.gy0, dp = xmajor ? a.gdx : a.gdy;
@@ -476,8 +482,9 @@ __global__ __launch_bounds__(64) void ray_gather_kernel(RayProjArgs a, RayTables
     const float4* tv = t.ray + (size_t)v * a.ncols;
     for (int m = 0; m < nc; ++m) {
       const int c = c0 + m;
-      const float4 e = tv[min(c, a.ncols - 1)];
-      const bool xm = __float_as_int(e.w) & 1;
+      const int cc = min(c, a.ncols - 1);
+      const float4 e = tv[cc];
+      const bool xm = x_planes(t, a.ncols, v, cc);
       const float prim = xm ? fix : fiy, sec = xm ? fiy : fix;
       // (The rows' own positions differ from the table's by rounding.)
       if (!(fabsf(fmaf(prim, e.y, e.x) - sec) < 1.001f) || c > c1) continue;
@@ -559,6 +566,7 @@ bool ray_tables_apply(const RayProjArgs& a) {
 size_t ray_table_bytes(const RayProjArgs& a) {
   const size_t nv = a.v1;
   return nv * a.ncols * sizeof(float4) + 2 * nv * sizeof(float4) + nv * sizeof(double) +
+         nv * ((a.ncols + 63) / 64) * sizeof(uint64_t) +
          (size_t)a.states * a.ncols * sizeof(float);
 }
 
@@ -578,6 +586,7 @@ RayTables ray_table_layout(const RayProjArgs& a, void* mem) {
   t.ray = reinterpret_cast<float4*>(take(nv * a.ncols * sizeof(float4)));
   t.view = reinterpret_cast<float4*>(take(2 * nv * sizeof(float4)));
   t.zoff = reinterpret_cast<double*>(take(nv * sizeof(double)));
+  t.axis = reinterpret_cast<uint64_t*>(take(nv * ((a.ncols + 63) / 64) * sizeof(uint64_t)));
   t.len2 = reinterpret_cast<float*>(take((size_t)a.states * a.ncols * sizeof(float)));
   for (int s = 0; s < a.states; ++s) t.zsrc[s] = a.ffs_off[s][2];
   return t;

@@ -227,9 +227,10 @@ struct RayProjArgs {
 
 // Geometry tables of the table-driven ray projector (rayproj.hip).
 struct RayTables {
-  float4* ray;     // [view][channel] A, B, T0, DT (low bit of DT: x planes)
+  float4* ray;     // [view][channel] A, B, T0, DT
   float4* view;    // [view][2]: cos, sin, R + o0, o1; (-cr drow - oz) / gdz, o0, -, -
   double* zoff;    // [view] focal spot z in slices
+  uint64_t* axis;  // [view][64 channels] bit: the ray's planes are x planes
   float* len2;     // [focal state][channel] squared in-plane source-detector distance
   double zsrc[4];  // focal state's z offset
 };
