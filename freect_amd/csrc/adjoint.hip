@@ -271,8 +271,8 @@ __global__ __launch_bounds__(256) void swap_volume_kernel(const float* __restric
 // whose channel position lies within one channel of the lane's (a fixed
 // small number of candidates around the ray, tested with the forward
 // kernels' FP32 position) add their slices into the lane's rows (one LDS read
-// and write of two rows per slice, conflict-free).  Bound by VALU issue: 25
-// instructions per slice of a candidate, of whose lanes half to three quarters
+// and write of two rows per slice, conflict-free).  23 VALU
+// instructions per slice of a candidate (14 in the matched projector), of whose lanes half to three quarters
 // hold one.  2952 views x 16 x 736 from 384 x 384 x 32 voxels: 287 ms with
 // four global atomics per sample -> 3.75 (weights) + 11.3 ms.  RC rows per
 // wave: 16 or 32, so that the rows in LDS leave at least 16 waves per CU.
@@ -414,11 +414,11 @@ __global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjG
             val *= fct_w_of_t(
                 __builtin_amdgcn_fmed3f(fmaf(-fabsf(qi - g.cr), g.wk, FCT_WC), 0.0f, 1.0f));
           val = sel ? val : 0.0f;
-          const float hi = val * __builtin_amdgcn_fractf(qi);
+          const float wq = __builtin_amdgcn_fractf(qi);
           float* r = lrow + min(l, (uint32_t)rspan) * 64;
           const float r0 = r[0], r1 = r[64];
-          r[0] = r0 + (val - hi);
-          r[64] = r1 + hi;
+          r[0] = fmaf(val, 1.0f - wq, r0);   // (finite weights: val may be infinite)
+          r[64] = fmaf(val, wq, r1);
         };
         const float* xp = vplane;
         int s = sl;

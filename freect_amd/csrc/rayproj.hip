@@ -281,17 +281,19 @@ struct RayWalk {
 };
 __device__ __forceinline__ float ray_combine(const RayTap& t) {
   const uint32_t a0 = t.a.x, a1 = t.a.y, b0 = t.b.x, b1 = t.b.y;
-  const float x0 = __uint_as_float(a0), y0 = __uint_as_float(b0);
-  const float lo = fmaf(t.wq, __uint_as_float(a1) - x0, x0);
-  const float hi = fmaf(t.wq, __uint_as_float(b1) - y0, y0);
-  return fmaf(t.wz, hi - lo, lo);
+  // Products with both weights, not a + w (b - a): an infinite sample gives an
+  // infinite value there, as in the general kernel, and not a NaN.
+  const float uq = 1.0f - t.wq, uz = 1.0f - t.wz;
+  const float lo = fmaf(t.wq, __uint_as_float(a1), uq * __uint_as_float(a0));
+  const float hi = fmaf(t.wq, __uint_as_float(b1), uq * __uint_as_float(b0));
+  return fmaf(t.wz, hi, uz * lo);
 }
 
 // One ray per lane, 64 neighbouring channels of one detector row per wave,
 // four rows per workgroup: the waves of a workgroup read the same columns of
 // neighbouring slices.  A wave's lanes advance plane by plane together; the
 // planes that every one of its rays samples run unmasked, four at a time
-// (their loads in flight).  About 15 VALU instructions and one 16-byte load
+// (their loads in flight).  18 VALU instructions and one 16-byte load
 // per sample instead of 40 and four loads: 1476 views x 16 x 736 rays through
 // 384 x 384 x 32 voxels 30.8 -> 5.9 ms with two 8-byte loads (which bound it:
 // 19 cycles of a CU's L1 each, VALU 2.8 ms of the 5.9), 4.3 ms with one of 16
@@ -403,7 +405,7 @@ __global__ __launch_bounds__(256) void ray_record_kernel(RayProjArgs a, RayTable
 // often (9.0 ms), and is used where the volume has no more slices.  The
 // views are split so that about 128 waves per CU are launched (at 32 the
 // last round of waves leaves the chip half empty: 11.7 ms); each adds its
-// sums to the volume once, at its end.  About 22 VALU instructions per row.
+// sums to the volume once, at its end.  15 VALU instructions per row.
 template <int K, bool FFS>
 __global__ __launch_bounds__(64) void ray_gather_kernel(RayProjArgs a, RayTables t, RayGather q) {
   // Slice k at row k + 2; rows 0, 1, K + 2, K + 3 take what falls outside.
@@ -496,11 +498,11 @@ __global__ __launch_bounds__(64) void ray_gather_kernel(RayProjArgs a, RayTables
         const float s = w > 0.0f ? w * __uint_as_float(V) : 0.0f;
         const float fz = fmaf(r, Sz, F0);
         const int k = min(max(floor_int(fz), -2), K);
-        const float hi = s * __builtin_amdgcn_fractf(fz);
+        const float wz = __builtin_amdgcn_fractf(fz);
         float* p = acc + (k + 2) * 64 + lane;
         const float x0 = p[0], x1 = p[64];
-        p[0] = x0 + (s - hi);
-        p[64] = x1 + hi;
+        p[0] = fmaf(s, 1.0f - wz, x0);   // (finite weights: s may be infinite)
+        p[64] = fmaf(s, wz, x1);
       };
       int r = rlo;
       for (; r + 3 <= rhi; r += 4) {

@@ -117,3 +117,33 @@ def test_weights_are_divided(ctx):
         want = np.zeros(8, np.float32)
         want[3:5] = xb * scale / np.float32(3.0) / np.float32(2.0)
         assert np.array_equal(got, want), (got, want)
+
+
+@pytest.mark.parametrize("bad", ["inf", "-inf", "nan"])
+@pytest.mark.parametrize("op", ["backproject_adjoint", "matched_project", "ray_project",
+                                "ray_backproject"])
+def test_nonfinite_samples(ctx, op, bad):
+    # One sample that is not finite: the gathers and the table projector give
+    # infinities and NaNs where the general kernels (a capture on a fresh plan)
+    # give them, an infinite sample no NaN.
+    from freect_amd import wfbp
+    w = S.tiny(nx=40, n_slices=12, rotations=2.5)
+    sc, rc = w.scan.replace(angle0=0.4), w.recon.replace(x_origin=3.1)
+    p, general = wfbp.Plan(ctx, sc, rc), wfbp.Plan(ctx, sc, rc)
+    x = (p.alloc_raw() if op == "ray_backproject" else p.alloc_native()).uniform_(0.1, 1.0)
+    x.view(-1)[x.numel() // 2 + 11] = float(bad)
+    got = {"ray_project": p.alloc_raw, "ray_backproject": p.alloc_native}.get(op, p.alloc_lines)()
+    ref = torch.empty_like(got)
+    getattr(p, op)(x, got)
+    s = torch.cuda.Stream()
+    general.set_stream(s)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        getattr(general, op)(x, ref)
+    g.replay()
+    torch.cuda.synchronize()
+    assert not ref.isfinite().all()
+    assert torch.equal(got.isnan(), ref.isnan())
+    for v in (float("inf"), float("-inf")):
+        assert torch.equal(got == v, ref == v)
