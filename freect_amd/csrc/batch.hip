@@ -31,12 +31,24 @@ struct fct_wfbp_gpu_batch {
   uint32_t* d_queue = nullptr;       // [8]
   int total_tiles = 0;
   int grid = 0;
+  bool apart = false;                // the jobs' backprojections are launched one by one
   int64_t device_bytes = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
 
 namespace {
+
+// Batches of fewer tiles launch their jobs' backprojections one by one, each
+// tile's theta~ segments in as many waves (bp_segments), instead of one wave per
+// tile in the persistent kernel, which leaves half of the chip or more idle.
+// Measured, persistent / one by one (the same volumes bitwise): 267 tiles of 2
+// FP32 jobs 3.40 / 0.51 ms, 1275 of 8 BF16 9.4 / 5.7, 2028 of 2 BF16 3.3 / 1.8, 3424 of
+// 4 BF16 3.9 / 3.3; 5064 of 4 FP16 4.0 / 3.6, 6915 of 4 FP32 4.5 / 6.5, 10 421 of 8
+// FP32 7.9 / 9.4 (two to eight waves per SIMD and the last waves of every job).
+// The one wave's sums over segments also made small FP32 batches slower than a
+// single sweep had been (3.25 ms the first).
+constexpr int kApartTiles = 4096;
 
 void set_err(fct_wfbp_gpu_ctx* ctx, const char* msg, hipError_t e = hipSuccess) {
   if (!ctx) return;
@@ -85,6 +97,8 @@ int upload_jobs(fct_wfbp_gpu_batch* b) {
   if (total >= (1LL << 30)) return set_err(b->ctx, "too many tiles in one batch"), FCT_ERR_LIMIT;
   start[n] = (int32_t)total;
   b->total_tiles = (int)total;
+  b->apart = n == 1 || total < kApartTiles;
+  for (const fct::BpArgs& a : jobs) b->apart = b->apart && (n == 1 || a.nseg > 1);
   BATCH_TRY(b, hipMemcpyAsync(b->d_jobs, jobs.data(), n * sizeof(fct::BpArgs),
                               hipMemcpyHostToDevice, b->stream));
   BATCH_TRY(b, hipMemcpyAsync(b->d_tile_start, start.data(), (n + 1) * sizeof(int32_t),
@@ -105,19 +119,20 @@ bool all_centered(const fct_wfbp_gpu_batch* b) {
 }
 
 // The persistent backprojection of every job (queue counters cleared by a
-// kernel, so the sequence can be recorded into a graph).  A batch of one job
-// has no tiles of other jobs to balance: it launches the single-plan grid
-// kernel, which runs the same tile code (the volume is bitwise the same) and
-// has no queue to walk.
+// kernel, so the sequence can be recorded into a graph).  A batch of one job,
+// which has no tiles of other jobs to balance, and a small one (kApartTiles)
+// launch the single-plan grid kernels, which run the same tile code (the volumes
+// are bitwise the same) and have no queue to walk.
 int enqueue_backproject(fct_wfbp_gpu_batch* b) {
-  if (b->plans.size() == 1) {
-    fct_wfbp_gpu_plan* p = b->plans[0];
-    fct::BpArgs a = fct::plan_bp_args(p);
-    a.filt = p->d_filtered;
-    a.filt_scale = p->d_scale;
-    a.native = p->d_native;
-    BATCH_TRY(b, fct::launch_backproject_v1(a, p->tile_z, p->storage(), fct::kBpAccumulate,
-                                            b->stream));
+  if (b->apart) {
+    for (fct_wfbp_gpu_plan* p : b->plans) {
+      fct::BpArgs a = fct::plan_bp_args(p);
+      a.filt = p->d_filtered;
+      a.filt_scale = p->d_scale;
+      a.native = p->d_native;
+      BATCH_TRY(b, fct::launch_backproject_v1(a, p->tile_z, p->storage(), fct::kBpAccumulate,
+                                              b->stream));
+    }
     return FCT_OK;
   }
   BATCH_TRY(b, fct::launch_fill(reinterpret_cast<float*>(b->d_queue), 8, 0.0f, b->stream));

@@ -361,7 +361,8 @@ FCT_API int fct_wfbp_gpu_phantom_project(fct_wfbp_gpu_ctx* ctx, const fct_scan_g
  * precision and tile_z, any geometry / matrix / slice range / filter) plus
  * every intermediate buffer.  One run is: rebin_filter of every job, ONE
  * persistent backprojection launch over the tiles of all jobs (work queue per
- * XCD; a batch of one job launches the single-plan grid kernel instead),
+ * XCD; a batch of one job or of few tiles launches the single-plan grid
+ * kernels instead),
  * thicken of every job -- recorded once into a hipGraph and replayed.
  * Each job's volume is bitwise identical to fct_wfbp_gpu_reconstruct on a
  * plan with the same options. */

@@ -129,3 +129,31 @@ def test_batch_errors(ctx):
     with pytest.raises(wfbp.FctError):
         b.autotune((5,))             # not a tile depth
     b.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("nx,slices,tile_z", [(240, 8, 4), (200, 8, 4), (40, 40, 32), (20, 9, 8)])
+def test_batch_launch_forms(ctx, precision, nx, slices, tile_z):
+    # Batches on both sides of the tile count up to which the jobs are launched
+    # one by one, and small ones whose tiles are too deep for segments: bitwise
+    # the single plans, recorded and eager.
+    from freect_amd import wfbp
+    ws = [S.tiny(seed=11, nx=nx, n_slices=slices, rotations=4.0),
+          S.tiny(seed=12, nx=nx - 9, n_slices=slices + 3, rotations=4.0, n_rows=12, ppr=64)]
+    raws = [ctx.phantom_project(w.scan, w.phantom, 0.0, w.seed) for w in ws]
+    torch.cuda.synchronize()
+    b = wfbp.Batch(ctx, [(w.scan, w.recon) for w in ws], precision=precision, tile_z=tile_z)
+    assert (b.info()["total_tiles"] >= 4096) == (nx == 240)
+    vols = [p.alloc_volume() for p in b.plans]
+    for j, (r, v) in enumerate(zip(raws, vols)):
+        b.submit(j, r, v)
+    ref = [_single(ctx, w, r, precision, tile_z) for w, r in zip(ws, raws)]
+    for mode in (wfbp.Batch.EAGER, wfbp.Batch.GRAPH, wfbp.Batch.GRAPH):
+        for v in vols:
+            v.fill_(float("nan"))
+        torch.cuda.synchronize()
+        b.run(mode)
+        b.synchronize()
+        for v, e in zip(vols, ref):
+            assert e.abs().max() > 0 and torch.equal(v, e)
+    b.close()
