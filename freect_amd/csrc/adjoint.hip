@@ -201,8 +201,10 @@ __global__ __launch_bounds__(64) void bp_adjoint_weights_kernel(BpAdjArgs a, Adj
   const float* ztc = b.zt + (size_t)chunk * b.nviews;
   const int* wrc = reinterpret_cast<const int*>(b.wrange + (size_t)chunk * b.nviews);
   const size_t plane = (size_t)b.nx * b.ny;
-  float* out = q.wgt + ((size_t)prim * b.n_native + s0) * ns + sec;
-  for (int ti = 0; ti < q.nt; ++ti, out += plane * b.n_native) {
+  const int ti0 = (int)((long long)q.nt * blockIdx.y / gridDim.y);
+  const int ti1 = (int)((long long)q.nt * (blockIdx.y + 1) / gridDim.y);
+  float* out = q.wgt + ti0 * plane * b.n_native + ((size_t)prim * b.n_native + s0) * ns + sec;
+  for (int ti = ti0; ti < ti1; ++ti, out += plane * b.n_native) {
     const int t = q.t0 + ti;
     float den[kAdjSlices];
 #pragma unroll
@@ -274,7 +276,10 @@ __global__ __launch_bounds__(256) void swap_volume_kernel(const float* __restric
 // and write of two rows per slice, conflict-free).  23 VALU
 // instructions per slice of a candidate (14 in the matched projector), of whose lanes half to three quarters
 // hold one.  2952 views x 16 x 736 from 384 x 384 x 32 voxels: 287 ms with
-// four global atomics per sample -> 3.75 (weights) + 11.3 ms.  RC rows per
+// four global atomics per sample -> 4.3 (weights) + 11.1 ms.  Planes on which no
+// lane has a voxel in its rows are left out (9840 views x 64 x 888, 32 x 32 x 4 of
+// 40 mm: 5.2 -> 2.4 ms, where the atomics take 2.6; 2304 views x 16 x 736, 512 x 1 x
+// 16: 2.7 -> 1.0 ms, atomics 1.8).  RC rows per
 // wave: 16 or 32, so that the rows in LDS leave at least 16 waves per CU.
 template <int RC, bool CENTERED, bool MATCHED>
 __global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjGather q) {
@@ -352,6 +357,7 @@ __global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjG
   const size_t pstride = MATCHED && !q.swap ? (size_t)b.nx : (size_t)b.n_native * ns;
   const size_t sstride = MATCHED && !q.swap ? (size_t)b.nx * b.ny : (size_t)ns;
 
+  bool touched = false;   // (wave-uniform)
   for (int chunk = 0; rspan >= 0 && chunk < nchunks; ++chunk) {
     const int a0 = chunk * fct_tables::kSliceChunk;
     const int na = min(fct_tables::kSliceChunk, b.n_native - a0);
@@ -381,13 +387,33 @@ __global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjG
     const float zc = ztv - kb0 - zfirst, sm = fmaf(zmargin, fabsf(inv_dz), 0.05f);
     const float A0 = fmaf(ra, L0, zc) * inv_dz, A1 = ra * L1 * inv_dz;
     const float B0 = fmaf(rb, L0, zc) * inv_dz, B1 = rb * L1 * inv_dz;
-    for (int i = i0; i < i1; ++i) {
+    // Planes on which the ray lies in the grid and these slices between the two
+    // rows (their crossings keep their order along the ray): for every lane an
+    // interval, as all of this is linear in the plane index.  A tenth of a column
+    // or slice covers the rounding of the positions, a plane that of the ends.
+    float lo = (float)i0, hi = (float)(i1 - 1);
+    auto at_least = [&](float a, float b, float c) {   // a + b i >= c
+      const float t = (c - a) / b;
+      if (b > 0.0f) lo = fmaxf(lo, t);
+      if (b < 0.0f) hi = fminf(hi, t);
+      if (b == 0.0f && a < c) hi = -1.0f;
+    };
+    const bool up = inv_dz > 0.0f;
+    at_least(J0, J1, -hw - 0.1f);
+    at_least(-J0, -J1, (float)(1 - ns) - hw - 0.1f);
+    at_least(up ? B0 : A0, up ? B1 : A1, (float)k0 - sm - 0.1f);
+    at_least(up ? -A0 : -B0, up ? -A1 : -B1, -(float)k1 - sm - 0.1f);
+    const bool meets = ch < g.ncols && lo <= hi;
+    const int ia = max(i0, wave_min_i(meets ? (int)floorf(lo) - 1 : INT32_MAX));
+    const int ib = min(i1 - 1, wave_max_i(meets ? (int)ceilf(hi) + 1 : -1));
+    for (int i = ia; i <= ib; ++i) {
       const float fi = (float)i, sa = fmaf(fi, A1, A0), sb = fmaf(fi, B1, B0);
       const int j0 = (int)ceilf(fmaf(fi, J1, J0) - hw);
       const bool some = ch < g.ncols && j0 < ns && j0 + nj > 0;
       const int sl = max(wave_min_i(some ? (int)ceilf(fminf(sa, sb) - sm) : INT32_MAX), k0);
       const int sh = min(wave_max_i(some ? (int)floorf(fmaxf(sa, sb) + sm) : -1), k1);
       if (sl > sh) continue;
+      touched = true;
       const float* vplane = vol + (size_t)i * pstride + (size_t)(a0 + sl) * sstride;
       for (int m = 0; m < nj; ++m) {
         const int j = j0 + m, jc = min(max(j, 0), ns - 1);
@@ -433,6 +459,7 @@ __global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjG
       }
     }
   }
+  if (q.nsplit > 1 && !touched) return;   // (gbar was cleared)
 #pragma unroll
   for (int r = 0; r < RC; ++r)
     if (R0 + r < g.nrows) {
@@ -535,8 +562,10 @@ hipError_t launch_adjoint_columns(const BpAdjArgs& a, const AdjGather& q, hipStr
 
 hipError_t launch_adjoint_weights(const BpAdjArgs& a, const AdjGather& q, hipStream_t s) {
   const int ns = q.swap ? a.bp.ny : a.bp.nx, np = q.swap ? a.bp.nx : a.bp.ny;
-  const dim3 grid((unsigned)((ns + 63) / 64 * np *
-                             ((a.bp.n_native + kAdjSlices - 1) / kAdjSlices)));
+  // Small volumes: the theta~ shared by several waves, towards 8192 (2304
+  // views x 16 x 736, 8 x 8 x 2 voxels, the whole call: 1.06 -> 0.19 ms).
+  const int waves = (ns + 63) / 64 * np * ((a.bp.n_native + kAdjSlices - 1) / kAdjSlices);
+  const dim3 grid((unsigned)waves, (unsigned)std::max(1, std::min(q.nt, 8192 / waves)));
   if (a.bp.g.cr == a.bp.g.hr)
     hipLaunchKernelGGL(bp_adjoint_weights_kernel<true>, grid, dim3(64), 0, s, a, q);
   else

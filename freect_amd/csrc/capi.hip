@@ -458,18 +458,26 @@ bool adjoint_gather(fct_wfbp_gpu_plan* p, const fct::BpAdjArgs& a, bool matched,
   // ray is as long as the launch: the planes of a ray are shared by several
   // waves, towards 65536 per launch (4096 x 16 rather than one wave per ray:
   // 2952 views x 16 x 736 from 384 x 384 x 32 voxels 18.7 -> 10.8 ms).
-  const long long launch = (long long)waves * (long long)nt;
-  const int np = std::min(p->recon.nx, p->recon.ny);
-  q.nsplit = (int)std::max(1LL, std::min<long long>(np / 16, (65536 + launch - 1) / launch));
-  if (q.nsplit > 1)
-    *err = fct::launch_fill(a.gbar, (size_t)p->nviews * p->nrows * p->cpitch, 0.0f, p->stream);
-  if (matched && *err == hipSuccess)
-    *err = fct::launch_swap_volume(a.xbar, q.wgt, p->recon.nx, p->recon.ny, p->n_native, p->stream);
-  for (int t = 0; t < p->H && *err == hipSuccess; t += q.nt) {
+  auto batch = [&](int t) {   // theta~ from t on with the same planes
     q.t0 = t;
     q.swap = p->h_xplanes[t];
     q.nt = 1;
     while (t + q.nt < p->H && q.nt < (int)nt && p->h_xplanes[t + q.nt] == q.swap) ++q.nt;
+    const long long launch = (long long)waves * q.nt;
+    const int np = q.swap ? p->recon.nx : p->recon.ny;
+    q.nsplit = (int)std::max(1LL, std::min<long long>(np / 16, (65536 + launch - 1) / launch));
+  };
+  bool split = false;
+  for (int t = 0; t < p->H; t += q.nt) {
+    batch(t);
+    split = split || q.nsplit > 1;
+  }
+  if (split)
+    *err = fct::launch_fill(a.gbar, (size_t)p->nviews * p->nrows * p->cpitch, 0.0f, p->stream);
+  if (matched && *err == hipSuccess)
+    *err = fct::launch_swap_volume(a.xbar, q.wgt, p->recon.nx, p->recon.ny, p->n_native, p->stream);
+  for (int t = 0; t < p->H && *err == hipSuccess; t += q.nt) {
+    batch(t);
     *err = fct::launch_adjoint_columns(a, q, p->stream);
     if (!matched && *err == hipSuccess) *err = fct::launch_adjoint_weights(a, q, p->stream);
     if (*err == hipSuccess) *err = fct::launch_adjoint_gather(a, q, matched, p->stream);

@@ -147,3 +147,36 @@ def test_nonfinite_samples(ctx, op, bad):
     assert torch.equal(got.isnan(), ref.isnan())
     for v in (float("inf"), float("-inf")):
         assert torch.equal(got == v, ref == v)
+
+
+@pytest.mark.parametrize("nx,ny,slices,fov,x0,rotations,flip",
+                         [(200, 1, 9, 400.0, 0.0, 2.3, False), (1, 200, 9, 400.0, 0.0, 2.3, True),
+                          (64, 64, 2, 20.0, 140.0, 9.0, False), (64, 33, 3, 60.0, -120.0, 9.0, True),
+                          (48, 48, 130, 450.0, 0.0, 12.0, False),
+                          (40, 90, 130, 300.0, 40.0, 12.0, True)])
+@pytest.mark.parametrize("op", ["backproject_adjoint", "matched_project"])
+def test_planes_left_out(ctx, op, nx, ny, slices, fov, x0, rotations, flip):
+    # Volumes that most rays miss, thin ones, and ones of several chunks of
+    # slices: the gather leaves out the planes where no lane of a wave has a
+    # voxel.  Against the scattering kernels, with the bound of the comparison
+    # above.
+    from freect_amd import wfbp
+    w = S.tiny(nx=nx, n_slices=slices, n_channels=192, n_rows=17, rotations=rotations)
+    rc = w.recon.replace(ny=ny, recon_fov=fov, x_origin=x0, y_origin=0.4 * x0)
+    if flip:
+        rc = rc.replace(start_pos=rc.end_pos, end_pos=rc.start_pos)
+    p, general = wfbp.Plan(ctx, w.scan, rc), wfbp.Plan(ctx, w.scan, rc)
+    gen = torch.Generator(device="cuda").manual_seed(nx)
+    x = torch.rand(p.alloc_native().shape, device="cuda", generator=gen) + 0.1
+    got, ref = p.alloc_lines().fill_(float("nan")), p.alloc_lines()
+    getattr(p, op)(x, got)
+    s = torch.cuda.Stream()
+    general.set_stream(s)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        getattr(general, op)(x, ref)
+    g.replay()
+    torch.cuda.synchronize()
+    assert ref.abs().max() > 0
+    assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
