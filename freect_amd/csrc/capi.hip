@@ -1550,26 +1550,8 @@ FCT_API int fct_wfbp_gpu_set_output_units(fct_wfbp_gpu_plan* p, int32_t units, d
 FCT_API int fct_wfbp_gpu_rebin(fct_wfbp_gpu_plan* p, const float* raw, float* lines_out) {
   if (!p || !raw || !lines_out) return FCT_ERR_INVALID_ARGUMENT;
   HIP_TRY(p->ctx, hipSetDevice(p->device));
-  fct::RebinFilterArgs a{};
-  a.raw = raw;
-  a.out = lines_out;
-  a.tab = p->d_rebin;
-  a.Hn = p->d_Hn;
-  a.tw = p->d_tw;
-  a.nviews = p->nviews;
-  a.nrows = p->nrows;
-  a.ncols = p->ncols;
-  a.cpitch = p->cpitch;
-  a.nfft = p->nfft;
-  a.log2n = p->log2n;
+  fct::RebinFilterArgs a = rf_args(p, raw, lines_out, nullptr);
   a.precision = FCT_PRECISION_FP32;
-  a.nlines = p->nviews * p->nrows;
-  a.ncu = p->ncu;
-  a.raw_nrows = p->raw_scan.n_rows;
-  a.raw_ncols = p->raw_scan.n_channels;
-  a.states = p->ffs.S;
-  a.zshift = fct_ffs::has_z(p->ffs.mode) ? 1 : 0;
-  set_gather_window(p, &a);
   a.rebin_only = 1;
   HIP_TRY(p->ctx, fct::launch_rebin_filter(a, p->stream));
   return FCT_OK;

@@ -115,3 +115,24 @@ def test_ffs_plan_errors(ctx):
         wfbp.Plan(ctx, w.scan.replace(views_per_rotation=196), w.recon)   # not a multiple of 8
     with pytest.raises(wfbp.FctError):
         wfbp.Plan(ctx, w.scan.replace(anode_angle=0.0), w.recon)
+
+
+@pytest.mark.parametrize("channels,mode", [(96, 0), (200, 0), (400, 0), (888, 0), (1500, 0),
+                                           (300, 1), (700, 1), (1200, 2), (600, 3)])
+def test_rebin_lines_match_oracle(ctx, oracle, channels, mode):
+    # The rebinning without the filter, every kernel size, every view (the
+    # first half fan of them reads clamped projections): three interpolations of
+    # FP32 samples with FP32 weights, at most eight roundings of 2^-24 of the
+    # largest raw sample.
+    from freect_amd import wfbp
+    w = S.tiny(n_channels=channels, n_rows=5, ppr=192, rotations=1.5, ffs_mode=mode)
+    raw_t = ctx.phantom_project(w.scan, w.phantom, 0.0, w.seed)
+    p = wfbp.Plan(ctx, w.scan, w.recon)
+    lines = p.alloc_lines().fill_(float("nan"))
+    p.rebin_lines(raw_t, lines)
+    p.synchronize()
+    n = p.info.n_filtered_channels
+    got, raw = to_np(lines), to_np(raw_t)
+    err = np.abs(got[..., :n] - oracle.rebin(w.scan, raw)).max()
+    say("rebin_lines channels %d mode %d nfft %d err %.3g" % (channels, mode, p.info.nfft, err))
+    assert err <= 8 * 2.0 ** -24 * np.abs(raw).max() and np.count_nonzero(got[..., n:]) == 0
