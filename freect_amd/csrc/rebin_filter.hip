@@ -633,8 +633,11 @@ __device__ __forceinline__ void fft_forward_regs(FctCplx* v, FctCplx* lds, int t
 // eight waves, of which three per SIMD hold only one: there four (128 VGPRs,
 // two blocks per CU, some twiddles spilled) take the rebinning of 1728 x 64 x
 // 1472 samples (phi + z FFS) from 1.9 to 1.4 ms, its chain from 10.34 to 9.85.
-template <int N>
-__global__ __launch_bounds__(N / 8) __attribute__((amdgpu_waves_per_eu(N == 4096 ? 4 : 3, 8)))
+// The rebinning without the filter (RebinFilterArgs::rebin_only) stays at three
+// there, which leave more loads in flight: 2000 x 16 x 2048 samples 0.147 ms,
+// at four 0.186 (1728 x 64 x 1472 0.58 both).
+template <int N, int WAVES>
+__global__ __launch_bounds__(N / 8) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
 void rebin_filter_reg_kernel(RebinFilterArgs a) {
   using S = FctFftShape<N>;
   constexpr int T = S::T;
@@ -838,13 +841,13 @@ void rebin_filter_reg_kernel(RebinFilterArgs a) {
   }
 }
 
-template <int N>
+template <int N, int WAVES = 3>
 hipError_t launch_reg(const RebinFilterArgs& a, hipStream_t s) {
   static int per_cu = -1;   // resident blocks per CU (same for every device here)
   if (per_cu < 0) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rebin_filter_reg_kernel<N>, N / 8, 0) !=
-            hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rebin_filter_reg_kernel<N, WAVES>, N / 8,
+                                                     0) != hipSuccess ||
         nb < 1)
       nb = 1;
     per_cu = nb;
@@ -852,7 +855,7 @@ hipError_t launch_reg(const RebinFilterArgs& a, hipStream_t s) {
   const int npairs = (a.nlines + 1) / 2;
   int blocks = std::max(1, std::min(npairs, per_cu * std::max(a.ncu, 1)));
   if (blocks >= 8) blocks &= ~7;   // whole XCD groups (the row-pair-major order)
-  hipLaunchKernelGGL(rebin_filter_reg_kernel<N>, dim3(blocks), dim3(N / 8), 0, s, a);
+  hipLaunchKernelGGL((rebin_filter_reg_kernel<N, WAVES>), dim3(blocks), dim3(N / 8), 0, s, a);
   return hipGetLastError();
 }
 
@@ -918,7 +921,7 @@ hipError_t launch_rebin_filter(const RebinFilterArgs& a, hipStream_t s) {
     case 512: return launch_reg<512>(a, s);
     case 1024: return launch_reg<1024>(a, s);
     case 2048: return launch_reg<2048>(a, s);
-    case 4096: return launch_reg<4096>(a, s);
+    case 4096: return a.rebin_only ? launch_reg<4096>(a, s) : launch_reg<4096, 4>(a, s);
   }
   const int blocks = (a.nlines + 1) / 2;
   const size_t lds = 2 * (size_t)a.nfft * sizeof(FctCplx);
