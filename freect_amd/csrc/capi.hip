@@ -1520,8 +1520,8 @@ FCT_API int fct_wfbp_gpu_ray_backproject(fct_wfbp_gpu_plan* p, const float* raw,
   fct::RayTables t;
   if (ray_tables(p, a, &t)) {
     if (!p->d_ray_rec)
-      p->d_ray_rec =
-          static_cast<float*>(try_scratch(p, (size_t)p->raw_elems() * 3 * sizeof(float)));
+      p->d_ray_rec = static_cast<float*>(try_scratch(
+          p, ((size_t)p->raw_elems() * 3 + 2 * (size_t)p->raw_scan.n_views) * sizeof(float)));
     if (p->d_ray_rec) {
       HIP_TRY(p->ctx, fct::launch_ray_gather(a, t, p->d_ray_rec, p->ncu, p->stream));
       return FCT_OK;

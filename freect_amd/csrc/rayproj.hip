@@ -370,11 +370,30 @@ __global__ __launch_bounds__(64 * kRayRows) void ray_project_table_kernel(RayPro
 // too: decided once more here, from the ray with its row's slope, the axis of
 // a ray within an FP32 rounding of the diagonal could differ from theirs, and
 // the gather lost the ray.
+// 32 channels of a view whose rays are all zero (a data term on some of the
+// views) get no records and are left out by the gather: bit c >> 5 of nz[view]
+// says that there is another value, a byte per block.
 __global__ __launch_bounds__(256) void ray_record_kernel(RayProjArgs a, RayTables t,
-                                                         float* __restrict__ rec) {
+                                                         float* __restrict__ rec,
+                                                         uint8_t* __restrict__ nz) {
+  __shared__ uint32_t groups[4];
   const int cg = (a.ncols + 255) >> 8;
-  const int v = blockIdx.x / cg, c = (blockIdx.x - v * cg) * 256 + threadIdx.x;
-  if (c >= a.ncols) return;
+  const int v = blockIdx.x / cg, g = blockIdx.x - v * cg, c = g * 256 + threadIdx.x;
+  const bool in = c < a.ncols;
+  const size_t o0 = (size_t)v * a.nrows * a.ncols + (in ? c : 0);
+  bool some = false;
+#pragma unroll 8
+  for (int row = 0; row < a.nrows; ++row)
+    some = some || a.raw_in[o0 + (size_t)row * a.ncols] != 0.0f;
+  const uint64_t m = __ballot(in && some);
+  const uint32_t half = threadIdx.x & 32 ? (uint32_t)(m >> 32) : (uint32_t)m;
+  if ((threadIdx.x & 63) == 0)
+    groups[threadIdx.x >> 6] = ((uint32_t)m ? 1u : 0u) | (m >> 32 ? 2u : 0u);
+  __syncthreads();
+  if (threadIdx.x == 0)
+    nz[(size_t)v * 8 + g] =
+        (uint8_t)(groups[0] | groups[1] << 2 | groups[2] << 4 | groups[3] << 6);
+  if (!in || !half) return;
   const RayDir d = ray_dir(a, v, c);
   const bool xmajor = x_planes(t, a.ncols, v, c);
   for (int row = 0; row < a.nrows; ++row) {
@@ -384,7 +403,7 @@ __global__ __launch_bounds__(256) void ray_record_kernel(RayProjArgs a, RayTable
     const float sp = xmajor ? r.sx : r.sy, sq = xmajor ? r.sy : r.sx;
     const float up = xmajor ? r.ux : r.uy, uq = xmajor ? r.uy : r.ux;
     const float t0 = (p0 - sp) / up, dt = dp / up;
-    const size_t o = ((size_t)v * a.nrows + row) * a.ncols + c;
+    const size_t o = o0 + (size_t)row * a.ncols;
     rec[3 * o] = (sq + t0 * uq - q0) / dq;
     rec[3 * o + 1] = dt * uq / dq;
     rec[3 * o + 2] = a.raw_in[o] * fabsf(dt);
@@ -440,7 +459,11 @@ __global__ __launch_bounds__(64) void ray_gather_kernel(RayProjArgs a, RayTables
   const float inv_dg = (float)(1.0 / a.dgamma), ccf = (float)a.cc, dsd = (float)a.dsd;
   const float az = (float)(a.drow / a.ddz), iaz = (float)(a.ddz / a.drow);
 
+  // (The bytes of channel groups past the detector are not written.)
+  const uint64_t groups = ~0ull >> (64 - ((a.ncols + 255) >> 8) * 8);
   for (int v = va; v < vb; ++v) {
+    const uint64_t nz = ld_uniform(q.nz + v) & groups;
+    if (!nz) continue;
     const float4 e0 = ld_uniform4(t.view + 2 * v), e1 = ld_uniform4(t.view + 2 * v + 1);
     const float ca = e0.x, sa = e0.y, bz = e1.x;
     const float zo = (float)(ld_uniform(t.zoff + v) - (double)s0);
@@ -472,7 +495,7 @@ __global__ __launch_bounds__(64) void ray_gather_kernel(RayProjArgs a, RayTables
     const float i1 = __builtin_amdgcn_rcpf(t1), i2 = __builtin_amdgcn_rcpf(t2);
     const float ea = -1.0f - zo, eb = (float)K - zo;
     const float ra = (fminf(ea * i1, ea * i2) - bz) * iaz, rb = (fmaxf(eb * i1, eb * i2) - bz) * iaz;
-    const bool some = c0 <= c1;
+    const bool some = c0 <= c1 && (nz >> (c0 >> 5) & ((2ull << ((c1 >> 5) - (c0 >> 5))) - 1));
     const int rlo = max(wave_min_i(some ? (int)ceilf(fminf(ra, rb) - 0.01f) : INT32_MAX), 0);
     const int rhi = min(wave_max_i(some ? (int)floorf(fmaxf(ra, rb) + 0.01f) : -1), a.nrows - 1);
     if (rlo > rhi) continue;
@@ -489,7 +512,7 @@ __global__ __launch_bounds__(64) void ray_gather_kernel(RayProjArgs a, RayTables
       const bool xm = x_planes(t, a.ncols, v, cc);
       const float prim = xm ? fix : fiy, sec = xm ? fiy : fix;
       // (The rows' own positions differ from the table's by rounding.)
-      if (!(fabsf(fmaf(prim, e.y, e.x) - sec) < 1.001f) || c > c1) continue;
+      if (!(fabsf(fmaf(prim, e.y, e.x) - sec) < 1.001f) || c > c1 || !(nz >> (cc >> 5) & 1)) continue;
       const float T = fmaf(prim, e.w, e.z), Sz = T * az, F0 = fmaf(T, bz, zo);
       const int co = c * 12;
       auto add = [&](float r, u32x3 d) {
@@ -629,6 +652,8 @@ hipError_t launch_ray_project_table(const RayProjArgs& a, const RayTables& t, fl
 hipError_t launch_ray_gather(const RayProjArgs& a, const RayTables& t, float* rec, int ncu,
                              hipStream_t s) {
   RayGather q{};
+  q.nz = reinterpret_cast<const uint64_t*>(rec);
+  rec += 2 * (size_t)a.v1;
   q.rec = rec;
   const int K = a.nz <= 16 ? 16 : 32;
   q.tiles_x = (a.nx + 7) / 8;
@@ -651,7 +676,7 @@ hipError_t launch_ray_gather(const RayProjArgs& a, const RayTables& t, float* re
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(ray_record_kernel, dim3(a.v1 * ((a.ncols + 255) / 256)), dim3(256), 0, s, a,
-                     t, rec);
+                     t, rec, reinterpret_cast<uint8_t*>(const_cast<uint64_t*>(q.nz)));
   const dim3 grid((unsigned)(waves * q.nsplit));
   const bool ffs = a.states > 1;
   if (K == 16 && ffs)

@@ -238,6 +238,7 @@ struct RayTables {
 struct RayGather {
   int32_t tiles_x, tiles_y, slabs, nsplit;   // 8 x 8 column tiles, slabs, splits of the views
   const float* rec;  // [view][row][channel] A, B, value x path length (ray_record_kernel)
+  const uint64_t* nz;  // [view] bit per 32 channels: some ray is not zero
   double reach;    // mm of table z beyond a slab whose views can meet it
 };
 
@@ -280,7 +281,7 @@ RayTables ray_table_layout(const RayProjArgs& a, void* mem);
 hipError_t launch_ray_table(const RayProjArgs& a, const RayTables& t, hipStream_t s);
 hipError_t launch_ray_project_table(const RayProjArgs& a, const RayTables& t, float* pad,
                                     bool pairs, hipStream_t s);
-// rec: 3 floats per ray.
+// rec: 2 floats per view and 3 per ray.
 hipError_t launch_ray_gather(const RayProjArgs& a, const RayTables& t, float* rec, int ncu,
                              hipStream_t s);
 // Adaptive filtration of raw views [v0, v1): per view the largest finite

@@ -187,3 +187,31 @@ def test_path_length_bits(ctx):
         assert err.size == 14400 and np.abs(err).max() < 5 * 2.0 ** -24
         means.append(err.mean())
     assert abs(means[0] - means[1]) < 1e-8, means
+
+
+@pytest.mark.parametrize("case", [1, 3, 4])
+def test_transpose_of_sparse_rays(ctx, oracle, case):
+    # Rays that are zero but for whole views, single rays at the ends of the
+    # 32-channel groups, or one row: against the FP64 restatement, with its bound
+    # above; scratch left by a dense call before is not read.
+    from freect_amd import wfbp
+    sc, rc = _setup(**CASES[case])
+    p = wfbp.Plan(ctx, sc, rc)
+    nz = p.info.n_slices_native
+    dense, out = p.alloc_raw().fill_(float("nan")), p.alloc_native()
+    gen = torch.Generator(device="cuda").manual_seed(case)
+    for keep in ("view", "channels", "row", "nothing"):
+        p.ray_backproject(dense, out)
+        y = torch.zeros_like(dense)
+        r = torch.rand(y.shape, device="cuda", generator=gen) + 0.1
+        if keep == "view":
+            y[sc.n_views // 2] = r[0]
+        elif keep == "channels":
+            for c in (0, 31, 32, 63, 64, sc.n_channels - 1):
+                y[c % 7::7, :, c] = r[c % 7::7, :, c]
+        elif keep == "row":
+            y[:, sc.n_rows // 2] = r[:, 0]
+        p.ray_backproject(y, out)
+        p.synchronize()
+        ref = oracle.ray_backproject(sc, rc, to_np(y).astype(np.float64), nz)
+        assert np.abs(to_np(out) - ref).max() <= 2e-5 * np.abs(ref).max()
