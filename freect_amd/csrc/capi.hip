@@ -155,7 +155,7 @@ int validate(fct_wfbp_gpu_ctx* ctx, const fct_scan_geometry* s, const fct_recon_
 
 void free_plan_buffers(fct_wfbp_gpu_plan* p) {
   void* bufs[] = {p->d_xs,       p->d_ys,        p->d_cs,        p->d_zs,       p->d_zt,
-                  p->d_slab_vrange, p->d_rebin, p->d_rebinT,  p->d_Hn,        p->d_tw,       p->d_thk_off,
+                  p->d_slab_vrange, p->d_rebin, p->d_rebinT, p->d_view_flags, p->d_Hn,        p->d_tw,       p->d_thk_off,
                   p->d_thk_idx,  p->d_thk_w,     p->d_filtered,  p->d_scale, p->d_native,
                   p->d_raw_stage, p->d_vol_stage, p->d_gbar, p->d_thkT_off, p->d_thkT_idx,
                   p->d_thkT_w, p->d_wrange, p->d_zbounds, p->d_ray_tab, p->d_ray_pad, p->d_ray_rec,
@@ -1359,6 +1359,8 @@ FCT_API int fct_wfbp_gpu_plan_create(fct_wfbp_gpu_ctx* ctx, const fct_scan_geome
   PLAN_TRY(upload(&p->d_rebin, tab, p->stream));
   p->h_rebin = tab;
   PLAN_TRY(upload(&p->d_rebinT, tabT, p->stream));
+  PLAN_TRY(hipMalloc(reinterpret_cast<void**>(&p->d_view_flags),
+                     (size_t)p->nviews * sizeof(uint32_t)));
   PLAN_TRY(upload(&p->d_Hn, Hn, p->stream));
   PLAN_TRY(upload(&p->d_tw, tw, p->stream));
   PLAN_TRY(upload(&p->d_thk_off, toff, p->stream));
@@ -1659,6 +1661,7 @@ FCT_API int fct_wfbp_gpu_rebin_adjoint(fct_wfbp_gpu_plan* p, const float* filter
   a.gbar = filtered_bar;
   a.pbar = raw_bar;
   a.ent = p->d_rebinT;
+  a.flags = p->d_view_flags;
   a.off = reinterpret_cast<const int32_t*>(p->d_rebinT + p->rebinT_entries);
   a.nviews = p->nviews;
   a.nrows = p->nrows;

@@ -262,6 +262,7 @@ struct RebinAdjArgs {
   float* pbar;               // [raw view][raw row][raw ch], overwritten
   const int32_t* off;        // [states * raw_ncols + 1] into ent
   const RebinTDev* ent;
+  uint32_t* flags;           // [nviews] scratch: the view has a value
   int32_t nviews, nrows, cpitch;          // parallel views, effective rows
   int32_t raw_nviews, raw_nrows, raw_ncols, states, zshift;
 };
@@ -403,6 +404,7 @@ struct fct_wfbp_gpu_plan {
   fct::RebinDev* d_rebin = nullptr;
   fct::RebinTDev* d_rebinT = nullptr;   // by raw channel; its offsets follow the entries
   int rebinT_entries = 0;
+  uint32_t* d_view_flags = nullptr;     // [nviews] scratch of the rebinning's transpose
   float* d_Hn = nullptr;
   float2* d_tw = nullptr;
   int32_t* d_thk_off = nullptr;

@@ -180,3 +180,34 @@ def test_planes_left_out(ctx, op, nx, ny, slices, fov, x0, rotations, flip):
     torch.cuda.synchronize()
     assert ref.abs().max() > 0
     assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("channels,rows,ffs,views",
+                         [(96, 5, 0, 300), (200, 17, 0, 300), (70, 33, 0, 130), (65, 9, 2, 260),
+                          (64, 16, 3, 400)])
+def test_rebin_transpose_of_sparse_lines(ctx, oracle, channels, rows, ffs, views):
+    # Lines that are zero but for some views (the first, the last, single ones,
+    # one sample), row counts on both sides of the rows that a workgroup takes at
+    # a time: against the FP64 restatement, FP32 sums of a few terms per sample
+    # (at the scan's ends of half a fan's views): 1e-5 of the largest.
+    import numpy as np
+
+    from freect_amd import wfbp
+    w = S.tiny(nx=8, n_slices=2, n_channels=channels, n_rows=rows, ppr=192, rotations=1.0,
+               ffs_mode=ffs)
+    sc = w.scan.replace(n_views=views)
+    p = wfbp.Plan(ctx, sc, w.recon)
+    i = p.info
+    shape = (i.n_parallel_views, i.n_filtered_rows, i.channel_pitch)
+    rng, nv = np.random.RandomState(views), i.n_parallel_views
+    for keep in ([0], [nv - 1], [nv // 2], [nv // 3, nv // 3 + 40], [], "one"):
+        g = np.zeros(shape, np.float32)
+        if keep == "one":
+            g[nv // 2, i.n_filtered_rows - 1, i.n_filtered_channels // 2] = 1.0
+        else:
+            g[keep] = rng.standard_normal((len(keep),) + shape[1:])
+        out = p.alloc_raw().fill_(float("nan"))
+        p.rebin_adjoint(torch.from_numpy(g).cuda(), out)
+        p.synchronize()
+        ref = oracle.rebin_adjoint(sc, g[..., : i.n_filtered_channels].astype(np.float64))
+        assert np.abs(out.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
