@@ -722,7 +722,7 @@ void bp_v1_kernel(BpArgs a) {
 
 // A workgroup of a.nseg waves per tile.
 template <int TZ, int PREC, int MODE, bool CENTERED>
-__global__ __launch_bounds__(64 * kBpMaxSegments)
+__global__ __launch_bounds__(64 * (TZ > 16 ? 256 / TZ : kBpMaxSegments))
 __attribute__((amdgpu_waves_per_eu(TZ >= 8 ? bp_min_waves<TZ, PREC>() : 1, 8)))
 void bp_v1_split_kernel(BpArgs a) {
   extern __shared__ float bp_lds[];
@@ -774,20 +774,16 @@ hipError_t launch3(const BpArgs& a, int mode, hipStream_t s) {
   int share = 0;
   for (int x = 0; x < 8; ++x) share = std::max(share, a.xcd_first[x + 1] - a.xcd_first[x]);
   const int blocks = 8 * share;
-  if constexpr (TZ <= 16) {
-    if (a.nseg > 1 && mode == kBpAccumulate) {
-      hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks),
-                         dim3(64 * a.nseg), a.nseg * TZ * 64 * sizeof(float), s,
-                         a);
+  if (a.nseg > 1 && mode == kBpAccumulate) {
+    hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpAccumulate, C>), dim3(blocks),
+                       dim3(64 * a.nseg), a.nseg * TZ * 64 * sizeof(float), s, a);
+    return hipGetLastError();
+  }
+  if constexpr (PREC == FCT_PRECISION_FP32 || PREC == kPrecisionPairs) {
+    if (a.nseg > 1 && mode == kBpMatched) {
+      hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks),
+                         dim3(64 * a.nseg), a.nseg * TZ * 64 * sizeof(float), s, a);
       return hipGetLastError();
-    }
-    if constexpr (PREC == FCT_PRECISION_FP32 || PREC == kPrecisionPairs) {
-      if (a.nseg > 1 && mode == kBpMatched) {
-        hipLaunchKernelGGL((bp_v1_split_kernel<TZ, PREC, kBpMatched, C>), dim3(blocks),
-                           dim3(64 * a.nseg), a.nseg * TZ * 64 * sizeof(float),
-                           s, a);
-        return hipGetLastError();
-      }
     }
   }
   if (mode == kBpAccumulate)

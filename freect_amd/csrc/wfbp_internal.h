@@ -166,13 +166,17 @@ __host__ __device__ __forceinline__ int2 tile_of(int l, int tiles_x, int tiles_y
 // tiles 5.78 / 5.81 / 5.45 / 5.40 / 6.02 ms; 8192 tiles 6.34 / 5.78 / 5.88 /
 // 5.85 / 7.48 ms and 4.89 / 4.81 / 4.84 / 5.32 / 7.08 ms; 33 264 tiles 17.7 /
 // 17.6 / 17.7 / 18.2 / 22.8 ms; 163 840 tiles 50.2 / 50.9 / 51.5 / 56.8 /
-// 77.6 ms (more segments read more views at a time through each L2).  It
+// 77.6 ms (more segments read more views at a time through each L2).  Tiles of 32
+// slices (four waves per SIMD, half the sums per 64 KB of LDS): up to 2560 waves
+// and 8 segments; 768 tiles FP32 / FP16 16.3 / 7.0 ms in one, 9.3 / 4.3 in two, 5.5 / 2.8
+// in four; 2048 tiles 15.4 / 7.2, 9.2 / 6.8, 9.5 / 5.4; 3072 tiles 10.7 / 7.4 (backprojection
+// 9.7 / 5.4), in two 11.2 / 6.9 (10.5 / 6.6).  It
 // depends on the volume and the tile depth only, so that every entry point
 // (streamed slab groups, batches) sums in the same order.
 inline int bp_segments(int tiles, int nslabs, int H, int tile_z) {
   int s = 1;
-  if (tile_z > 16) return s;   // (their sums do not fit a workgroup's registers)
-  while (s < kBpMaxSegments && (int64_t)tiles * nslabs * s < 16384 && H / (2 * s) >= 4) s *= 2;
+  const int most = imin(kBpMaxSegments, 256 / tile_z), waves = tile_z > 16 ? 2560 : 16384;
+  while (s < most && (int64_t)tiles * nslabs * s < waves && H / (2 * s) >= 4) s *= 2;
   return s;
 }
 
