@@ -636,7 +636,9 @@ __device__ __forceinline__ void fft_forward_regs(FctCplx* v, FctCplx* lds, int t
 // The rebinning without the filter (RebinFilterArgs::rebin_only) stays at three
 // there, which leave more loads in flight: 2000 x 16 x 2048 samples 0.147 ms,
 // at four 0.186 (1728 x 64 x 1472 0.58 both).
-template <int N, int WAVES>
+// PAIRS (RebinFilterArgs::pairs) is a form of its own: as a branch it took 2 % of
+// the stage call that stores quads (400 x 128 x 888 samples 0.331 -> 0.338 ms).
+template <int N, int WAVES, bool PAIRS>
 __global__ __launch_bounds__(N / 8) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
 void rebin_filter_reg_kernel(RebinFilterArgs a) {
   using S = FctFftShape<N>;
@@ -758,7 +760,7 @@ void rebin_filter_reg_kernel(RebinFilterArgs a) {
           const FctCplx y = w[fct_fft_final_reg<N>(m)];
           const bool in = c < a.ncols;
           const float y0 = in ? y.x : 0.0f, y1 = in ? -y.y : 0.0f;
-          if (!a.pairs) {
+          if (!PAIRS) {
             st_nt(out + o0 + c, y0);
             if (has1) st_nt(out + o1 + c, y1);
           } else if (has1 && (r0 & 1) == 0 && r1 == r0 + 1) {
@@ -779,7 +781,7 @@ void rebin_filter_reg_kernel(RebinFilterArgs a) {
       ya[m] = in ? y.x * is : 0.0f;
       yb[m] = in ? -y.y * is : 0.0f;
     }
-    if (a.pairs) {
+    if (PAIRS) {
       const bool same = has1 && (r0 & 1) == 0 && r1 == r0 + 1;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
@@ -841,13 +843,13 @@ void rebin_filter_reg_kernel(RebinFilterArgs a) {
   }
 }
 
-template <int N, int WAVES = 3>
-hipError_t launch_reg(const RebinFilterArgs& a, hipStream_t s) {
+template <int N, int WAVES, bool PAIRS>
+hipError_t launch_reg1(const RebinFilterArgs& a, hipStream_t s) {
   static int per_cu = -1;   // resident blocks per CU (same for every device here)
   if (per_cu < 0) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rebin_filter_reg_kernel<N, WAVES>, N / 8,
-                                                     0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, rebin_filter_reg_kernel<N, WAVES, PAIRS>,
+                                                     N / 8,                                                     0) != hipSuccess ||
         nb < 1)
       nb = 1;
     per_cu = nb;
@@ -855,8 +857,13 @@ hipError_t launch_reg(const RebinFilterArgs& a, hipStream_t s) {
   const int npairs = (a.nlines + 1) / 2;
   int blocks = std::max(1, std::min(npairs, per_cu * std::max(a.ncu, 1)));
   if (blocks >= 8) blocks &= ~7;   // whole XCD groups (the row-pair-major order)
-  hipLaunchKernelGGL((rebin_filter_reg_kernel<N, WAVES>), dim3(blocks), dim3(N / 8), 0, s, a);
+  hipLaunchKernelGGL((rebin_filter_reg_kernel<N, WAVES, PAIRS>), dim3(blocks), dim3(N / 8), 0, s, a);
   return hipGetLastError();
+}
+
+template <int N, int WAVES = 3>
+hipError_t launch_reg(const RebinFilterArgs& a, hipStream_t s) {
+  return a.pairs ? launch_reg1<N, WAVES, true>(a, s) : launch_reg1<N, WAVES, false>(a, s);
 }
 
 }  // namespace
