@@ -7,8 +7,8 @@ into 512 x 512 x 320 slices at 0.625 mm, 500 mm FOV, ramp filter.
 
 A step is one whole reconstruction (rebin + filter -> backprojection ->
 thickening) with the raw scan already resident in HBM.  The chosen path
-stores filtered projections as FP16 2 x 2 bilinear quads with one FP32 scale
-per scan, accumulates in FP32 and runs as a Batch: the step recorded once
+stores filtered projections as FP16 row pairs with one FP32 scale per scan,
+accumulates in FP32 and runs as a Batch: the step recorded once
 into a hipGraph, the tile depth from the autotuner (a batch of this one job
 backprojects with the single-plan grid kernel; several jobs share one
 persistent launch).
@@ -798,14 +798,18 @@ def main():
         torch.cuda.empty_cache()
         counters = measure_counters(args, chosen.get("tile_z", info.tile_z))
     key = "bp_" + args.precision
+    # The batch backprojects the chain's row pairs, a single plan's bp_ms is that
+    # of the stage call; the counters below are of the same kernel.
+    layout = "row pairs" if args.path == "batch" else (
+        "rows" if args.precision == "fp32" else "quads")
     roof = {"bound": "hbm", "kernel": f"bp_v1_kernel<{chosen.get('tile_z', info.tile_z)}, "
-                                      f"{args.precision.upper()}>",
+                                      f"{args.precision.upper()} {layout}>",
             "achieved": None, "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": None,
             "traffic": None, "bp_ms": chosen["bp_ms"],
             "gather_rate": {"GBps": gather / 1e9, "bytes_per_voxel_view": bpv,
                             "note": "4 bilinear taps per voxel-view read from L1/L2 (the "
                                     "algorithmic gather rate, not HBM traffic)"},
-            "lds_bytes": 0}
+            "lds_bytes": 256 * chosen.get("tile_z", info.tile_z)}
     if counters and key in counters:
         c = counters[key]
         hbm = c["fetch_bytes"] + c["write_bytes"]
@@ -819,12 +823,13 @@ def main():
                      "valu_insts_per_voxel_view_wave": c.get("valu_insts", 0) * 64.0 / n_vv,
                      "limiter": "VALU issue (a wave64 FP32 instruction holds a 16-lane SIMD "
                                 "for 4 cycles; the kernel issues above 0.25 per SIMD-cycle "
-                                "only through its faster integer instructions), then the tap "
-                                "gathers' latency; HBM at frac of peak",
+                                "only through its faster integer instructions) together with "
+                                "the tap gathers' address unit (profiles/timed_calls.md: 84 % "
+                                "busy); HBM at frac of peak",
                      "counters": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE / SQ_ACTIVE_INST_VALU "
                                  "on a child run of this build (bench.py --probe), calibrated "
-                                 "by the abs-max pass (reads the raw scan) and the thickening "
-                                 "(writes the volume)"})
+                                 "by the abs-max pass (reads the raw views used) and the "
+                                 "thickening (writes the volume)"})
     out = {
         "metric": "voxel-views/s + s/volume at 512^2, mixed+batched vs plain FP32, <=1 HU RMSE",
         "value": chosen["voxel_views_per_s"],
@@ -875,7 +880,8 @@ def main():
 def traffic_probe(args, torch):
     """Child of bench.py's counter runs (rocprofv3 --pmc): one FP16 and one
     FP32 pass of rebin+filter -> backprojection -> thickening over the full
-    workload, nothing else on the GPU but the scan generation and the plans'
+    workload (the whole chain, as a batch runs it, or with --path plan the
+    stage calls), nothing else on the GPU but the scan generation and the plans'
     set-up kernels."""
     from freect_amd import scans as S
     from freect_amd import wfbp
@@ -885,17 +891,24 @@ def traffic_probe(args, torch):
     torch.cuda.synchronize()
     for prec in ("fp16", "fp32"):
         plan = wfbp.Plan(ctx, w.scan, w.recon, precision=prec, tile_z=args.tile_z)
-        filt, scale = plan.alloc_filtered()
-        nat, vol = plan.alloc_native(), plan.alloc_volume()
-        plan.rebin_filter(raw, filt, scale)
-        plan.backproject(filt, scale, nat)
-        plan.thicken(nat, vol)
-        plan.synchronize()
         info = plan.info
-        del filt, scale, nat, vol, plan
+        vol = plan.alloc_volume()
+        views = w.scan.n_views   # read by the abs-max pass
+        if args.path == "batch":
+            plan.reconstruct(raw, vol)
+            views = info.read_views_end - info.read_views_first
+        else:
+            filt, scale = plan.alloc_filtered()
+            nat = plan.alloc_native()
+            plan.rebin_filter(raw, filt, scale)
+            plan.backproject(filt, scale, nat)
+            plan.thicken(nat, vol)
+        plan.synchronize()
+        filt = scale = nat = vol = None
+        plan.close()
         torch.cuda.empty_cache()
-    print(json.dumps({"raw_bytes": info.raw_elems * 4, "volume_bytes": info.volume_elems * 4}),
-          flush=True)
+    print(json.dumps({"raw_bytes": views * w.scan.n_rows * w.scan.n_channels * 4,
+                      "volume_bytes": info.volume_elems * 4}), flush=True)
 
 
 def _read_counter_csv(d):
@@ -942,7 +955,7 @@ def measure_counters(args, tile_z, simds=1024):
         d = tempfile.mkdtemp(prefix="fct_pmc_")
         cmd = ["timeout", "-s", "KILL", "180", rp, "--pmc", *counters, "--output-format", "csv",
                "-d", d, "-o", "pmc", "--", sys.executable, os.path.abspath(__file__),
-               "--probe", "--tile-z", str(tile_z)]
+               "--probe", "--path", args.path, "--tile-z", str(tile_z)]
         log("counters:", " ".join(counters))
         r = subprocess.run(cmd, capture_output=True, text=True)
         for line in r.stdout.splitlines():
