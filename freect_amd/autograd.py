@@ -65,7 +65,7 @@ class ProjectFunction(torch.autograd.Function):
 def _p0(plan, x):
     """P0 x = R^T M^T x (raw fan data), M^T the matched voxel-driven projector."""
     lines = plan.alloc_lines()
-    plan.matched_project(x.contiguous(), lines)   # zero-fills, then scatters
+    plan.matched_project(x.contiguous(), lines)
     p = plan.alloc_raw()
     plan.rebin_adjoint(lines, p)
     return p

@@ -171,8 +171,8 @@ __global__ __launch_bounds__(256) void bp_adjoint_column_kernel(BpAdjArgs a, Adj
 
 // xbar * scale / sum W of every voxel for the theta~ [t0, t0 + nt) (0 where no
 // view selects the voxel), in that order: one wave per 64 voxels along the
-// secondary axis and eight slices.  Bound by the writes (9.3 GB for 384 x 384 x
-// 32 voxels x 492 theta~) and by VALU issue together: 4.5 -> 4.3 ms with the
+// secondary axis and eight slices.  9.3 GB of writes for 384 x 384 x 32 voxels x
+// 492 theta~ at 2.2 TB/s, VALU issue 66 % of its cycles: 4.5 -> 4.3 ms with the
 // mask-free weight.  The division is correctly rounded, as in the scattering
 // kernel; v_rcp_f32 in its place saves 0.5 ms and is a bit less precise.
 constexpr int kAdjSlices = 8;
@@ -273,14 +273,16 @@ __global__ __launch_bounds__(256) void swap_volume_kernel(const float* __restric
 // whose channel position lies within one channel of the lane's (a fixed
 // small number of candidates around the ray, tested with the forward
 // kernels' FP32 position) add their slices into the lane's rows (one LDS read
-// and write of two rows per slice, conflict-free).  23 VALU
-// instructions per slice of a candidate (14 in the matched projector), of whose lanes half to three quarters
-// hold one.  2952 views x 16 x 736 from 384 x 384 x 32 voxels: 287 ms with
-// four global atomics per sample -> 4.3 (weights) + 11.1 ms.  Planes on which no
-// lane has a voxel in its rows are left out (9840 views x 64 x 888, 32 x 32 x 4 of
-// 40 mm: 5.2 -> 2.4 ms, where the atomics take 2.6; 2304 views x 16 x 736, 512 x 1 x
-// 16: 2.7 -> 1.0 ms, atomics 1.8).  RC rows per
-// wave: 16 or 32, so that the rows in LDS leave at least 16 waves per CU.
+// and write of two rows per slice, conflict-free).  23 VALU instructions per slice
+// of a candidate, 14 in the matched projector; counters (2952 views x 16 x 736,
+// 384 x 384 x 32 voxels): VALU issue 92 % of the kernel's cycles with 39 of 64 lanes
+// active (half to three quarters of the lanes hold a column), address unit 47 %;
+// matched (2304 views, 256 x 256 x 32) 76 % with 49 lanes, 56 %.  287 ms with four
+// global atomics per sample -> 4.3 (weights) + 11.1 ms.  Planes on which no lane
+// has a voxel in its rows are left out (9840 views x 64 x 888, 32 x 32 x 4 of 40 mm:
+// 5.2 -> 2.4 ms, where the atomics take 2.6; 2304 views x 16 x 736, 512 x 1 x 16: 2.7
+// -> 1.0 ms, atomics 1.8).  RC rows per wave: 16 or 32, so that the rows in LDS
+// leave at least 16 waves per CU.
 template <int RC, bool CENTERED, bool MATCHED>
 __global__ __launch_bounds__(64) void bp_adjoint_gather_kernel(BpAdjArgs a, AdjGather q) {
   // Detector rows rlo .. rlo + rspan + 1 (below): this wave's and the

@@ -628,11 +628,12 @@ __device__ __forceinline__ void fft_forward_regs(FctCplx* v, FctCplx* lds, int t
   }
 }
 
-// Three waves per SIMD (162 VGPRs; 128 spill and are slower at N <= 2048, 4.96
-// against 3.97 ms for all lines of the full workload).  A block of N = 4096 is
-// eight waves, of which three per SIMD hold only one: there four (128 VGPRs,
-// two blocks per CU, some twiddles spilled) take the rebinning of 1728 x 64 x
-// 1472 samples (phi + z FFS) from 1.9 to 1.4 ms, its chain from 10.34 to 9.85.
+// Three waves per SIMD (157 VGPRs with pairs, 161 without; 128 spill and are
+// slower at N <= 2048, 4.96 against 3.97 ms for all lines of the full workload).
+// A block of N = 4096 is eight waves, of which three per SIMD hold only one:
+// there four (128 VGPRs, two blocks per CU, 39 to 52 VGPRs spilled, 128 to 144
+// bytes per lane) take the rebinning of 1728 x 64 x 1472 samples (phi + z FFS)
+// from 1.9 to 1.4 ms, its chain from 10.34 to 9.85.
 // The rebinning without the filter (RebinFilterArgs::rebin_only) stays at three
 // there, which leave more loads in flight: 2000 x 16 x 2048 samples 0.147 ms,
 // at four 0.186 (1728 x 64 x 1472 0.58 both).
@@ -928,7 +929,7 @@ hipError_t launch_rebin_filter(const RebinFilterArgs& a, hipStream_t s) {
     case 512: return launch_reg<512>(a, s);
     case 1024: return launch_reg<1024>(a, s);
     case 2048: return launch_reg<2048>(a, s);
-    case 4096: return a.rebin_only ? launch_reg<4096>(a, s) : launch_reg<4096, 4>(a, s);
+    case 4096: return a.rebin_only ? launch_reg1<4096, 3, false>(a, s) : launch_reg<4096, 4>(a, s);
   }
   const int blocks = (a.nlines + 1) / 2;
   const size_t lds = 2 * (size_t)a.nfft * sizeof(FctCplx);

@@ -9,7 +9,24 @@
  * throws.  Device buffers are hipMalloc'd by the caller unless stated.
  *
  * Threading: a plan is bound to one device and one stream and is not
- * re-entrant; distinct plans may be driven from distinct host threads.
+ * re-entrant; distinct plans may be driven from distinct host threads.  Calls of
+ * one plan, captured into a graph or not, share the buffers it owns and must not
+ * overlap.
+ *
+ * Memory: a plan allocates its buffers on first use and keeps them, at the same
+ * addresses, until it is destroyed (a graph captured after that first use may be
+ * replayed as long as the plan lives).  The chain calls need the filtered
+ * projections (row pairs where they leave room for the plan's other buffers,
+ * filtered_bytes otherwise) and the native volume, host buffers also the raw
+ * scan and the output volume; fct_wfbp_gpu_adjoint FP32 lines.  The projectors
+ * take more where it is free: fct_wfbp_gpu_ray_project 16 bytes per (view,
+ * channel) and two copies of the volume with 8 bytes per voxel (4 where 8 exceed
+ * 4 GiB), fct_wfbp_gpu_ray_backproject 12 bytes per ray,
+ * fct_wfbp_gpu_backproject_adjoint and fct_wfbp_gpu_matched_project each up to
+ * 2 GiB of per-theta~ tables (at least one theta~'s: 16 bytes per voxel column
+ * and 4 per voxel), fct_wfbp_gpu_matched_backproject the row pairs of large FP32
+ * plans.  Without that memory, and inside a capture before their first use, they
+ * run kernels that need none and are 3 to 60 times slower.
  */
 #ifndef FCT_WFBP_GPU_H
 #define FCT_WFBP_GPU_H
@@ -307,7 +324,7 @@ FCT_API int fct_wfbp_gpu_rebin(fct_wfbp_gpu_plan* plan, const float* raw, float*
  * sum over the same samples (the W-weighted backprojection without the
  * weights' normalisation or the view window).  With fct_wfbp_gpu_rebin_adjoint
  * / fct_wfbp_gpu_rebin this projects onto the fan data; up to one scale it
- * approximates line integrals.  lines is zero-filled first. */
+ * approximates line integrals.  lines is overwritten. */
 FCT_API int fct_wfbp_gpu_matched_project(fct_wfbp_gpu_plan* plan, const float* native,
                                          float* lines);
 FCT_API int fct_wfbp_gpu_matched_backproject(fct_wfbp_gpu_plan* plan, const float* lines,
@@ -365,7 +382,7 @@ FCT_API int fct_wfbp_gpu_phantom_project(fct_wfbp_gpu_ctx* ctx, const fct_scan_g
  * kernels instead),
  * thicken of every job -- recorded once into a hipGraph and replayed.
  * Each job's volume is bitwise identical to fct_wfbp_gpu_reconstruct on a
- * plan with the same options. */
+ * plan with the same options and tile_z. */
 typedef struct fct_wfbp_gpu_batch fct_wfbp_gpu_batch;
 
 typedef struct {
@@ -404,7 +421,11 @@ FCT_API int fct_wfbp_gpu_batch_backproject(fct_wfbp_gpu_batch* batch);
 /* Autotuner: runs rebin_filter of every job once, then times the
  * backprojection `reps` times for each candidate tile_z (HIP events on the
  * batch stream), keeps the fastest and returns each candidate's mean ms in
- * ms_out (host, n entries, may be NULL).  Synchronous; needs every job bound. */
+ * ms_out (host, n entries, may be NULL).  Synchronous; needs every job bound.
+ * The order in which a voxel's views are summed depends on tile_z, so volumes
+ * of different tile depths differ by FP32 rounding, and an autotuned batch may
+ * differ in its last bits from one run to the next; set tile_z where volumes
+ * have to be the same to the bit. */
 FCT_API int fct_wfbp_gpu_batch_autotune(fct_wfbp_gpu_batch* batch, const int32_t* tile_z,
                                         int32_t n, int32_t reps, float* ms_out);
 FCT_API int fct_wfbp_gpu_batch_info(const fct_wfbp_gpu_batch* batch, fct_batch_info* info);
