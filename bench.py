@@ -824,8 +824,8 @@ def main():
                      "limiter": "VALU issue (a wave64 FP32 instruction holds a 16-lane SIMD "
                                 "for 4 cycles; the kernel issues above 0.25 per SIMD-cycle "
                                 "only through its faster integer instructions) together with "
-                                "the tap gathers' address unit (profiles/timed_calls.md: 84 % "
-                                "busy); HBM at frac of peak",
+                                "the tap gathers' address unit (84 % busy with 8 slices per "
+                                "tile); HBM at frac of peak",
                      "counters": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE / SQ_ACTIVE_INST_VALU "
                                  "on a child run of this build (bench.py --probe), calibrated "
                                  "by the abs-max pass (reads the raw views used) and the "
